@@ -1,7 +1,9 @@
 // Gravity tree build on the device: the tree of gasoline's pkdBuildBinary
 // (pkd.c:2627-2723), node for node.
 //
-// Level by level, every cell of a level is split at the midpoint of the
+// Large cells level by level over the whole chip, then each cell of at most
+// 4096 particles in one workgroup, then each of at most 512 in another:
+// every cell is split at the midpoint of the
 // longest axis of its particles' bounding box (pkd.c:2493-2505) unless it
 // holds nBucket particles or fewer or has no extent (pkd.c:2489).  The
 // partition reproduces pkdUpperPart's Hoare scan (pkd.c:1109-1157): a Hoare
@@ -35,10 +37,12 @@ int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 constexpr int MOM_CH = 2048;     // particles per moment work item
 constexpr int NM = 32;           // per item: raw Q (6), O (10), H (15), Bmax
 constexpr int MOM_SMALL = 64;    // cells of at most this many particles: a thread each
-constexpr int BOX_CH = 1024;     // particles per bounds work item
 constexpr int LMAX = 512;        // cells of at most LMAX particles finish in one workgroup
+constexpr int MID = 4096;        // cells of at most MID particles reach LMAX in one workgroup
 
-// Per cell in creation (breadth-first) order.
+constexpr int DMAX = 2048;       // depths a tree may have
+
+// Per cell in creation order.
 struct GNode {
     int lo, hi, par, side;       // particle range, parent, 0 lower / 1 upper
     int ch0, ch1, dim, root;     // children (-1), split axis (-1: bucket), root cell
@@ -46,98 +50,720 @@ struct GNode {
     double split;
 };
 
-__global__ void k_gt_init(int n, const double *__restrict__ r, double *__restrict__ x,
-                          double *__restrict__ y, double *__restrict__ z, int *__restrict__ src)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    x[i] = r[3 * (size_t)i];
-    y[i] = r[3 * (size_t)i + 1];
-    z[i] = r[3 * (size_t)i + 2];
-    src[i] = i;
-}
-
-// Flag of position i of a partitioning cell: 1 = belongs to the lower part.
-// mode 0: coordinate below the cell's split; mode 1: type bits & mask set.
-// Evaluated inside the prefix-sum pass and again by the rank and swap
-// kernels, each time before the position's particle can have moved.
-struct FlagFn {
-    const int *pnode;
-    const GNode *nd;
-    const double *x, *y, *z;
-    const int *src;
-    const uint32_t *bits;
-    int a, b, mode;
-    uint32_t mask;
-    __device__ __forceinline__ int operator()(int64_t i) const
-    {
-        const int c = pnode[i];
-        if (c < a || c >= b) return 0;
-        const GNode &g = nd[c];
-        if (mode == 1) return (bits[src[i]] & mask) != 0;
-        if (g.dim < 0) return 0;
-        const double v = g.dim == 0 ? x[i] : (g.dim == 1 ? y[i] : z[i]);
-        return v < g.split;
-    }
+// ------------------------------------------------------------ levels
+// Cells of more than MID particles split level by level over tiles of ts
+// particles; each tile lies in one cell of the level.  A level takes four
+// launches: k_gt_ctl (one workgroup: split decisions, child ids, the tile
+// list), k_gt_count (each tile's lower-part flags as bits, and their number),
+// k_gt_rank (the upper part's misplaced particles by rank) and k_gt_swap (the
+// Hoare swaps, and the children's bounds as the particles pass through
+// registers).  Only particles of cells that still split are read.  Cells of
+// at most MID particles are left to k_gt_mid.
+struct GLevel {
+    int a, b;            // cells of the level: ids a..b-1
+    int ntile;           // tiles of its splitting cells
+    int nunit;           // cells left to k_gt_mid so far
+    int next;            // first free node id once the levels are done
+    int err;             // 1: a split left one side empty
+    int need[2];         // particles lacking a type bit of each order
+    int maxb;            // largest bucket
+    int maxdep;          // deepest cell k_gt_mid made
 };
 
-// Split position s = lo + number of lower-part particles.  A split that
-// leaves one side empty (the reference asserts against it, pkd.c:2512-2516)
-// sets *err.
-__global__ void k_gt_count(int a, int b, int mode, const int64_t *__restrict__ F,
-                           GNode *__restrict__ nd, int *__restrict__ err)
+// Doubles as unsigned integers of the same order, for atomic min and max.
+__device__ __forceinline__ unsigned long long ord_key(double v)
 {
-    const int c = a + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= b) return;
-    GNode &g = nd[c];
-    const bool part = mode == 1 || g.dim >= 0;
-    g.s = part ? g.lo + (int)(F[g.hi + 1] - F[g.lo]) : g.lo;
-    if (mode == 0 && part && (g.s == g.lo || g.s > g.hi)) atomicOr(err, 1);
+    const long long b = __double_as_longlong(v);
+    return (unsigned long long)(b < 0 ? ~b : (b | (long long)0x8000000000000000ull));
 }
 
-// Positions of the upper-part positions that hold a lower particle, by
-// rank counted down from hi: posR[lo + k].
-__global__ void k_gt_rank(int n, FlagFn fl, const int64_t *__restrict__ F, int *__restrict__ posR)
+__device__ __forceinline__ double ord_val(unsigned long long k)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = fl.pnode[i];
-    if (c < fl.a || c >= fl.b) return;
-    const GNode &g = fl.nd[c];
-    if (fl.mode == 0 && g.dim < 0) return;
-    if (i >= g.s && fl(i)) {
-        const int k = (int)(F[g.hi + 1] - F[i + 1]);
-        posR[g.lo + k] = i;
+    const long long b = (long long)k;
+    return __longlong_as_double(b < 0 ? (b & 0x7fffffffffffffffll) : ~b);
+}
+
+__device__ __forceinline__ void box_init(unsigned long long *b)
+{
+    for (int d = 0; d < 3; ++d) {
+        b[d] = ~0ull;
+        b[3 + d] = 0ull;
+    }
+}
+
+// The last root whose first position is <= i.
+__device__ __forceinline__ int root_of(int i, int nr, const int *__restrict__ rlo)
+{
+    int lo = 0, hi = nr - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (rlo[mid] <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Root cells, their empty bounds and the level state.
+__global__ void k_gt_roots(int nr, const int *__restrict__ rlo, const int *__restrict__ rhi,
+                           GNode *__restrict__ nd, unsigned long long *__restrict__ box,
+                           int *__restrict__ unit, GLevel *__restrict__ L)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k == 0) {
+        L->a = 0;
+        L->b = L->next = nr;
+        L->ntile = L->nunit = L->err = L->need[0] = L->need[1] = L->maxb = L->maxdep = 0;
+    }
+    if (k >= nr) return;
+    GNode &g = nd[k];
+    g.lo = rlo[k];
+    g.hi = rhi[k];
+    g.par = -1;
+    g.side = -1;
+    g.root = k;
+    g.ch0 = g.ch1 = -1;
+    g.dim = -1;
+    g.split = 0.0;
+    g.depth = 0;
+    box_init(box + 6 * (size_t)k);
+    unit[k] = k;
+}
+
+// Min/max of a workgroup's lo/hi (256 threads), left to threads 0..5 as
+// order keys: thread d < 3 the lower bound d, 3 + d the upper.
+__device__ __forceinline__ unsigned long long block_box(double *lo, double *hi, double (*sm)[6])
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int o = 32; o > 0; o >>= 1)
+        for (int d = 0; d < 3; ++d) {
+            const double l = __shfl_xor(lo[d], o), h = __shfl_xor(hi[d], o);
+            lo[d] = l < lo[d] ? l : lo[d];
+            hi[d] = h > hi[d] ? h : hi[d];
+        }
+    if (lane == 0)
+        for (int d = 0; d < 3; ++d) {
+            sm[w][d] = lo[d];
+            sm[w][3 + d] = hi[d];
+        }
+    __syncthreads();
+    if (threadIdx.x >= 6) return 0;
+    double v = sm[0][threadIdx.x];
+    for (int k = 1; k < 4; ++k) {
+        const double t = sm[k][threadIdx.x];
+        v = threadIdx.x < 3 ? (t < v ? t : v) : (t > v ? t : v);
+    }
+    return ord_key(v);
+}
+
+constexpr int INIT_E = 8;        // particles per thread of k_gt_init
+
+// Positions into storage order, the roots' bounds, and whether a particle
+// lacks the type bits of msrBuildTree's orders (*need, master.c:4262).
+__global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__restrict__ rlo,
+                                                 const double *__restrict__ r,
+                                                 const uint32_t *__restrict__ bits,
+                                                 double *__restrict__ x, double *__restrict__ y,
+                                                 double *__restrict__ z, int *__restrict__ src,
+                                                 unsigned long long *__restrict__ box,
+                                                 GLevel *__restrict__ L)
+{
+    __shared__ double sm[4][6];
+    const int first = blockIdx.x * (256 * INIT_E), last = min(n, first + 256 * INIT_E) - 1;
+    const int r0 = root_of(first, nr, rlo), r1 = root_of(last, nr, rlo);
+    double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+    bool lack0 = false, lack1 = false;
+    for (int e = 0; e < INIT_E; ++e) {
+        const int i = first + e * 256 + threadIdx.x;
+        if (i > last) break;
+        const double v[3] = {r[3 * (size_t)i], r[3 * (size_t)i + 1], r[3 * (size_t)i + 2]};
+        x[i] = v[0];
+        y[i] = v[1];
+        z[i] = v[2];
+        src[i] = i;
+        const uint32_t t = bits[i];
+        lack0 |= !(t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
+        lack1 |= !(t & GG_TYPE_TREEACTIVE);
+        if (r0 == r1) {
+            for (int d = 0; d < 3; ++d) {
+                lo[d] = v[d] < lo[d] ? v[d] : lo[d];
+                hi[d] = v[d] > hi[d] ? v[d] : hi[d];
+            }
+        } else {
+            unsigned long long *b = box + 6 * (size_t)root_of(i, nr, rlo);
+            for (int d = 0; d < 3; ++d) {
+                if (v[d] != v[d]) continue;
+                atomicMin(b + d, ord_key(v[d]));
+                atomicMax(b + 3 + d, ord_key(v[d]));
+            }
+        }
+    }
+    const unsigned long long m0 = __ballot(lack0), m1 = __ballot(lack1);
+    if ((threadIdx.x & 63) == 0) {
+        if (m0) atomicOr(&L->need[0], 1);
+        if (m1) atomicOr(&L->need[1], 1);
+    }
+    if (r0 != r1) return;
+    const unsigned long long k = block_box(lo, hi, sm);
+    unsigned long long *b = box + 6 * (size_t)r0;
+    if (threadIdx.x < 3) atomicMin(b + threadIdx.x, k);
+    else if (threadIdx.x < 6) atomicMax(b + threadIdx.x, k);
+}
+
+// The host's copy of a device word (pinned memory, -1 until written).
+__device__ __forceinline__ void tell_host(int *p, int v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void k_gt_tell(const int *__restrict__ v, int *__restrict__ host)
+{
+    tell_host(host, *v);
+}
+
+// One workgroup decides the level's cells (mode 0, pkd.c:2489-2505): cells of
+// more than MID particles with any extent split at the middle of their
+// longest axis and get two child ids; the others join the unit list.  Then
+// the tiles of the splitting cells.  mode 1 (the type orders): every cell
+// is partitioned, none split.  The tile count goes to *host.  One workgroup
+// because a level has at most 2 n / MID cells and every later launch waits
+// for it: 4-6 us a level, against the three scans, the decision and id
+// kernels and the host's wait it replaces.
+constexpr int CTL_T = 1024;
+__global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, GLevel *L,
+                                                  GNode *__restrict__ nd,
+                                                  const unsigned long long *__restrict__ box,
+                                                  unsigned long long *__restrict__ kbox,
+                                                  int4 *__restrict__ tiles,
+                                                  int *__restrict__ unit, int *host)
+{
+#pragma clang fp contract(off)
+    __shared__ int soff[CTL_T + 1], scell[CTL_T], sfirst[CTL_T];
+    __shared__ int ws[CTL_T / 64][3];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int a = L->a, b = L->b, nunit0 = L->nunit;
+    const bool bad = L->err != 0;
+    int nsp = 0, ntl = 0, nun = 0;       // splits, tiles and units so far
+    for (int base = a; base < b && !bad; base += CTL_T) {
+        const int c = base + tid;
+        int split = 0, nt = 0, un = 0, lo = 0;
+        if (c < b) {
+            GNode &g = nd[c];
+            lo = g.lo;
+            const int cnt = g.hi - lo + 1;
+            if (mode == 1) {
+                nt = (cnt + ts - 1) / ts;
+            } else if (cnt <= MID) {
+                un = 1;
+            } else {
+                const unsigned long long *k = box + 6 * (size_t)(c - a);
+                double bmin[3], bmax[3];
+                for (int d = 0; d < 3; ++d) {
+                    bmin[d] = ord_val(k[d]);
+                    bmax[d] = ord_val(k[3 + d]);
+                }
+                bool extent = false;
+                for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
+                if (extent) {
+                    int d = 0;
+                    for (int q = 1; q < 3; ++q)
+                        if (bmax[q] - bmin[q] > bmax[d] - bmin[d]) d = q;
+                    g.dim = d;
+                    g.split = 0.5 * (bmin[d] + bmax[d]);
+                    split = 1;
+                    nt = (cnt + ts - 1) / ts;
+                } else {
+                    un = 1;              // coincident particles: a bucket (dim -1)
+                }
+            }
+        }
+        int is = split, it = nt, iu = un;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int us = __shfl_up(is, o), ut = __shfl_up(it, o), uu = __shfl_up(iu, o);
+            if (lane >= o) {
+                is += us;
+                it += ut;
+                iu += uu;
+            }
+        }
+        if (lane == 63) {
+            ws[w][0] = is;
+            ws[w][1] = it;
+            ws[w][2] = iu;
+        }
+        __syncthreads();
+        int ts0 = 0, tt0 = 0, tu0 = 0, ps = 0, pt = 0, pu = 0;
+        for (int k = 0; k < CTL_T / 64; ++k) {
+            if (k < w) {
+                ps += ws[k][0];
+                pt += ws[k][1];
+                pu += ws[k][2];
+            }
+            ts0 += ws[k][0];
+            tt0 += ws[k][1];
+            tu0 += ws[k][2];
+        }
+        const int t0 = pt + it - nt;     // this cell's first tile in the chunk
+        soff[tid] = t0;
+        scell[tid] = c;
+        sfirst[tid] = lo;
+        if (tid == 0) soff[CTL_T] = tt0;
+        if (split) {
+            const int kid = 2 * (nsp + ps + is - 1);
+            GNode &g = nd[c];
+            g.ch0 = b + kid;
+            g.ch1 = b + kid + 1;
+            for (int q = 0; q < 2; ++q) {
+                GNode &h = nd[b + kid + q];
+                h.par = c;
+                h.side = q;
+                h.root = g.root;
+                h.ch0 = h.ch1 = -1;
+                h.dim = -1;
+                h.split = 0.0;
+                h.depth = depth + 1;
+                box_init(kbox + 6 * (size_t)(kid + q));
+            }
+        }
+        if (un) unit[nunit0 + nun + pu + iu - 1] = c;
+        __syncthreads();
+        for (int t = tid; t < tt0; t += CTL_T) {   // the last cell whose first tile is <= t
+            int l = 0, h = CTL_T - 1;
+            while (l < h) {
+                const int mid = (l + h + 1) >> 1;
+                if (soff[mid] <= t) l = mid;
+                else h = mid - 1;
+            }
+            tiles[ntl + t] = make_int4(scell[l], sfirst[l] + (t - soff[l]) * ts, ntl + soff[l],
+                                       ntl + soff[l + 1]);
+        }
+        nsp += ts0;
+        ntl += tt0;
+        nun += tu0;
+        __syncthreads();
+    }
+    if (tid == 0) {
+        L->ntile = ntl;
+        if (mode == 0) {
+            L->a = b;
+            L->b = L->next = b + 2 * nsp;
+            L->nunit = nunit0 + nun;
+            tell_host(host + 1, nunit0 + nun);
+            tell_host(host + 2, b + 2 * nsp);
+        }
+        tell_host(host, ntl);
+    }
+}
+
+struct TileArgs {
+    int ts;                              // particles per tile (a multiple of 256)
+    uint32_t mask;                       // type orders: the bits of the lower part
+    const GLevel *L;
+    const int4 *tiles;                   // cell, first particle, the cell's tiles
+    GNode *nd;
+    double *x, *y, *z;
+    int *src;
+    const uint32_t *bits;                // caller order
+    unsigned long long *flag;            // lower-part flags, ts / 64 words per tile
+    int *tcnt, *tpre;                    // per tile: lower-part particles, those before it
+    int *posR;
+    int *err;
+};
+
+// mode 0: the coordinate below the cell's split; mode 1: a type bit of mask.
+template <int MODE>
+__device__ __forceinline__ bool lower_flag(const TileArgs &A, const double *v, double split, int i)
+{
+    if (MODE == 1) return (A.bits[A.src[i]] & A.mask) != 0;
+    return v[i] < split;
+}
+
+__device__ __forceinline__ const double *split_axis(const TileArgs &A, int dim)
+{
+    return dim == 0 ? A.x : (dim == 1 ? A.y : A.z);
+}
+
+template <int MODE> __global__ __launch_bounds__(256) void k_gt_count(TileArgs A)
+{
+    __shared__ int wc[4];
+    const int t = blockIdx.x;
+    if (t >= A.L->ntile) return;
+    const int4 T = A.tiles[t];
+    const int hi = A.nd[T.x].hi, last = min(hi, T.y + A.ts - 1);
+    const double split = A.nd[T.x].split;
+    const double *v = split_axis(A, A.nd[T.x].dim);
+    unsigned long long *fw = A.flag + (size_t)t * (A.ts / 64);
+    int c = 0;
+    for (int j = threadIdx.x; j < A.ts; j += 256) {
+        const int i = T.y + j;
+        const bool f = i <= last && lower_flag<MODE>(A, v, split, i);
+        const unsigned long long m = __ballot(f);
+        if ((threadIdx.x & 63) == 0) fw[j >> 6] = m;
+        c += __popcll(m);
+    }
+    if ((threadIdx.x & 63) == 0) wc[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) A.tcnt[t] = wc[0] + wc[1] + wc[2] + wc[3];
+}
+
+constexpr int TW = 64;                   // flag words of the largest tile
+
+// The tile's flag words and, before each, the number of flags of its cell
+// (pre: those of the cell's earlier tiles).
+__device__ __forceinline__ void tile_flags(const TileArgs &A, int t, int pre,
+                                           unsigned long long *fw, int *fp)
+{
+    if (threadIdx.x < 64) {
+        const int l = threadIdx.x;
+        const unsigned long long m = l < A.ts / 64 ? A.flag[(size_t)t * (A.ts / 64) + l] : 0;
+        const int c = __popcll(m);
+        int inc = c;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o);
+            if (l >= o) inc += u;
+        }
+        fw[l] = m;
+        fp[l] = pre + inc - c;
+    }
+    __syncthreads();
+}
+
+// Split position s = lo + number of lower-part particles (the first tile of
+// a cell writes it and the children's ranges); a split that leaves one side
+// empty (the reference asserts against it, pkd.c:2512-2516) sets *err.  Then
+// the upper part's positions that hold a lower particle, by rank counted
+// down from hi: posR[lo + k].
+template <int MODE> __global__ __launch_bounds__(256) void k_gt_rank(TileArgs A)
+{
+    __shared__ unsigned long long fw[TW];
+    __shared__ int fp[TW], red[2][4];
+    const int t = blockIdx.x;
+    if (t >= A.L->ntile) return;
+    const int4 T = A.tiles[t];
+    int pre = 0, tot = 0;
+    for (int k = T.z + threadIdx.x; k < T.w; k += 256) {
+        const int c = A.tcnt[k];
+        tot += c;
+        if (k < t) pre += c;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        pre += __shfl_xor(pre, o);
+        tot += __shfl_xor(tot, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = pre;
+        red[1][threadIdx.x >> 6] = tot;
+    }
+    __syncthreads();
+    pre = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    const int nl = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    tile_flags(A, t, pre, fw, fp);
+    GNode &g = A.nd[T.x];
+    const int lo = g.lo, hi = g.hi, s = lo + nl;
+    if (threadIdx.x == 0) {
+        A.tpre[t] = pre;
+        if (t == T.z) {
+            g.s = s;
+            if (MODE == 0) {
+                if (s == lo || s > hi) atomicOr(A.err, 1);
+                GNode &l = A.nd[g.ch0], &u = A.nd[g.ch1];
+                l.lo = lo;
+                l.hi = s - 1;
+                u.lo = s;
+                u.hi = hi;
+            }
+        }
+    }
+    const int last = min(hi, T.y + A.ts - 1);
+    for (int i = T.y + threadIdx.x; i <= last; i += 256) {
+        if (i < s) continue;
+        const int j = i - T.y;
+        const unsigned long long m = fw[j >> 6], bit = 1ull << (j & 63);
+        if (!(m & bit)) continue;
+        A.posR[lo + nl - 1 - (fp[j >> 6] + __popcll(m & (bit - 1)))] = i;
     }
 }
 
 // The swaps of the Hoare scan: the lower-part position holding the k-th
 // upper particle (counted up from lo) <-> posR[lo + k], each pair swapped
-// by its lower member.  With descend set, every position of the level also
-// moves to its cell's child (lower part: ch0, upper: ch1; -1 in a bucket).
-__global__ void k_gt_swap(int n, FlagFn fl, int descend, const int64_t *__restrict__ F,
-                          const int *__restrict__ posR, double *__restrict__ x,
-                          double *__restrict__ y, double *__restrict__ z, int *__restrict__ src,
-                          int *pnode)
+// by its lower member.  Every particle passes through registers once, so
+// the children's bounds are taken on the way (mode 0).  It moves 24-28 bytes
+// a particle and 56 a swapped one.  Measured per level: 31 us on a 2^21
+// Plummer sphere (count 6.3, rank 4.6, control 5.9) and 14 us on 3 10^5
+// particles (4.3, 3.9, 5.4), where the chain of loads and the bounds'
+// reduction bound it rather than the bytes.
+template <int MODE>
+__global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long *__restrict__ kbox)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = fl.pnode[i];
-    if (c < fl.a || c >= fl.b) return;
-    const GNode &g = fl.nd[c];
-    if (fl.mode == 0 && g.dim < 0) {
-        if (descend) pnode[i] = -1;
+    __shared__ unsigned long long fw[TW];
+    __shared__ int fp[TW];
+    __shared__ double sm[2][4][6];
+    const int t = blockIdx.x;
+    if (t >= A.L->ntile) return;
+    const int4 T = A.tiles[t];
+    tile_flags(A, t, A.tpre[t], fw, fp);
+    const GNode &g = A.nd[T.x];
+    const int hi = g.hi, s = g.s, ch0 = g.ch0;
+    const int last = min(hi, T.y + A.ts - 1);
+    double bl[2][3], bh[2][3];
+    for (int q = 0; q < 2; ++q)
+        for (int d = 0; d < 3; ++d) {
+            bl[q][d] = DBL_MAX;
+            bh[q][d] = -DBL_MAX;
+        }
+    auto grow = [&](int q, const double *v) {
+        for (int d = 0; d < 3; ++d) {
+            bl[q][d] = v[d] < bl[q][d] ? v[d] : bl[q][d];
+            bh[q][d] = v[d] > bh[q][d] ? v[d] : bh[q][d];
+        }
+    };
+    for (int i = T.y + threadIdx.x; i <= last; i += 256) {
+        const int j = i - T.y;
+        const unsigned long long m = fw[j >> 6], bit = 1ull << (j & 63);
+        const bool f = m & bit, low = i < s;
+        if (!low && f) continue;         // its partner's thread takes it
+        if (MODE == 1 && (!low || f)) continue;
+        const double v[3] = {A.x[i], A.y[i], A.z[i]};
+        if (low && !f) {
+            const int p = A.posR[i - (fp[j >> 6] + __popcll(m & (bit - 1)))];
+            const double u[3] = {A.x[p], A.y[p], A.z[p]};
+            const int si = A.src[i], sp = A.src[p];
+            A.x[i] = u[0];
+            A.y[i] = u[1];
+            A.z[i] = u[2];
+            A.src[i] = sp;
+            A.x[p] = v[0];
+            A.y[p] = v[1];
+            A.z[p] = v[2];
+            A.src[p] = si;
+            if (MODE == 0) {
+                grow(0, u);
+                grow(1, v);
+            }
+        } else if (MODE == 0) {
+            if (low) grow(0, v);
+            else grow(1, v);
+        }
+    }
+    if (MODE == 1) return;
+    const int kid = ch0 - A.L->a;        // the children's level starts at L->a now
+    for (int q = 0; q < 2; ++q) {
+        const unsigned long long k = block_box(bl[q], bh[q], sm[q]);
+        unsigned long long *b = kbox + 6 * (size_t)(kid + q);
+        if (threadIdx.x < 3) atomicMin(b + threadIdx.x, k);
+        else if (threadIdx.x < 6) atomicMax(b + threadIdx.x, k);
+    }
+}
+
+// The cells of the unit list, each by one workgroup: a cell of LMAX..MID
+// particles is split in LDS, level by level with the rules above, until its
+// parts hold at most LMAX (marked for k_gt_local, dim -2, or left buckets).
+// At most MID / LMAX parts are open at a time, so a level is a handful of
+// wavefront passes over the particles between barriers (7 us measured on one
+// full cell) instead of four launches.  Flags are bits, 64 particles a word, and ranks come
+// from a prefix over the 64 words.  MID is what the LDS holds: 124 KB, one
+// workgroup per CU.
+constexpr int MID_T = 1024, MID_O = MID / LMAX, MID_W = MID / 64;
+static_assert(MID_W == 64, "one wavefront scans the flag words");
+__global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, GLevel *L,
+                                                  int nBucket, GNode *__restrict__ nd,
+                                                  double *__restrict__ px, double *__restrict__ py,
+                                                  double *__restrict__ pz, int *__restrict__ perm,
+                                                  int *__restrict__ err)
+{
+#pragma clang fp contract(off)
+    __shared__ double lx[MID], ly[MID], lz[MID];
+    __shared__ int ls[MID];
+    __shared__ unsigned short posR[MID];
+    __shared__ unsigned long long fbits[MID_W + 1];
+    __shared__ int wpre[MID_W + 1];
+    __shared__ int olo[2][MID_O], ohi[2][MID_O], onode[2][MID_O];
+    __shared__ unsigned long long cb[MID_O][6];
+    __shared__ double csplit[MID_O];
+    __shared__ int cdim[MID_O], nopen[2];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int rootId = unit[blockIdx.x];
+    const int glo = nd[rootId].lo, cnt = nd[rootId].hi - glo + 1;
+    const int troot = nd[rootId].root, rdepth = nd[rootId].depth;
+    if (cnt > MID) return;               // coincident particles: a bucket
+    if (cnt <= LMAX) {
+        if (tid == 0 && cnt > nBucket) nd[rootId].dim = -2;
         return;
     }
-    if (i < g.s && !fl(i)) {
-        const int k = (i - g.lo) - (int)(F[i] - F[g.lo]);
-        const int j = posR[g.lo + k];
-        double t = x[i]; x[i] = x[j]; x[j] = t;
-        t = y[i]; y[i] = y[j]; y[j] = t;
-        t = z[i]; z[i] = z[j]; z[j] = t;
-        const int u = src[i]; src[i] = src[j]; src[j] = u;
+    for (int i = tid; i < cnt; i += MID_T) {
+        lx[i] = px[glo + i];
+        ly[i] = py[glo + i];
+        lz[i] = pz[glo + i];
+        ls[i] = perm[glo + i];
     }
-    if (descend) pnode[i] = i < g.s ? g.ch0 : g.ch1;
+    if (tid == 0) {
+        olo[0][0] = 0;
+        ohi[0][0] = cnt - 1;
+        onode[0][0] = rootId;
+        nopen[0] = 1;
+        fbits[MID_W] = 0;
+    }
+    __syncthreads();
+    // flags of positions below i
+    auto F = [&](int i) {
+        return wpre[i >> 6] + __popcll(fbits[i >> 6] & ((1ull << (i & 63)) - 1));
+    };
+    const int w0 = w * (MID / (MID_T / 64));             // this wavefront's particles
+    constexpr int WN = MID / MID_T;                      // its words
+    int cur = 0, depth = 0;
+    for (; nopen[cur] > 0; ++depth) {
+        const int no = nopen[cur];
+        if (tid < 6 * no) cb[tid / 6][tid % 6] = tid % 6 < 3 ? ~0ull : 0ull;
+        if (tid == 0) nopen[cur ^ 1] = 0;
+        __syncthreads();
+        for (int q = 0; q < no; ++q) {                   // bounds
+            const int lo = olo[cur][q], hi = ohi[cur][q];
+            if (hi < w0 || lo >= w0 + 64 * WN) continue;
+            double bl[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, bh[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+            for (int k = 0; k < WN; ++k) {
+                const int i = w0 + 64 * k + lane;
+                if (i < lo || i > hi) continue;
+                const double v[3] = {lx[i], ly[i], lz[i]};
+                for (int d = 0; d < 3; ++d) {
+                    bl[d] = v[d] < bl[d] ? v[d] : bl[d];
+                    bh[d] = v[d] > bh[d] ? v[d] : bh[d];
+                }
+            }
+            for (int o = 32; o > 0; o >>= 1)
+                for (int d = 0; d < 3; ++d) {
+                    const double l = __shfl_xor(bl[d], o), h = __shfl_xor(bh[d], o);
+                    bl[d] = l < bl[d] ? l : bl[d];
+                    bh[d] = h > bh[d] ? h : bh[d];
+                }
+            if (lane == 0)
+                for (int d = 0; d < 3; ++d) {
+                    atomicMin(&cb[q][d], ord_key(bl[d]));
+                    atomicMax(&cb[q][3 + d], ord_key(bh[d]));
+                }
+        }
+        __syncthreads();
+        if (tid < no) {                                  // split decisions
+            double bmin[3], bmax[3];
+            bool extent = false;
+            for (int d = 0; d < 3; ++d) {
+                bmin[d] = ord_val(cb[tid][d]);
+                bmax[d] = ord_val(cb[tid][3 + d]);
+                extent |= bmax[d] > bmin[d];
+            }
+            int d = 0;
+            for (int k = 1; k < 3; ++k)
+                if (bmax[k] - bmin[k] > bmax[d] - bmin[d]) d = k;
+            cdim[tid] = extent ? d : -1;                 // -1: coincident, a bucket
+            csplit[tid] = 0.5 * (bmin[d] + bmax[d]);
+        }
+        __syncthreads();
+        for (int k = 0; k < WN; ++k) {                   // lower-part flags
+            const int i = w0 + 64 * k + lane;
+            bool f = false;
+            for (int q = 0; q < no; ++q)
+                if (i >= olo[cur][q] && i <= ohi[cur][q] && cdim[q] >= 0)
+                    f = (cdim[q] == 0 ? lx[i] : (cdim[q] == 1 ? ly[i] : lz[i])) < csplit[q];
+            const unsigned long long m = __ballot(f);
+            if (lane == 0) fbits[(w0 >> 6) + k] = m;
+        }
+        __syncthreads();
+        if (w == 0) {
+            const int c = __popcll(fbits[lane]);
+            int inc = c;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(inc, o);
+                if (lane >= o) inc += u;
+            }
+            wpre[lane] = inc - c;
+            if (lane == 63) wpre[MID_W] = inc;
+        }
+        __syncthreads();
+        int part[WN];                                    // swap partner's rank slot, -1: none
+        for (int k = 0; k < WN; ++k) {
+            const int i = w0 + 64 * k + lane;
+            part[k] = -1;
+            for (int q = 0; q < no; ++q) {
+                const int lo = olo[cur][q], hi = ohi[cur][q];
+                if (i < lo || i > hi || cdim[q] < 0) continue;
+                const int F0 = F(lo), nl = F(hi + 1) - F0, Fi = F(i) - F0;
+                const bool f = (fbits[i >> 6] >> (i & 63)) & 1;
+                if (i >= lo + nl && f) posR[lo + nl - 1 - Fi] = (unsigned short)i;
+                if (i < lo + nl && !f) part[k] = i - Fi;
+            }
+        }
+        if (w == 0) {                                    // nodes of the two parts
+            const bool in = lane < no;
+            int lo = 0, hi = -1, s = 0;
+            bool sp = false;
+            if (in) {
+                lo = olo[cur][lane];
+                hi = ohi[cur][lane];
+                s = lo;
+                if (cdim[lane] >= 0) {
+                    s = lo + F(hi + 1) - F(lo);
+                    sp = s > lo && s <= hi;
+                    if (!sp) atomicOr(err, 1);           // one side empty: reported
+                }
+            }
+            const unsigned long long ms = __ballot(sp);
+            int id0 = 0;
+            if (lane == 0 && ms) id0 = atomicAdd(&L->next, 2 * __popcll(ms));
+            id0 = __shfl(id0, 0) + 2 * __popcll(ms & ((1ull << lane) - 1));
+            const int me = in ? onode[cur][lane] : 0;
+            if (sp) {
+                GNode &g = nd[me];
+                g.dim = cdim[lane];
+                g.split = csplit[lane];
+                g.s = glo + s;
+                g.ch0 = id0;
+                g.ch1 = id0 + 1;
+            }
+            for (int q = 0; q < 2; ++q) {
+                const int a0 = q ? s : lo, a1 = q ? hi : s - 1;
+                const bool open = sp && a1 - a0 + 1 > LMAX;
+                const unsigned long long mo = __ballot(open);
+                if (sp) {
+                    GNode &h = nd[id0 + q];
+                    h.lo = glo + a0;
+                    h.hi = glo + a1;
+                    h.par = me;
+                    h.side = q;
+                    h.root = troot;
+                    h.ch0 = h.ch1 = -1;
+                    h.split = 0.0;
+                    h.depth = rdepth + depth + 1;
+                    h.dim = !open && a1 - a0 + 1 > nBucket ? -2 : -1;
+                }
+                const int at = nopen[cur ^ 1] + __popcll(mo & ((1ull << lane) - 1));
+                if (open) {
+                    olo[cur ^ 1][at] = a0;
+                    ohi[cur ^ 1][at] = a1;
+                    onode[cur ^ 1][at] = id0 + q;
+                }
+                if (lane == 0) nopen[cur ^ 1] += __popcll(mo);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+        }
+        __syncthreads();
+        for (int k = 0; k < WN; ++k) {                   // the swaps
+            if (part[k] < 0) continue;
+            const int i = w0 + 64 * k + lane, j = posR[part[k]];
+            double d = lx[i]; lx[i] = lx[j]; lx[j] = d;
+            d = ly[i]; ly[i] = ly[j]; ly[j] = d;
+            d = lz[i]; lz[i] = lz[j]; lz[j] = d;
+            const int u = ls[i]; ls[i] = ls[j]; ls[j] = u;
+        }
+        cur ^= 1;
+        __syncthreads();
+    }
+    if (tid == 0) atomicMax(&L->maxdep, rdepth + depth);
+    for (int i = tid; i < cnt; i += MID_T) {
+        px[glo + i] = lx[i];
+        py[glo + i] = ly[i];
+        pz[glo + i] = lz[i];
+        perm[glo + i] = ls[i];
+    }
 }
 
 // Work items of the cells [a, b): ceil(count / ch) each for cells of more
@@ -149,146 +775,6 @@ __global__ void k_gt_items(int a, int b, int ch, int minc, const GNode *__restri
     if (c >= b) return;
     const int cnt = nd[c].hi - nd[c].lo + 1;
     nit[c - a] = cnt > minc ? (cnt + ch - 1) / ch : 0;
-}
-
-// The cell (relative index) of work item k: the last r with ioff[r] <= k
-// (cells without items share their offset with the next cell).
-__device__ __forceinline__ int item_cell(const int64_t *__restrict__ ioff, int ncell, int64_t k)
-{
-    int lo = 0, hi = ncell - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ioff[mid] <= k) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// Bounds of BOX_CH particles of a cell of more than BOX_CH particles (one
-// wavefront per work item): part[6k..] = min xyz, max xyz.
-__global__ __launch_bounds__(256) void k_gt_box(int a, int b, const int64_t *__restrict__ ioff,
-                                                const GNode *__restrict__ nd,
-                                                const double *__restrict__ x,
-                                                const double *__restrict__ y,
-                                                const double *__restrict__ z,
-                                                double *__restrict__ part)
-{
-    const int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, ncell = b - a;
-    if (k >= ioff[ncell]) return;
-    const int r = item_cell(ioff, ncell, k);
-    const GNode &g = nd[a + r];
-    const int first = g.lo + (int)(k - ioff[r]) * BOX_CH;
-    const int last = min(g.hi, first + BOX_CH - 1);
-    double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    for (int i = first + lane; i <= last; i += 64) {
-        const double v[3] = {x[i], y[i], z[i]};
-        for (int d = 0; d < 3; ++d) {
-            lo[d] = v[d] < lo[d] ? v[d] : lo[d];
-            hi[d] = v[d] > hi[d] ? v[d] : hi[d];
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1)
-        for (int d = 0; d < 3; ++d) {
-            const double l = __shfl_xor(lo[d], o), h = __shfl_xor(hi[d], o);
-            lo[d] = l < lo[d] ? l : lo[d];
-            hi[d] = h > hi[d] ? h : hi[d];
-        }
-    if (lane == 0)
-        for (int d = 0; d < 3; ++d) {
-            part[6 * k + d] = lo[d];
-            part[6 * k + 3 + d] = hi[d];
-        }
-}
-
-// Split decision of each cell of the level (pkd.c:2489-2505), one wavefront
-// per cell: its bounds from its particles, or from its items' bounds for a
-// cell of more than BOX_CH particles.
-__global__ __launch_bounds__(256) void k_gt_decide(int a, int b, int nBucket, int depth,
-                                                   const int64_t *__restrict__ ioff,
-                                                   const double *__restrict__ part,
-                                                   const double *__restrict__ x,
-                                                   const double *__restrict__ y,
-                                                   const double *__restrict__ z,
-                                                   GNode *__restrict__ nd, int *__restrict__ nch)
-{
-#pragma clang fp contract(off)
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (r >= b - a) return;
-    GNode &g = nd[a + r];
-    double bmin[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, bmax[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    if (g.hi - g.lo + 1 > BOX_CH) {
-        for (int64_t it = ioff[r] + lane; it < ioff[r + 1]; it += 64)
-            for (int d = 0; d < 3; ++d) {
-                const double l = part[6 * it + d], h = part[6 * it + 3 + d];
-                bmin[d] = l < bmin[d] ? l : bmin[d];
-                bmax[d] = h > bmax[d] ? h : bmax[d];
-            }
-    } else {
-        for (int i = g.lo + lane; i <= g.hi; i += 64) {
-            const double v[3] = {x[i], y[i], z[i]};
-            for (int d = 0; d < 3; ++d) {
-                bmin[d] = v[d] < bmin[d] ? v[d] : bmin[d];
-                bmax[d] = v[d] > bmax[d] ? v[d] : bmax[d];
-            }
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1)
-        for (int d = 0; d < 3; ++d) {
-            const double l = __shfl_xor(bmin[d], o), h = __shfl_xor(bmax[d], o);
-            bmin[d] = l < bmin[d] ? l : bmin[d];
-            bmax[d] = h > bmax[d] ? h : bmax[d];
-        }
-    if (lane) return;
-    bool extent = false;
-    nch[r] = 0;
-    for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
-    g.dim = -1;
-    g.split = 0.0;
-    g.ch0 = g.ch1 = -1;
-    g.depth = depth;
-    if (g.hi - g.lo + 1 > nBucket && extent) {
-        if (g.hi - g.lo + 1 <= LMAX) {   // split by k_gt_local
-            g.dim = -2;
-            return;
-        }
-        int d = 0;
-        for (int k = 1; k < 3; ++k)
-            if (bmax[k] - bmin[k] > bmax[d] - bmin[d]) d = k;
-        g.dim = d;
-        g.split = 0.5 * (bmin[d] + bmax[d]);
-        nch[r] = 2;
-    }
-}
-
-// Child ids of the level's split cells: next + their offsets.
-__global__ void k_gt_kids(int a, int b, int next, const int64_t *__restrict__ choff,
-                          GNode *__restrict__ nd)
-{
-    const int c = a + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= b) return;
-    GNode &g = nd[c];
-    if (g.dim < 0) return;
-    g.ch0 = next + (int)choff[c - a];
-    g.ch1 = g.ch0 + 1;
-}
-
-// The children's records once the split positions are known.
-__global__ void k_gt_children(int a, int b, GNode *__restrict__ nd)
-{
-    const int c = a + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= b) return;
-    const GNode &g = nd[c];
-    if (g.dim < 0) return;
-    GNode &l = nd[g.ch0], &u = nd[g.ch1];
-    l.lo = g.lo;
-    l.hi = g.s - 1;
-    u.lo = g.s;
-    u.hi = g.hi;
-    l.par = u.par = c;
-    l.side = 0;
-    u.side = 1;
-    l.root = u.root = g.root;
 }
 
 // Subtree sizes and preorder ids, over the nodes of one depth (list).
@@ -312,7 +798,6 @@ __global__ void k_gt_pre(int m, const int *__restrict__ list, GNode *__restrict_
 // Nodes by depth: a count per depth, then each node to its depth's list.
 // Each workgroup counts in LDS
 // first, so the global counters see one atomic per workgroup and depth.
-constexpr int DMAX = 2048;       // depths a tree may have (level loop + local builds)
 
 __global__ __launch_bounds__(256) void k_gt_depth_count(int nn, int ndep,
                                                         const GNode *__restrict__ nd,
@@ -966,65 +1451,38 @@ __global__ void k_gt_rootof(int nn, const GNode *__restrict__ nd, int *__restric
     rootOf[nd[b].pre] = nd[nd[b].root].pre;
 }
 
-__global__ void k_gt_pos2root(int n, int nr, const int *__restrict__ rlo,
-                              int *__restrict__ pos2root)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int lo = 0, hi = nr - 1;   // last root whose first position <= i
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (rlo[mid] <= i) lo = mid;
-        else hi = mid - 1;
-    }
-    pos2root[i] = lo;
-}
-
-__global__ void k_gt_roots(int nr, const int *__restrict__ rlo, const int *__restrict__ rhi,
-                           GNode *__restrict__ nd)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nr) return;
-    GNode &g = nd[k];
-    g.lo = rlo[k];
-    g.hi = rhi[k];
-    g.par = -1;
-    g.side = -1;
-    g.root = k;
-    g.ch0 = g.ch1 = -1;
-    g.dim = 0;      // partitioned by type first
-}
-
 }  // namespace
 
-// One partition pass over the cells [a, b) (mode 0: their splits, and every
-// position moves to its child; mode 1: type bits & mask, every cell).
-static int gt_partition(GGPKD pkd, int a, int b, int mode, uint32_t mask)
+// Waits until the kernels queued on the stream have written *p (pinned,
+// tell_host; -1 before).  The stream running dry without it is an error, so
+// the wait always ends.
+static int host_word(hipStream_t st, const int *p, int *v)
 {
-    GravDev &G = pkd->grav;
-    hipStream_t st = pkd->stream;
-    const int n = pkd->nLocal;
-    GNode *nd = G.gnode.as<GNode>();
-    FlagFn fl;
-    fl.pnode = G.gpn.as<int>();
-    fl.nd = nd;
-    fl.x = G.px.as<double>();
-    fl.y = G.py.as<double>();
-    fl.z = G.pz.as<double>();
-    fl.src = G.perm.as<int>();
-    fl.bits = pkd->f[GG_IACTIVE].as<uint32_t>();
-    fl.a = a;
-    fl.b = b;
-    fl.mode = mode;
-    fl.mask = mask;
-    GG_TRY(exclusive_scan(st, fl, G.gF.as<int64_t>(), n, G.scan, nullptr));
-    hipLaunchKernelGGL(k_gt_count, dim3(nblk(b - a, 256)), dim3(256), 0, st, a, b, mode,
-                       G.gF.as<int64_t>(), nd, G.gerr.as<int>());
-    hipLaunchKernelGGL(k_gt_rank, dim3(nblk(n, 256)), dim3(256), 0, st, n, fl,
-                       G.gF.as<int64_t>(), G.gposR.as<int>());
-    hipLaunchKernelGGL(k_gt_swap, dim3(nblk(n, 256)), dim3(256), 0, st, n, fl, mode == 0 ? 1 : 0,
-                       G.gF.as<int64_t>(), G.gposR.as<int>(), G.px.as<double>(),
-                       G.py.as<double>(), G.pz.as<double>(), G.perm.as<int>(), G.gpn.as<int>());
+    for (unsigned it = 0;; ++it) {
+        *v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+        if (*v != -1) return GG_OK;
+        if ((it & 1023u) != 1023u) continue;
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) continue;
+        GG_HIP(e);
+        *v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+        GG_CHECK(*v != -1, GG_EHIP, "the tree build's device state never arrived");
+        return GG_OK;
+    }
+}
+
+// Particles per tile: enough tiles to fill the chip on a small store, fewer
+// of them (each block adds up its cell's tile counts) on a large one.
+static int tile_size(int n) { return n < (1 << 19) ? 1024 : (n < (1 << 22) ? 2048 : 4096); }
+
+// One partition pass over the tiles k_gt_ctl listed.
+template <int MODE>
+static int gt_partition(GravDev &G, hipStream_t st, const TileArgs &A, int grid,
+                        unsigned long long *kbox)
+{
+    hipLaunchKernelGGL(k_gt_count<MODE>, dim3(grid), dim3(256), 0, st, A);
+    hipLaunchKernelGGL(k_gt_rank<MODE>, dim3(grid), dim3(256), 0, st, A);
+    hipLaunchKernelGGL(k_gt_swap<MODE>, dim3(grid), dim3(256), 0, st, A, kbox);
     GG_HIP(hipGetLastError());
     return GG_OK;
 }
@@ -1038,12 +1496,19 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
     G.built = 0;
     // roots: the non-empty systems
     std::vector<int> rlo;
+    int maxRoot = 0;
     for (int s = 0; s < nSys; ++s)
-        if (sysOff[s + 1] > sysOff[s]) rlo.push_back(sysOff[s]);
+        if (sysOff[s + 1] > sysOff[s]) {
+            rlo.push_back(sysOff[s]);
+            maxRoot = std::max(maxRoot, sysOff[s + 1] - sysOff[s]);
+        }
     const int nr = (int)rlo.size();
     for (int k = 0; k < nr; ++k) rlo.push_back(k + 1 < nr ? rlo[k + 1] - 1 : n - 1);
     const size_t n1 = (size_t)std::max(n, 1);
     const size_t cap = 2 * n1 + 2;   // cells at most: every split has two children
+    const int ts = tile_size(n);
+    const size_t mtile = n1 / ts + n1 / MID + std::max(nr, 1) + 1;   // tiles of a level, at most
+    const size_t mbox = std::max<size_t>(2 * (n1 / MID) + 2, nr);    // its cells
     GG_TRY(G.px.reserve(sizeof(double) * n1));
     GG_TRY(G.py.reserve(sizeof(double) * n1));
     GG_TRY(G.pz.reserve(sizeof(double) * n1));
@@ -1052,77 +1517,108 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
     GG_TRY(G.pact.reserve(sizeof(uint32_t) * n1));
     GG_TRY(G.perm.reserve(sizeof(int) * n1));
     GG_TRY(G.acc.reserve(sizeof(double) * 5 * n1));
-    GG_TRY(G.gpn.reserve(sizeof(int) * n1));
-    GG_TRY(G.gF.reserve(sizeof(int64_t) * (n1 + 1)));
     GG_TRY(G.gposR.reserve(sizeof(int) * n1));
     GG_TRY(G.gnode.reserve(sizeof(GNode) * cap));
-    GG_TRY(G.gbox.reserve(sizeof(double) * 6 * (2 * (n1 / BOX_CH) + 2)));
+    GG_TRY(G.gbox.reserve(sizeof(unsigned long long) * 12 * mbox));
+    GG_TRY(G.gtile.reserve(sizeof(int4) * mtile));
+    GG_TRY(G.gflag.reserve(sizeof(unsigned long long) * mtile * (ts / 64)));
+    GG_TRY(G.gtcnt.reserve(sizeof(int) * 2 * mtile));
+    GG_TRY(G.gunit.reserve(sizeof(int) * cap));
+    GG_TRY(G.glev.reserve(sizeof(GLevel)));
     GG_TRY(G.gnit.reserve(sizeof(int) * cap));
     GG_TRY(G.gioff.reserve(sizeof(int64_t) * (cap + 1)));
-    GG_TRY(G.gnch.reserve(sizeof(int) * cap));
     GG_TRY(G.gchoff.reserve(sizeof(int64_t) * (cap + 1)));
-    GG_TRY(G.gerr.reserve(sizeof(int) * 2));
     GG_TRY(G.groot.reserve(sizeof(int) * 2 * std::max(nr, 1)));
-    GG_HIP(hipMemsetAsync(G.gerr.p, 0, sizeof(int) * 2, st));
+    if (!G.hst)
+        GG_HIP(hipHostMalloc((void **)&G.hst, sizeof(int) * GravDev::NHST, hipHostMallocDefault));
+    GLevel *L = G.glev.as<GLevel>();
     GNode *nd = G.gnode.as<GNode>();
     int nn = 0;
-    std::vector<std::pair<int, int>> levels, depths;
+    std::vector<std::pair<int, int>> depths;
     if (nr > 0) {
         const int *rl = G.groot.as<int>(), *rh = rl + nr;
+        unsigned long long *box[2];
+        box[0] = G.gbox.as<unsigned long long>();
+        box[1] = box[0] + 6 * mbox;
+        volatile int *hv = G.hst;
+        for (int k = 0; k < 8; ++k) hv[k] = -1;
         GG_HIP(hipMemcpyAsync(G.groot.p, rlo.data(), sizeof(int) * 2 * nr, hipMemcpyHostToDevice,
                               st));
-        hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, nr, rl, rh, nd);
-        // every position starts in its system's root (the offsets cover the store)
-        hipLaunchKernelGGL(k_gt_pos2root, dim3(nblk(n, 256)), dim3(256), 0, st, n, nr, rl,
-                           G.gpn.as<int>());
-        hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256)), dim3(256), 0, st, n,
-                           pkd->f[GG_R].as<double>(), G.px.as<double>(), G.py.as<double>(),
-                           G.pz.as<double>(), G.perm.as<int>());
+        hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, nr, rl, rh, nd,
+                           box[0], G.gunit.as<int>(), L);
+        hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, n, nr, rl,
+                           pkd->f[GG_R].as<double>(), pkd->f[GG_IACTIVE].as<uint32_t>(),
+                           G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
+                           G.perm.as<int>(), box[0], L);
+        hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need[1], G.hst + 3);
         GG_HIP(hipGetLastError());
-        // msrBuildTree's active-type orders (master.c:4262), then the tree
-        GG_TRY(gt_partition(pkd, 0, nr, 1, GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
-        GG_TRY(gt_partition(pkd, 0, nr, 1, GG_TYPE_TREEACTIVE));
-        int a = 0, b = nr;
-        while (b > a) {
-            levels.push_back({a, b});
-            // bounds by work items of BOX_CH particles (at most one per cell
-            // plus n / BOX_CH), then the split decisions
-            hipLaunchKernelGGL(k_gt_items, dim3(nblk(b - a, 256)), dim3(256), 0, st, a, b, BOX_CH,
-                               BOX_CH, nd, G.gnit.as<int>());
-            GG_TRY(exclusive_scan_i64(st, G.gnit.as<int>(), G.gioff.as<int64_t>(), b - a, G.scan,
-                                      nullptr));
-            hipLaunchKernelGGL(k_gt_box, dim3(nblk(2 * (int64_t)(n / BOX_CH) + 1, 4)), dim3(256),
-                               0, st, a, b, G.gioff.as<int64_t>(), nd, G.px.as<double>(),
-                               G.py.as<double>(), G.pz.as<double>(), G.gbox.as<double>());
-            hipLaunchKernelGGL(k_gt_decide, dim3(nblk(b - a, 4)), dim3(256), 0, st, a, b, nBucket,
-                               (int)levels.size() - 1, G.gioff.as<int64_t>(), G.gbox.as<double>(),
-                               G.px.as<double>(),
-                               G.py.as<double>(), G.pz.as<double>(), nd, G.gnch.as<int>());
-            // child ids (two per split), then the partition, which also moves
-            // every position to its child
-            int64_t nch = 0;
-            GG_TRY(exclusive_scan_i64(st, G.gnch.as<int>(), G.gchoff.as<int64_t>(), b - a,
-                                      G.scan, &nch));
-            int err = 0;
-            GG_HIP(hipMemcpyAsync(&err, G.gerr.p, sizeof(int), hipMemcpyDeviceToHost, st));
-            GG_HIP(hipStreamSynchronize(st));
-            GG_CHECK(!err, GG_EUNSUP,
-                     "a cell split leaves one side empty (positions differ in the last bit only)");
-            GG_CHECK((size_t)b + (size_t)nch <= cap, GG_EHIP, "tree cell capacity exceeded");
-            if (nch > 0) {
-                hipLaunchKernelGGL(k_gt_kids, dim3(nblk(b - a, 256)), dim3(256), 0, st, a, b, b,
-                                   G.gchoff.as<int64_t>(), nd);
-                GG_TRY(gt_partition(pkd, a, b, 0, 0));
-                hipLaunchKernelGGL(k_gt_children, dim3(nblk(b - a, 256)), dim3(256), 0, st, a, b,
-                                   nd);
-            }
-            GG_HIP(hipGetLastError());
-            a = b;
-            b += (int)nch;
+        TileArgs A;
+        A.ts = ts;
+        A.mask = 0;
+        A.L = L;
+        A.tiles = G.gtile.as<int4>();
+        A.nd = nd;
+        A.x = G.px.as<double>();
+        A.y = G.py.as<double>();
+        A.z = G.pz.as<double>();
+        A.src = G.perm.as<int>();
+        A.bits = pkd->f[GG_IACTIVE].as<uint32_t>();
+        A.flag = G.gflag.as<unsigned long long>();
+        A.tcnt = G.gtcnt.as<int>();
+        A.tpre = A.tcnt + mtile;
+        A.posR = G.gposR.as<int>();
+        A.err = &L->err;
+        const int grid = (int)mtile;
+        auto ctl = [&](int mode, int depth, int *host) {
+            hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, mode, ts, depth, L, nd,
+                               box[depth & 1], box[(depth & 1) ^ 1], G.gtile.as<int4>(),
+                               G.gunit.as<int>(), host);
+        };
+        // msrBuildTree's active-type orders (master.c:4262).  A particle with
+        // the second order's bit has one of the first's, so where all have it
+        // both orders leave everything in place.
+        int lack = 0;
+        GG_TRY(host_word(st, G.hst + 3, &lack));
+        if (lack) {
+            ctl(1, 0, G.hst + 4);
+            A.mask = GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE;
+            GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
+            A.mask = GG_TYPE_TREEACTIVE;
+            GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
         }
-        const int nng = b;
+        int nunit = nr, nng = nr, nlev = 1;
+        if (maxRoot > MID) {
+            // The levels.  The host learns a level's tile count while its
+            // partition runs, in time to queue the next level behind it.
+            for (int depth = 0;; ++depth) {
+                GG_CHECK(depth < DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
+                int *h = G.hst + 8 + 4 * (depth & 3);
+                for (int k = 0; k < 3; ++k) ((volatile int *)h)[k] = -1;
+                ctl(0, depth, h);
+                GG_TRY(gt_partition<0>(G, st, A, grid, box[(depth & 1) ^ 1]));
+                int nt = 0;
+                GG_TRY(host_word(st, h, &nt));
+                if (nt == 0) {
+                    GG_TRY(host_word(st, h + 1, &nunit));
+                    GG_TRY(host_word(st, h + 2, &nng));
+                    nlev = depth + 1;
+                    break;
+                }
+            }
+        }
+        if (nunit > 0)
+            hipLaunchKernelGGL(k_gt_mid, dim3(nunit), dim3(MID_T), 0, st, G.gunit.as<int>(), L,
+                               nBucket, nd, G.px.as<double>(), G.py.as<double>(),
+                               G.pz.as<double>(), G.perm.as<int>(), &L->err);
+        GG_HIP(hipGetLastError());
+        GLevel hl;
+        GG_HIP(hipMemcpyAsync(&hl, L, sizeof hl, hipMemcpyDeviceToHost, st));
+        GG_HIP(hipStreamSynchronize(st));
+        GG_CHECK(!hl.err, GG_EUNSUP,
+                 "a cell split leaves one side empty (positions differ in the last bit only)");
+        nng = hl.next;
         // cells of at most LMAX particles: their subtrees in one launch, each
-        // in node slots reserved after the level loop's cells
+        // in node slots reserved after the cells above them
         GG_TRY(G.gbflag.reserve(sizeof(int) * (size_t)nng));
         hipLaunchKernelGGL(k_gt_lmark, dim3(nblk(nng, 256)), dim3(256), 0, st, nng, nd,
                            G.gbflag.as<int>(), G.gnit.as<int>());
@@ -1143,13 +1639,13 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
                                G.glroot.as<int>(), G.gioff.as<int64_t>(), nBucket, nd,
                                G.gscr.as<GNode>(), G.glused.as<int>(), G.px.as<double>(),
                                G.py.as<double>(), G.pz.as<double>(), G.perm.as<int>(),
-                               G.gerr.as<int>());
+                               &L->err);
             GG_HIP(hipGetLastError());
             int64_t nused = 0;
             GG_TRY(exclusive_scan_i64(st, G.glused.as<int>(), G.glbase.as<int64_t>(), (int)nloc,
                                       G.scan, &nused));
             int err = 0;
-            GG_HIP(hipMemcpyAsync(&err, G.gerr.p, sizeof(int), hipMemcpyDeviceToHost, st));
+            GG_HIP(hipMemcpyAsync(&err, &L->err, sizeof(int), hipMemcpyDeviceToHost, st));
             GG_HIP(hipStreamSynchronize(st));
             GG_CHECK(!err, GG_EUNSUP,
                      "a cell split leaves one side empty (positions differ in the last bit only)");
@@ -1159,8 +1655,8 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
                                G.glbase.as<int64_t>(), nng, nd, G.gscr.as<GNode>());
             GG_HIP(hipGetLastError());
         }
-        // nodes by depth (the level loop's levels, then up to LMAX local ones)
-        const int ndep = (int)levels.size() + LMAX + 1;
+        // nodes by depth
+        const int ndep = std::max(nlev, hl.maxdep + 1) + LMAX + 1;
         GG_CHECK(ndep <= DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
         GG_TRY(G.gdcnt.reserve(sizeof(int) * 2 * (size_t)ndep));
         GG_TRY(G.gdlist.reserve(sizeof(int) * (size_t)nn));
@@ -1275,7 +1771,7 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
         hipLaunchKernelGGL(k_gt_bucket, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, nd,
                            G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
                            G.ph.as<double>(), G.pact.as<uint32_t>(), G.gbflag.as<int>(),
-                           G.gbb8.as<double>(), G.gerr.as<int>() + 1);
+                           G.gbb8.as<double>(), &L->maxb);
         hipLaunchKernelGGL(k_gt_rootof, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, nd,
                            G.grootof.as<int>());
         int64_t nb64 = 0;
@@ -1283,7 +1779,7 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
                                   &nb64));
         nb = (int)nb64;
         int maxb = 0;
-        GG_HIP(hipMemcpyAsync(&maxb, G.gerr.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost,
+        GG_HIP(hipMemcpyAsync(&maxb, &L->maxb, sizeof(int), hipMemcpyDeviceToHost,
                               st));
         GG_HIP(hipStreamSynchronize(st));
         G.maxBucket = maxb;     // > 64 only for cells of coincident particles (pkd.c:2489)

@@ -79,7 +79,9 @@ struct GravDev {
     DevBuf broot;          // per active bucket: the root of its tree
     DevBuf tint, tdbl;     // per node: 6 ints, 8 doubles (gg_tree_info's layout)
     // tree build scratch
-    DevBuf gpn, gF, gposR, gnode, gbox, gnch, gchoff, gerr, groot, gcm;
+    DevBuf gposR, gnode, gbox, gtile, gflag, gtcnt, gunit, glev, gchoff, groot, gcm;
+    static constexpr int NHST = 32;
+    int *hst = nullptr;             // pinned words the build's kernels tell the host
     DevBuf gnit, gioff, gicell, gpart, gbflag, gbb8, grootof, glroot, gdcnt, gdlist, glused, glbase, gscr;
     DevBuf ewt, emom, ewh;          // Ewald: moment partials, root moments, k-space table
     DevBuf ewl;                     // Ewald: real-space terms per slot (for fWeight)
@@ -101,10 +103,12 @@ struct GravDev {
     {
         DevBuf *all[] = {&px, &py, &pz, &pm, &ph, &pact, &perm, &wnode, &cell, &momOH, &bucket,
                          &bbox, &cnt, &off, &ent, &acc, &stats, &scan, &werr, &broot, &tint,
-                         &tdbl, &gpn, &gF, &gposR, &gnode, &gbox, &gnch, &gchoff, &gerr,
-                         &groot, &gcm, &gnit, &gioff, &gicell, &gpart, &gbflag, &gbb8, &grootof, &glroot, &gdcnt, &gdlist, &glused, &glbase, &gscr,
+                         &tdbl, &gposR, &gnode, &gbox, &gtile, &gflag, &gtcnt, &gunit, &glev,
+                         &gchoff, &groot, &gcm, &gnit, &gioff, &gicell, &gpart, &gbflag, &gbb8, &grootof, &glroot, &gdcnt, &gdlist, &glused, &glbase, &gscr,
                          &ewt, &emom, &ewh, &ewl, &qorder, &qbin, &qhist, &qnext};
         for (DevBuf *b : all) b->release();
+        if (hst) (void)hipHostFree(hst);
+        hst = nullptr;
     }
 };
 

@@ -1,0 +1,85 @@
+"""The device tree build at the sizes where its stages hand over, node for
+node and bit for bit against the CPU oracle: cells at the limits of the
+in-LDS splits (512 and 4096 particles) and one beyond, tiles that end with a
+cell, type orders that move particles over several tiles, coincident
+particles larger than either limit, and systems of both kinds in one forest.
+Everything compared is exact, so the tolerance is equality."""
+import numpy as np
+import pytest
+
+from gasoline_amd import ics
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def check(gpu, r, m, soft, nb, order, act=None, off=None):
+    with gpu.Pkd(len(m), prec=gpu.PREC_FP64) as pk:
+        pk.put("r", r)
+        pk.put("fMass", m)
+        pk.put("fSoft", soft)
+        if act is not None:
+            pk.put("iActive", act)
+        for _ in range(2):                 # a second build starts from used scratch
+            if off is None:
+                pk.build_binary(nb, 1, 0.7, order)
+            else:
+                pk.build_forest(off, nb, 1, 0.7, order)
+        root, perm, ints, dbls = pk.tree_info()
+    parts = [(0, len(m))] if off is None else list(zip(off[:-1], off[1:]))
+    n0 = 0
+    for a, b in parts:
+        if a == b:                         # an empty system has no root
+            continue
+        T = O.Tree(r[a:b], m[a:b], soft[a:b], iactive=None if act is None else act[a:b],
+                   nBucket=nb, dTheta=0.7, iOrder=order)
+        oi, od = T.nodes()
+        k = slice(n0, n0 + len(oi))
+        n0 += len(oi)
+        oi = oi[:, :5].copy()
+        oi[:, 1:3] += a                    # particle ranges of the whole store
+        for c in (3, 4):                   # node ids likewise
+            oi[oi[:, c] >= 0, c] += k.start
+        assert np.array_equal(perm[a:b], T.perm() + a)
+        assert np.array_equal(ints[k, :5], oi)
+        assert np.array_equal(dbls[k, :6], od[:, [7, 8, 9, 10, 11, 12]])
+        assert np.array_equal(dbls[k, 6], od[:, 44])
+    assert n0 == len(ints)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 512, 513, 1024, 4096, 4097, 8192, 30011])
+@pytest.mark.parametrize("order", [2, 4])
+def test_tree_at_the_stage_limits(gpu, n, order):
+    r, v, m = ics.plummer(n, seed=n)
+    m = m * np.random.default_rng(n).uniform(0.5, 1.5, n)
+    check(gpu, r, m, np.full(n, 0.01), 16, order)
+
+
+@pytest.mark.parametrize("lack", [1, 2, 3])
+def test_tree_type_orders_over_tiles(gpu, lack):
+    # particles lacking TREEACTIVE (1), ACTIVE (2), or some of either
+    n = 21000
+    r, v, m = ics.plummer(n, seed=5)
+    u = np.random.default_rng(6).uniform(size=n)
+    act = np.full(n, 3, np.uint32)
+    if lack & 1:
+        act[u < 0.4] &= ~np.uint32(2)
+    if lack & 2:
+        act[(u > 0.2) & (u < 0.7)] &= ~np.uint32(1)
+    check(gpu, r, m, np.full(n, 0.01), 8, 2, act=act)
+
+
+@pytest.mark.parametrize("clump", [600, 5000])
+def test_tree_large_coincident_bucket(gpu, clump):
+    n = 9000
+    r, v, m = ics.plummer(n, seed=8)
+    r[100:100 + clump] = r[100]
+    check(gpu, r, m, np.full(n, 0.01), 16, 4)
+
+
+def test_forest_of_large_and_small_systems(gpu):
+    sizes = [1, 4096, 0, 9000, 17, 4097, 300, 700]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    r, v, m = ics.plummer(off[-1], seed=9)
+    act = np.where(np.arange(off[-1]) % 5 == 0, 1, 3).astype(np.uint32)
+    check(gpu, r, m, np.full(off[-1], 0.01), 16, 2, act=act, off=off)
