@@ -1,31 +1,33 @@
 // Gravity tree build on the device: the tree of gasoline's pkdBuildBinary
 // (pkd.c:2627-2723), node for node.
 //
-// Large cells level by level over the whole chip, then each cell of at most
-// 4096 particles in one workgroup, then each of at most 512 in another:
-// every cell is split at the midpoint of the
-// longest axis of its particles' bounding box (pkd.c:2493-2505) unless it
-// holds nBucket particles or fewer or has no extent (pkd.c:2489).  The
-// partition reproduces pkdUpperPart's Hoare scan (pkd.c:1109-1157): a Hoare
-// scan swaps the k-th particle of the lower part that belongs above with the
-// k-th particle, counted from the top, of the upper part that belongs below,
-// so each particle's destination follows from prefix counts and the cells
-// of a level partition in parallel.  pkdActiveTypeOrder's partitions
-// (pkd.c:1304-1355) run the same way over each system.  Cells are numbered
-// in preorder afterwards, from subtree sizes.  Mass, softening and centre of
-// mass are summed as the reference sums them (buckets over their particles
-// in storage order, cells from their children, lower then upper), and
-// bounds, Bmax and fOpen2 are exact, so every quantity the walk decides on
-// is the reference's to the bit.  The multipole moments (pkdCalcCell,
-// pkd.c:2018-2135) are direct sums over each cell's particles in a fixed
-// but different order; they enter only the force arithmetic.
+// Cells split in three stages: those of more than 4096 particles level by
+// level over the whole chip, then each cell of at most 4096 in one workgroup
+// down to 512, then each of at most 512 in another, which also makes that
+// subtree's records.  Every cell is split at the midpoint of the longest axis
+// of its particles' bounding box (pkd.c:2493-2505) unless it holds nBucket
+// particles or fewer or has no extent (pkd.c:2489).  The partition reproduces
+// pkdUpperPart's Hoare scan (pkd.c:1109-1157): a Hoare scan swaps the k-th
+// particle of the lower part that belongs above with the k-th particle,
+// counted from the top, of the upper part that belongs below, so each
+// particle's destination follows from prefix counts.  pkdActiveTypeOrder's
+// partitions (pkd.c:1304-1355) run the same way over each system.  Cells get
+// their preorder ids from subtree sizes, which climb from the buckets with
+// the records.  Mass, softening and centre of mass are summed as the
+// reference sums them (buckets over their particles in storage order, cells
+// from their children, lower then upper), and bounds, Bmax and fOpen2 are
+// exact, so every quantity the walk decides on is the reference's to the
+// bit.  The multipole moments (pkdCalcCell, pkd.c:2018-2135) are sums over a
+// bucket's particles and, above, the children's moved to the cell's centre;
+// they enter only the force arithmetic, which they change by 1e-16 of itself
+// against sums over every cell's particles.
 //
 // Several independent systems build at once: each is a root of its own.
 #include "gg_internal.h"
-#include "gg_scan.h"
 
 #include <algorithm>
 #include <cfloat>
+#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -34,21 +36,27 @@ namespace {
 
 int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 
-constexpr int MOM_CH = 2048;     // particles per moment work item
-constexpr int NM = 32;           // per item: raw Q (6), O (10), H (15), Bmax
-constexpr int MOM_SMALL = 64;    // cells of at most this many particles: a thread each
 constexpr int LMAX = 512;        // cells of at most LMAX particles finish in one workgroup
 constexpr int MID = 4096;        // cells of at most MID particles reach LMAX in one workgroup
+constexpr int DMAX = 2048;       // levels above MID a tree may have
 
-constexpr int DMAX = 2048;       // depths a tree may have
-
-// Per cell in creation order.
+// A cell, in a slot of its own: the cells above LMAX from slot 0 up, the
+// subtrees of k_gt_sub from the last slot down, each in its preorder.
 struct GNode {
-    int lo, hi, par, side;       // particle range, parent, 0 lower / 1 upper
-    int ch0, ch1, dim, root;     // children (-1), split axis (-1: bucket), root cell
-    int s, size, pre, depth;     // split position, subtree size, preorder id, level
+    int lo, hi, par, root;       // particle range, parent and root slots
+    int ch0, ch1, dim, s;        // children (-1), split axis (-1: bucket), split position
+    int size, nab;               // cells and buckets with active particles of the subtree
+    int pre, bpre;               // preorder id and bucket rank (within the subtree of
+                                 // k_gt_sub; absolute for a root)
+    int sizeLo, nabLo;           // the lower child's, above LMAX
     double split;
 };
+
+// Numeric record of a cell: mass, softening, centre of mass, the largest
+// squared distance of a particle from it, and the raw moments about it of
+// second (6: xx yy zz xy xz yz), third (10) and fourth (15) order.
+constexpr int GM_B = 5, GM_Q = 6, GM_T = 12, GM_F = 22;
+constexpr int gm_stride(int order) { return order >= 4 ? 37 : (order == 3 ? 22 : 12); }
 
 // ------------------------------------------------------------ levels
 // Cells of more than MID particles split level by level over tiles of ts
@@ -63,11 +71,13 @@ struct GLevel {
     int a, b;            // cells of the level: ids a..b-1
     int ntile;           // tiles of its splitting cells
     int nunit;           // cells left to k_gt_mid so far
-    int next;            // first free node id once the levels are done
-    int err;             // 1: a split left one side empty
+    int next;            // slots taken from the first one up
+    int nloc;            // slots taken from the last one down
+    int nsub;            // cells left to k_gt_sub
+    int err;             // 1: a split left one side empty, 2: out of slots
     int need[2];         // particles lacking a type bit of each order
     int maxb;            // largest bucket
-    int maxdep;          // deepest cell k_gt_mid made
+    int lv[DMAX + 1];    // first cell of each level
 };
 
 // Doubles as unsigned integers of the same order, for atomic min and max.
@@ -104,7 +114,8 @@ __device__ __forceinline__ int root_of(int i, int nr, const int *__restrict__ rl
 }
 
 // Root cells, their empty bounds and the level state.
-__global__ void k_gt_roots(int nr, const int *__restrict__ rlo, const int *__restrict__ rhi,
+__global__ void k_gt_roots(int n, int nr, const int *__restrict__ rlo,
+                           const int *__restrict__ rhi,
                            GNode *__restrict__ nd, unsigned long long *__restrict__ box,
                            int *__restrict__ unit, GLevel *__restrict__ L)
 {
@@ -112,19 +123,18 @@ __global__ void k_gt_roots(int nr, const int *__restrict__ rlo, const int *__res
     if (k == 0) {
         L->a = 0;
         L->b = L->next = nr;
-        L->ntile = L->nunit = L->err = L->need[0] = L->need[1] = L->maxb = L->maxdep = 0;
+        L->ntile = L->nunit = L->nloc = L->nsub = L->err = 0;
+        L->need[0] = L->need[1] = L->maxb = 0;
     }
     if (k >= nr) return;
     GNode &g = nd[k];
-    g.lo = rlo[k];
-    g.hi = rhi[k];
+    g.lo = nr > 1 ? rlo[k] : 0;
+    g.hi = nr > 1 ? rhi[k] : n - 1;
     g.par = -1;
-    g.side = -1;
     g.root = k;
     g.ch0 = g.ch1 = -1;
     g.dim = -1;
     g.split = 0.0;
-    g.depth = 0;
     box_init(box + 6 * (size_t)k);
     unit[k] = k;
 }
@@ -229,7 +239,7 @@ __global__ void k_gt_tell(const int *__restrict__ v, int *__restrict__ host)
 // for it: 4-6 us a level, against the three scans, the decision and id
 // kernels and the host's wait it replaces.
 constexpr int CTL_T = 1024;
-__global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, GLevel *L,
+__global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, int cap, GLevel *L,
                                                   GNode *__restrict__ nd,
                                                   const unsigned long long *__restrict__ box,
                                                   unsigned long long *__restrict__ kbox,
@@ -263,7 +273,9 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, G
                 }
                 bool extent = false;
                 for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
-                if (extent) {
+                if (extent && b + 2 * (c - a) + 2 > cap) {   // (a bound on its children's slots)
+                    atomicOr(&L->err, 2);
+                } else if (extent) {
                     int d = 0;
                     for (int q = 1; q < 3; ++q)
                         if (bmax[q] - bmin[q] > bmax[d] - bmin[d]) d = q;
@@ -315,12 +327,10 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, G
             for (int q = 0; q < 2; ++q) {
                 GNode &h = nd[b + kid + q];
                 h.par = c;
-                h.side = q;
                 h.root = g.root;
                 h.ch0 = h.ch1 = -1;
                 h.dim = -1;
                 h.split = 0.0;
-                h.depth = depth + 1;
                 box_init(kbox + 6 * (size_t)(kid + q));
             }
         }
@@ -344,11 +354,11 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, G
     if (tid == 0) {
         L->ntile = ntl;
         if (mode == 0) {
+            L->lv[depth] = a;
             L->a = b;
             L->b = L->next = b + 2 * nsp;
             L->nunit = nunit0 + nun;
             tell_host(host + 1, nunit0 + nun);
-            tell_host(host + 2, b + 2 * nsp);
         }
         tell_host(host, ntl);
     }
@@ -556,19 +566,24 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
 
 // The cells of the unit list, each by one workgroup: a cell of LMAX..MID
 // particles is split in LDS, level by level with the rules above, until its
-// parts hold at most LMAX (marked for k_gt_local, dim -2, or left buckets).
+// parts hold at most LMAX (listed for k_gt_sub).  The cells it closes (split,
+// or coincident and left buckets) are listed in seg from the cell's first
+// particle on, level by level, with the levels' ends in segl and their
+// numbers in useg, for the upward pass.
 // At most MID / LMAX parts are open at a time, so a level is a handful of
 // wavefront passes over the particles between barriers (7 us measured on one
 // full cell) instead of four launches.  Flags are bits, 64 particles a word, and ranks come
 // from a prefix over the 64 words.  MID is what the LDS holds: 124 KB, one
 // workgroup per CU.
 constexpr int MID_T = 1024, MID_O = MID / LMAX, MID_W = MID / 64;
+static_assert(MID_O <= 64, "one lane per open part");
 static_assert(MID_W == 64, "one wavefront scans the flag words");
-__global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, GLevel *L,
-                                                  int nBucket, GNode *__restrict__ nd,
+__global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, int cap,
+                                                  GLevel *L, GNode *__restrict__ nd,
                                                   double *__restrict__ px, double *__restrict__ py,
                                                   double *__restrict__ pz, int *__restrict__ perm,
-                                                  int *__restrict__ err)
+                                                  int *__restrict__ sub, int *__restrict__ seg,
+                                                  int *__restrict__ segl, int2 *__restrict__ useg)
 {
 #pragma clang fp contract(off)
     __shared__ double lx[MID], ly[MID], lz[MID];
@@ -579,14 +594,21 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     __shared__ int olo[2][MID_O], ohi[2][MID_O], onode[2][MID_O];
     __shared__ unsigned long long cb[MID_O][6];
     __shared__ double csplit[MID_O];
-    __shared__ int cdim[MID_O], nopen[2];
+    __shared__ int cdim[MID_O], nopen[2], full;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int rootId = unit[blockIdx.x];
     const int glo = nd[rootId].lo, cnt = nd[rootId].hi - glo + 1;
-    const int troot = nd[rootId].root, rdepth = nd[rootId].depth;
-    if (cnt > MID) return;               // coincident particles: a bucket
-    if (cnt <= LMAX) {
-        if (tid == 0 && cnt > nBucket) nd[rootId].dim = -2;
+    const int troot = nd[rootId].root;
+    if (cnt > MID || cnt <= LMAX) {
+        if (tid == 0) {
+            useg[blockIdx.x] = make_int2(cnt > MID, cnt > MID);
+            if (cnt > MID) {             // coincident particles: a bucket
+                seg[glo] = rootId;
+                segl[glo] = 1;
+            } else {
+                sub[atomicAdd(&L->nsub, 1)] = rootId;
+            }
+        }
         return;
     }
     for (int i = tid; i < cnt; i += MID_T) {
@@ -600,6 +622,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
         ohi[0][0] = cnt - 1;
         onode[0][0] = rootId;
         nopen[0] = 1;
+        full = 0;
         fbits[MID_W] = 0;
     }
     __syncthreads();
@@ -609,7 +632,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     };
     const int w0 = w * (MID / (MID_T / 64));             // this wavefront's particles
     constexpr int WN = MID / MID_T;                      // its words
-    int cur = 0, depth = 0;
+    int cur = 0, depth = 0, nseg = 0;
     for (; nopen[cur] > 0; ++depth) {
         const int no = nopen[cur];
         if (tid < 6 * no) cb[tid / 6][tid % 6] = tid % 6 < 3 ? ~0ull : 0ull;
@@ -701,14 +724,32 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
                 if (cdim[lane] >= 0) {
                     s = lo + F(hi + 1) - F(lo);
                     sp = s > lo && s <= hi;
-                    if (!sp) atomicOr(err, 1);           // one side empty: reported
+                    if (!sp) atomicOr(&L->err, 1);       // one side empty: reported
                 }
             }
-            const unsigned long long ms = __ballot(sp);
-            int id0 = 0;
-            if (lane == 0 && ms) id0 = atomicAdd(&L->next, 2 * __popcll(ms));
-            id0 = __shfl(id0, 0) + 2 * __popcll(ms & ((1ull << lane) - 1));
+            const bool sub0 = sp && s - lo <= LMAX, sub1 = sp && hi - s + 1 <= LMAX;
+            const unsigned long long ms = __ballot(sp), u0 = __ballot(sub0), u1 = __ballot(sub1);
+            const unsigned long long below = (1ull << lane) - 1;
+            int got = 0;                                 // slots (lane 0), list places (lane 1)
+            if (lane < 2) {
+                const int want = lane ? __popcll(u0) + __popcll(u1) : 2 * __popcll(ms);
+                if (want) got = atomicAdd(lane ? &L->nsub : &L->next, want);
+            }
+            const int id0 = __shfl(got, 0) + 2 * __popcll(ms & below);
+            const int su0 = __shfl(got, 1) + __popcll(u0 & below) + __popcll(u1 & below);
+            if (__shfl(got, 0) + 2 * __popcll(ms) > cap) {   // out of slots: built again
+                sp = false;
+                if (lane == 0) {
+                    atomicOr(&L->err, 2);
+                    full = 1;
+                }
+            }
+            if (sp && sub0) sub[su0] = id0;
+            if (sp && sub1) sub[su0 + sub0] = id0 + 1;
             const int me = in ? onode[cur][lane] : 0;
+            if (in) seg[glo + nseg + lane] = me;
+            nseg += no;
+            if (lane == 0) segl[glo + depth] = nseg;
             if (sp) {
                 GNode &g = nd[me];
                 g.dim = cdim[lane];
@@ -726,12 +767,10 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
                     h.lo = glo + a0;
                     h.hi = glo + a1;
                     h.par = me;
-                    h.side = q;
                     h.root = troot;
                     h.ch0 = h.ch1 = -1;
                     h.split = 0.0;
-                    h.depth = rdepth + depth + 1;
-                    h.dim = !open && a1 - a0 + 1 > nBucket ? -2 : -1;
+                    h.dim = -1;
                 }
                 const int at = nopen[cur ^ 1] + __popcll(mo & ((1ull << lane) - 1));
                 if (open) {
@@ -746,6 +785,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
             }
         }
         __syncthreads();
+        if (full) return;
         for (int k = 0; k < WN; ++k) {                   // the swaps
             if (part[k] < 0) continue;
             const int i = w0 + 64 * k + lane, j = posR[part[k]];
@@ -757,7 +797,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
         cur ^= 1;
         __syncthreads();
     }
-    if (tid == 0) atomicMax(&L->maxdep, rdepth + depth);
+    if (tid == 0) useg[blockIdx.x] = make_int2(nseg, depth);
     for (int i = tid; i < cnt; i += MID_T) {
         px[glo + i] = lx[i];
         py[glo + i] = ly[i];
@@ -766,689 +806,869 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     }
 }
 
-// Work items of the cells [a, b): ceil(count / ch) each for cells of more
-// than minc particles, none for the others.
-__global__ void k_gt_items(int a, int b, int ch, int minc, const GNode *__restrict__ nd,
-                           int *__restrict__ nit)
+// ------------------------------------------------------ numeric records
+// Positions of the raw moments: third order xxx xyy xxy yyy xxz yyz xyz xzz
+// yzz zzz, fourth xxxx xyyy xxxy yyyy xxxz yyyz xxyy xxyz xyyz xxzz xyzz
+// xzzz yyzz yzzz zzzz.
+__device__ constexpr int T_IX[10][3] = {{0, 0, 0}, {0, 1, 1}, {0, 0, 1}, {1, 1, 1}, {0, 0, 2},
+                                        {1, 1, 2}, {0, 1, 2}, {0, 2, 2}, {1, 2, 2}, {2, 2, 2}};
+__device__ constexpr int F_IX[15][4] = {{0, 0, 0, 0}, {0, 1, 1, 1}, {0, 0, 0, 1}, {1, 1, 1, 1},
+                                        {0, 0, 0, 2}, {1, 1, 1, 2}, {0, 0, 1, 1}, {0, 0, 1, 2},
+                                        {0, 1, 1, 2}, {0, 0, 2, 2}, {0, 1, 2, 2}, {0, 2, 2, 2},
+                                        {1, 1, 2, 2}, {1, 2, 2, 2}, {2, 2, 2, 2}};
+__device__ constexpr int q_at(int a, int b)   // xx yy zz xy xz yz
 {
-    const int c = a + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= b) return;
-    const int cnt = nd[c].hi - nd[c].lo + 1;
-    nit[c - a] = cnt > minc ? (cnt + ch - 1) / ch : 0;
+    return a == b ? a : a + b + 2;
+}
+__device__ constexpr int t_at(int a, int b, int c)   // any order of indices
+{
+    const int n[3] = {(a == 0) + (b == 0) + (c == 0), (a == 1) + (b == 1) + (c == 1),
+                      (a == 2) + (b == 2) + (c == 2)};
+    for (int k = 0; k < 10; ++k) {
+        int m[3] = {0, 0, 0};
+        for (int j = 0; j < 3; ++j) ++m[T_IX[k][j]];
+        if (m[0] == n[0] && m[1] == n[1] && m[2] == n[2]) return k;
+    }
+    return -1;
 }
 
-// Subtree sizes and preorder ids, over the nodes of one depth (list).
-__global__ void k_gt_size(int m, const int *__restrict__ list, GNode *__restrict__ nd)
+// The raw moments of a particle of mass m at d from the expansion centre,
+// added to g.
+template <int ORDER>
+__device__ __forceinline__ void mom_particle(double m, const double *d, double *g)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    GNode &g = nd[list[k]];
-    g.size = 1 + (g.ch0 >= 0 ? nd[g.ch0].size : 0) + (g.ch1 >= 0 ? nd[g.ch1].size : 0);
+    double q[6];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = a; b < 3; ++b) {
+            q[q_at(a, b)] = m * d[a] * d[b];
+            g[GM_Q + q_at(a, b)] += q[q_at(a, b)];
+        }
+    if constexpr (ORDER >= 3) {
+        double t[10];
+#pragma unroll
+        for (int k = 0; k < 10; ++k) {
+            t[k] = q[q_at(T_IX[k][0], T_IX[k][1])] * d[T_IX[k][2]];
+            g[GM_T + k] += t[k];
+        }
+        if constexpr (ORDER >= 4) {
+#pragma unroll
+            for (int k = 0; k < 15; ++k)
+                g[GM_F + k] += t[t_at(F_IX[k][0], F_IX[k][1], F_IX[k][2])] * d[F_IX[k][3]];
+        }
+    }
 }
 
-__global__ void k_gt_pre(int m, const int *__restrict__ list, GNode *__restrict__ nd)
+// A child's raw moments c moved from its centre of mass to the parent's,
+// which lies -d from it, and added to g.  The child's first moment about
+// its own centre vanishes.
+template <int ORDER>
+__device__ __forceinline__ void mom_shift(const double *c, const double *d, double *g)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    const GNode &g = nd[list[k]];
-    if (g.ch0 >= 0) nd[g.ch0].pre = g.pre + 1;
-    if (g.ch1 >= 0) nd[g.ch1].pre = g.pre + 1 + (g.ch0 >= 0 ? nd[g.ch0].size : 0);
+    const double m = c[0];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = a; b < 3; ++b)
+            g[GM_Q + q_at(a, b)] += c[GM_Q + q_at(a, b)] + m * d[a] * d[b];
+    if constexpr (ORDER >= 3) {
+#pragma unroll
+        for (int k = 0; k < 10; ++k) {
+            constexpr auto &X = T_IX;
+            const int i = X[k][0], j = X[k][1], l = X[k][2];
+            g[GM_T + k] += c[GM_T + k] + c[GM_Q + q_at(i, j)] * d[l]
+                           + c[GM_Q + (i <= l ? q_at(i, l) : q_at(l, i))] * d[j]
+                           + c[GM_Q + (j <= l ? q_at(j, l) : q_at(l, j))] * d[i]
+                           + m * d[i] * d[j] * d[l];
+        }
+    }
+    if constexpr (ORDER >= 4) {
+#pragma unroll
+        for (int k = 0; k < 15; ++k) {
+            const int i = F_IX[k][0], j = F_IX[k][1], l = F_IX[k][2], o = F_IX[k][3];
+            // i <= j <= l <= o throughout F_IX
+            g[GM_F + k] += c[GM_F + k] + c[GM_T + t_at(i, j, l)] * d[o]
+                           + c[GM_T + t_at(i, j, o)] * d[l] + c[GM_T + t_at(i, l, o)] * d[j]
+                           + c[GM_T + t_at(j, l, o)] * d[i]
+                           + c[GM_Q + q_at(i, j)] * d[l] * d[o] + c[GM_Q + q_at(i, l)] * d[j] * d[o]
+                           + c[GM_Q + q_at(i, o)] * d[j] * d[l] + c[GM_Q + q_at(j, l)] * d[i] * d[o]
+                           + c[GM_Q + q_at(j, o)] * d[i] * d[l] + c[GM_Q + q_at(l, o)] * d[i] * d[j]
+                           + m * d[i] * d[j] * d[l] * d[o];
+        }
+    }
 }
 
-// Nodes by depth: a count per depth, then each node to its depth's list.
-// Each workgroup counts in LDS
-// first, so the global counters see one atomic per workgroup and depth.
-
-__global__ __launch_bounds__(256) void k_gt_depth_count(int nn, int ndep,
-                                                        const GNode *__restrict__ nd,
-                                                        int *__restrict__ cnt)
-{
-    __shared__ int h[DMAX];
-    for (int d = threadIdx.x; d < ndep; d += 256) h[d] = 0;
-    __syncthreads();
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c < nn) atomicAdd(&h[nd[c].depth], 1);
-    __syncthreads();
-    for (int d = threadIdx.x; d < ndep; d += 256)
-        if (h[d]) atomicAdd(&cnt[d], h[d]);
-}
-
-__global__ __launch_bounds__(256) void k_gt_depth_list(int nn, int ndep,
-                                                       const GNode *__restrict__ nd,
-                                                       int *__restrict__ cur,
-                                                       int *__restrict__ list)
-{
-    __shared__ int h[DMAX], b0[DMAX];
-    for (int d = threadIdx.x; d < ndep; d += 256) h[d] = 0;
-    __syncthreads();
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    const bool ok = c < nn;
-    const int dep = ok ? nd[c].depth : 0;
-    const int r = ok ? atomicAdd(&h[dep], 1) : 0;
-    __syncthreads();
-    for (int d = threadIdx.x; d < ndep; d += 256)
-        if (h[d]) b0[d] = atomicAdd(&cur[d], h[d]);
-    __syncthreads();
-    if (ok) list[b0[dep] + r] = c;
-}
-
-// Cells marked for the local build, and the scratch node slots each
-// reserves for its descendants (2 count - 2 at most).
-__global__ void k_gt_lmark(int nn, const GNode *__restrict__ nd, int *__restrict__ flag,
-                           int *__restrict__ res)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nn) return;
-    const bool l = nd[c].dim == -2;
-    flag[c] = l;
-    res[c] = l ? 2 * (nd[c].hi - nd[c].lo + 1) - 2 : 0;
-}
-
-__global__ void k_gt_lcompact(int nn, const int *__restrict__ flag, const int64_t *__restrict__ pos,
-                              int *__restrict__ list)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < nn && flag[c]) list[pos[c]] = c;
-}
-
-// The subtree of one marked cell (at most LMAX particles), built in LDS by
-// one workgroup with the rules of the level loop: per level, each cell's
-// bounds and split decision (a wavefront per cell), child ids in order,
-// then each split cell's partition by the Hoare pairing of the k-th
-// misplaced particles from either end (a wavefront per cell).  The cell is
-// local node 0; descendant k >= 1 (in creation order) goes to scratch slot
-// lres[root] + k - 1 with its links as local ids, and *used receives the
-// node count; k_gt_lcopy then moves them into place.  The particles are
-// written back in their new order.
-__global__ __launch_bounds__(256) void k_gt_local(const int *__restrict__ lroot,
-                                                  const int64_t *__restrict__ lres, int nBucket,
-                                                  GNode *__restrict__ nd, GNode *__restrict__ scr,
-                                                  int *__restrict__ used,
-                                                  double *__restrict__ px, double *__restrict__ py,
-                                                  double *__restrict__ pz, int *__restrict__ perm,
-                                                  int *__restrict__ err)
+// Mass, mass-weighted softening and centre of mass of a cell from its
+// children's, lower then upper (pkd.c:2510-2576).
+__device__ __forceinline__ void mass_children(const double *c0, const double *c1, double *g)
 {
 #pragma clang fp contract(off)
-    __shared__ double lx[LMAX], ly[LMAX], lz[LMAX];
-    __shared__ int ls[LMAX];
-    __shared__ short posR[LMAX];
-    __shared__ short qa[2][LMAX];              // cells of the current / next level
-    __shared__ short nlo[2 * LMAX], nhi[2 * LMAX];   // cell ranges (local positions)
-    __shared__ short coff[LMAX], cs[LMAX];     // child offset (-1: none), split position
-    __shared__ signed char cdim[LMAX];
-    __shared__ double csplit[LMAX];
-    __shared__ int wsum[4];
-    __shared__ int nsplit_sh;
-    const int rootId = lroot[blockIdx.x];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int glo = nd[rootId].lo, cnt = nd[rootId].hi - glo + 1;
-    const int troot = nd[rootId].root, rdepth = nd[rootId].depth;
-    GNode *const sb = scr + lres[rootId] - 1;   // local node k >= 1 at sb[k]
-    for (int i = threadIdx.x; i < cnt; i += 256) {
-        lx[i] = px[glo + i];
-        ly[i] = py[glo + i];
-        lz[i] = pz[glo + i];
-        ls[i] = perm[glo + i];
+    double M = 0.0, S = 0.0, R[3] = {0.0, 0.0, 0.0};
+    for (int k = 0; k < 2; ++k) {
+        const double *q = k ? c1 : c0;
+        const double fm = q[0];
+        M += fm;
+        S += fm * q[1];
+        for (int d = 0; d < 3; ++d) R[d] += fm * q[2 + d];
     }
-    if (threadIdx.x == 0) {
-        nlo[0] = 0;
-        nhi[0] = (short)(cnt - 1);
-        qa[0][0] = 0;
+    if (M > 0) {
+        S /= M;
+        for (int d = 0; d < 3; ++d) R[d] /= M;
     }
-    __syncthreads();
-    int nq = 1, cur = 0, nloc = 1, depth = 0;
-    while (nq > 0) {
-        // bounds, decision and lower-part count, a wavefront per cell
-        for (int t = w; t < nq; t += 4) {
-            const int k = qa[cur][t];
-            const int lo = nlo[k], hi = nhi[k];
-            double bmin[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
-            double bmax[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-            for (int i = lo + lane; i <= hi; i += 64) {
-                const double v[3] = {lx[i], ly[i], lz[i]};
-                for (int d = 0; d < 3; ++d) {
-                    bmin[d] = v[d] < bmin[d] ? v[d] : bmin[d];
-                    bmax[d] = v[d] > bmax[d] ? v[d] : bmax[d];
-                }
-            }
-            for (int o = 32; o > 0; o >>= 1)
-                for (int d = 0; d < 3; ++d) {
-                    const double l = __shfl_xor(bmin[d], o), h = __shfl_xor(bmax[d], o);
-                    bmin[d] = l < bmin[d] ? l : bmin[d];
-                    bmax[d] = h > bmax[d] ? h : bmax[d];
-                }
-            bool extent = false;
-            for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
-            int dim = -1;
-            double split = 0.0;
-            if (hi - lo + 1 > nBucket && extent) {
-                int d = 0;
-                for (int q = 1; q < 3; ++q)
-                    if (bmax[q] - bmin[q] > bmax[d] - bmin[d]) d = q;
-                dim = d;
-                split = 0.5 * (bmin[d] + bmax[d]);
-            }
-            int s = lo;
-            if (dim >= 0) {
-                const double *cc = dim == 0 ? lx : (dim == 1 ? ly : lz);
-                int nl = 0;
-                for (int c0 = lo; c0 <= hi; c0 += 64) {
-                    const int i = c0 + lane;
-                    nl += __popcll(__ballot(i <= hi && cc[i] < split));
-                }
-                s = lo + nl;
-                if (s == lo || s > hi) {   // one side empty: reported, left a bucket
-                    if (lane == 0) atomicOr(err, 1);
-                    dim = -1;
-                    s = lo;
-                }
-            }
-            if (lane == 0) {
-                GNode &g = k == 0 ? nd[rootId] : sb[k];
-                g.lo = glo + lo;
-                g.hi = glo + hi;
-                g.dim = dim;
-                g.split = dim >= 0 ? split : 0.0;
-                g.ch0 = g.ch1 = -1;
-                g.s = glo + s;
-                g.root = troot;
-                g.depth = rdepth + depth;
-                coff[t] = dim >= 0 ? 1 : 0;
-                cdim[t] = (signed char)dim;
-                csplit[t] = split;
-                cs[t] = (short)s;
-            }
-        }
-        __syncthreads();
-        {   // child offsets: exclusive sum of the split flags
-            int v[4], sum = 0;
-            for (int q = 0; q < 4; ++q) {
-                const int t = threadIdx.x * 4 + q;
-                v[q] = t < nq ? coff[t] : 0;
-                sum += v[q];
-            }
-            int inc = sum;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int u = __shfl_up(inc, o);
-                if (lane >= o) inc += u;
-            }
-            if (lane == 63) wsum[w] = inc;
-            __syncthreads();
-            int ex = inc - sum, tot = 0;
-            for (int q = 0; q < 4; ++q) {
-                if (q < w) ex += wsum[q];
-                tot += wsum[q];
-            }
-            for (int q = 0; q < 4; ++q) {
-                const int t = threadIdx.x * 4 + q;
-                if (t < nq) coff[t] = v[q] ? (short)ex : (short)-1;
-                ex += v[q];
-            }
-            if (threadIdx.x == 0) nsplit_sh = tot;
-        }
-        __syncthreads();
-        const int nsplit = nsplit_sh;
-        // partitions and children, a wavefront per split cell
-        for (int t = w; t < nq; t += 4) {
-            const int co = coff[t];
-            if (co < 0) continue;
-            const int k = qa[cur][t];
-            const int lo = nlo[k], hi = nhi[k], s = cs[t];
-            const double split = csplit[t];
-            const double *cc = cdim[t] == 0 ? lx : (cdim[t] == 1 ? ly : lz);
-            const int nl = s - lo;
-            int run = 0;
-            for (int c0 = lo; c0 <= hi; c0 += 64) {   // upper positions holding a lower particle
-                const int i = c0 + lane;
-                const bool f = i <= hi && cc[i] < split;
-                const unsigned long long m = __ballot(f);
-                const int incl = run + __popcll(m & (lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1)));
-                if (f && i >= s) posR[lo + (nl - incl)] = (short)i;
-                run += __popcll(m);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            run = 0;
-            for (int c0 = lo; c0 < s; c0 += 64) {     // lower positions holding an upper one
-                const int i = c0 + lane;
-                const bool in = i < s;
-                const bool f = in && cc[i] < split;
-                const unsigned long long m = __ballot(f);
-                const int excl = run + __popcll(m & ((1ull << lane) - 1));
-                if (in && !f) {
-                    const int j = posR[lo + (i - lo) - excl];
-                    double d = lx[i]; lx[i] = lx[j]; lx[j] = d;
-                    d = ly[i]; ly[i] = ly[j]; ly[j] = d;
-                    d = lz[i]; lz[i] = lz[j]; lz[j] = d;
-                    const int u = ls[i]; ls[i] = ls[j]; ls[j] = u;
-                }
-                run += __popcll(m);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (lane == 0) {
-                const int a0 = nloc + 2 * co, a1 = a0 + 1;
-                nlo[a0] = (short)lo;
-                nhi[a0] = (short)(s - 1);
-                nlo[a1] = (short)s;
-                nhi[a1] = (short)hi;
-                qa[cur ^ 1][2 * co] = (short)a0;
-                qa[cur ^ 1][2 * co + 1] = (short)a1;
-                GNode &g = k == 0 ? nd[rootId] : sb[k];
-                g.ch0 = a0;
-                g.ch1 = a1;
-                sb[a0].par = k;
-                sb[a0].side = 0;
-                sb[a1].par = k;
-                sb[a1].side = 1;
-            }
-        }
-        __syncthreads();
-        nloc += 2 * nsplit;
-        nq = 2 * nsplit;
-        cur ^= 1;
-        ++depth;
-    }
-    for (int i = threadIdx.x; i < cnt; i += 256) {
-        px[glo + i] = lx[i];
-        py[glo + i] = ly[i];
-        pz[glo + i] = lz[i];
-        perm[glo + i] = ls[i];
-    }
-    if (threadIdx.x == 0) used[blockIdx.x] = nloc - 1;
+    g[0] = M;
+    g[1] = S;
+    for (int d = 0; d < 3; ++d) g[2 + d] = R[d];
 }
 
-// The descendants of local build r from scratch to nodes nng + dbase[r] ...,
-// links turned from local ids (0: the marked cell) to node ids.
-__global__ __launch_bounds__(256) void k_gt_lcopy(const int *__restrict__ lroot,
-                                                  const int64_t *__restrict__ lres,
-                                                  const int *__restrict__ used,
-                                                  const int64_t *__restrict__ dbase, int nng,
-                                                  GNode *__restrict__ nd,
-                                                  const GNode *__restrict__ scr)
-{
-    const int r = blockIdx.x, rootId = lroot[r], u = used[r];
-    const int db = nng + (int)dbase[r];
-    const GNode *const sb = scr + lres[rootId] - 1;
-    auto fin = [&](int k) { return k < 0 ? -1 : (k == 0 ? rootId : db + k - 1); };
-    for (int k = 1 + threadIdx.x; k <= u; k += 256) {
-        GNode g = sb[k];
-        g.ch0 = fin(g.ch0);
-        g.ch1 = fin(g.ch1);
-        g.par = fin(g.par);
-        nd[db + k - 1] = g;
-    }
-    if (threadIdx.x == 0) {
-        GNode &g = nd[rootId];
-        g.ch0 = fin(g.ch0);
-        g.ch1 = fin(g.ch1);
-    }
-}
-
-// Storage-order particle fields: masses, softenings, type bits by source.
-__global__ void k_gt_gather(int n, const int *__restrict__ src, const double *__restrict__ m,
-                            const double *__restrict__ h, const uint32_t *__restrict__ bits,
-                            double *__restrict__ pm, double *__restrict__ ph,
-                            uint32_t *__restrict__ pact)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int s = src[i];
-    pm[i] = m[s];
-    ph[i] = h[s];
-    pact[i] = bits[s];
-}
-
-// Mass, mass-weighted softening and centre of mass (pkd.c:2510-2576):
-// buckets over their particles in storage order, cells from their
-// children, lower then upper.  Deepest level first, one depth per launch.
-__global__ void k_gt_mass(int m, const int *__restrict__ list, const GNode *__restrict__ nd,
-                          const double *__restrict__ x, const double *__restrict__ y,
-                          const double *__restrict__ z, const double *__restrict__ pm,
-                          const double *__restrict__ ph, double *__restrict__ cm)
+// Squared distance as Bmax takes it (pkd.c:2018-2135), before its root.
+__device__ __forceinline__ double cm_d2(double x, double y, double z, const double *cm)
 {
 #pragma clang fp contract(off)
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    const int c = list[k];
-    const GNode &g = nd[c];
-    double fm, M = 0.0, S = 0.0, R[3] = {0.0, 0.0, 0.0};
-    if (g.dim >= 0) {
-        for (int k = 0; k < 2; ++k) {
-            const int ch = k ? g.ch1 : g.ch0;
-            if (ch == -1) continue;
-            const double *q = cm + 5 * (size_t)ch;
-            fm = q[0];
-            M += fm;
-            S += fm * q[1];
-            for (int d = 0; d < 3; ++d) R[d] += fm * q[2 + d];
-        }
-    } else {
-        for (int i = g.lo; i <= g.hi; ++i) {
-            fm = pm[i];
-            M += fm;
-            S += fm * ph[i];
-            R[0] += fm * x[i];
-            R[1] += fm * y[i];
-            R[2] += fm * z[i];
+    const double dx = x - cm[0], dy = y - cm[1], dz = z - cm[2];
+    return dx * dx + dy * dy + dz * dz;
+}
+
+// A bucket's record by one thread: mass, softening and centre of mass over
+// its particles in storage order, then the moments, and bb: the active
+// particles' bounds, the largest softening and their number (pkd.c:2916-2937,
+// walk.c:319-324).  get(i, p, m, h) loads particle i; returns whether active.
+template <int ORDER, typename Get>
+__device__ __forceinline__ int bucket_record(int lo, int hi, Get get, double *g, double *bb)
+{
+#pragma clang fp contract(off)
+    double M = 0.0, S = 0.0, R[3] = {0.0, 0.0, 0.0};
+    double bl[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, bh[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+    double fsm = 0.0;
+    int na = 0;
+    for (int i = lo; i <= hi; ++i) {
+        double p[3], m, h;
+        const bool act = get(i, p, m, h);
+        M += m;
+        S += m * h;
+        for (int d = 0; d < 3; ++d) R[d] += m * p[d];
+        if (h > fsm) fsm = h;
+        if (!act) continue;
+        ++na;
+        for (int d = 0; d < 3; ++d) {
+            if (p[d] < bl[d]) bl[d] = p[d];
+            if (p[d] > bh[d]) bh[d] = p[d];
         }
     }
     if (M > 0) {
         S /= M;
         for (int d = 0; d < 3; ++d) R[d] /= M;
     }
-    double *o = cm + 5 * (size_t)c;
-    o[0] = M;
-    o[1] = S;
-    for (int d = 0; d < 3; ++d) o[2 + d] = R[d];
-}
-
-// Cell of each moment item (a thread per cell writes its items).
-__global__ void k_gt_itemcell(int nn, const int64_t *__restrict__ ioff, int *__restrict__ icell)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nn) return;
-    for (int64_t k = ioff[c]; k < ioff[c + 1]; ++k) icell[k] = c;
-}
-
-// One particle's terms of the moments about (cx, cy, cz): raw Q (6),
-// reduced O (10) and H (15), and its distance for Bmax.
-template <int ORDER>
-__device__ __forceinline__ void mom_accum(double mm, double dx, double dy, double dz, double *Q,
-                                          double *O, double *H, double &Bmax)
-{
-#pragma clang fp contract(off)
-    constexpr bool wantO = ORDER >= 3, wantH = ORDER >= 4;
-    const double d2 = dx * dx + dy * dy + dz * dz;
-    const double d1 = sqrt(d2);
-    if (d1 > Bmax) Bmax = d1;
-    if (wantH) {
-        H[0] += mm * (dx * dx * dx * dx - 6.0 / 7.0 * d2 * (dx * dx - 0.1 * d2));
-        H[1] += mm * (dx * dy * dy * dy - 3.0 / 7.0 * d2 * dx * dy);
-        H[2] += mm * (dx * dx * dx * dy - 3.0 / 7.0 * d2 * dx * dy);
-        H[3] += mm * (dy * dy * dy * dy - 6.0 / 7.0 * d2 * (dy * dy - 0.1 * d2));
-        H[4] += mm * (dx * dx * dx * dz - 3.0 / 7.0 * d2 * dx * dz);
-        H[5] += mm * (dy * dy * dy * dz - 3.0 / 7.0 * d2 * dy * dz);
-        H[6] += mm * (dx * dx * dy * dy - 1.0 / 7.0 * d2 * (dx * dx + dy * dy - 0.2 * d2));
-        H[7] += mm * (dx * dx * dy * dz - 1.0 / 7.0 * d2 * dy * dz);
-        H[8] += mm * (dx * dy * dy * dz - 1.0 / 7.0 * d2 * dx * dz);
-        H[9] += mm * (dx * dx * dz * dz - 1.0 / 7.0 * d2 * (dx * dx + dz * dz - 0.2 * d2));
-        H[10] += mm * (dx * dy * dz * dz - 1.0 / 7.0 * d2 * dx * dy);
-        H[11] += mm * (dx * dz * dz * dz - 3.0 / 7.0 * d2 * dx * dz);
-        H[12] += mm * (dy * dy * dz * dz - 1.0 / 7.0 * d2 * (dy * dy + dz * dz - 0.2 * d2));
-        H[13] += mm * (dy * dz * dz * dz - 3.0 / 7.0 * d2 * dy * dz);
-        H[14] += mm * (dz * dz * dz * dz - 6.0 / 7.0 * d2 * (dz * dz - 0.1 * d2));
+    g[0] = M;
+    g[1] = S;
+    for (int d = 0; d < 3; ++d) g[2 + d] = R[d];
+    double b2 = 0.0;
+    for (int i = lo; i <= hi; ++i) {
+        double p[3], m, h;
+        get(i, p, m, h);
+        const double d2 = cm_d2(p[0], p[1], p[2], R);
+        if (d2 > b2) b2 = d2;
+        const double d[3] = {p[0] - R[0], p[1] - R[1], p[2] - R[2]};
+        mom_particle<ORDER>(m, d, g);
     }
-    if (wantO) {
-        O[0] += mm * (dx * dx * dx - 0.6 * d2 * dx);
-        O[1] += mm * (dx * dy * dy - 0.2 * d2 * dx);
-        O[2] += mm * (dx * dx * dy - 0.2 * d2 * dy);
-        O[3] += mm * (dy * dy * dy - 0.6 * d2 * dy);
-        O[4] += mm * (dx * dx * dz - 0.2 * d2 * dz);
-        O[5] += mm * (dy * dy * dz - 0.2 * d2 * dz);
-        O[6] += mm * dx * dy * dz;
-        O[7] += mm * (dx * dz * dz - 0.2 * d2 * dx);
-        O[8] += mm * (dy * dz * dz - 0.2 * d2 * dy);
-        O[9] += mm * (dz * dz * dz - 0.6 * d2 * dz);
+    g[GM_B] = b2;
+    for (int d = 0; d < 3; ++d) {
+        bb[d] = bl[d];
+        bb[3 + d] = bh[d];
     }
-    Q[0] += mm * dx * dx;
-    Q[1] += mm * dy * dy;
-    Q[2] += mm * dz * dz;
-    Q[3] += mm * dx * dy;
-    Q[4] += mm * dx * dz;
-    Q[5] += mm * dy * dz;
+    bb[6] = fsm;
+    bb[7] = (double)na;
+    return na;
 }
 
-// Partial moments of one item (one wavefront): raw Q (6), reduced O (10)
-// and H (15) about the cell's centre of mass, and the largest distance.
-// Per-lane sums, then a fixed butterfly: the result does not depend on
-// scheduling.
-template <int ORDER>
-__global__ __launch_bounds__(256) void k_gt_moments(int nitem, const int *__restrict__ icell,
-                                                    const int64_t *__restrict__ ioff,
-                                                    const GNode *__restrict__ nd,
-                                                    const double *__restrict__ cm,
-                                                    const double *__restrict__ x,
-                                                    const double *__restrict__ y,
-                                                    const double *__restrict__ z,
-                                                    const double *__restrict__ pm,
-                                                    double *__restrict__ part)
+struct TreeArgs {
+    int nBucket, cap;                    // slots
+    GLevel *L;
+    GNode *nd;
+    double *gm, *bb8;                    // numeric record and bucket bounds per slot
+    double *px, *py, *pz, *pm, *ph;      // storage order
+    uint32_t *pact;
+    int *perm;
+    const double *m, *h;                 // caller order
+    const uint32_t *bits;
+    const int *sub;                      // cells left to k_gt_sub
+    int2 *subn;                          // their first slot and cells below them
+    const int *unit, *seg, *segl;        // cells left to k_gt_mid and what it closed
+    const int2 *useg;
+};
+
+// The subtree of one cell of at most LMAX particles, by one workgroup in LDS:
+// the splits with the rules above, then the preorder of its cells, their
+// slots, and their records from the particles that are still in LDS.  A level
+// of splits takes one barrier: a part of more than 32 particles is split by
+// one wavefront, two smaller ones by its halves, and each reserves its
+// children with LDS atomics.  Sizes and records climb from the buckets, the
+// second child to arrive computing the parent, so a level needs no barrier
+// there.  Moments come from the children's by shifting (31 values, ~400
+// operations a cell) instead of from every particle of every cell.
+constexpr int SUB_T = 256, SN = 2 * LMAX;
+template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs A)
 {
 #pragma clang fp contract(off)
-    const int it = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (it >= nitem) return;
-    const int c = icell[it];
-    const GNode &g = nd[c];
-    if (g.hi - g.lo + 1 <= MOM_SMALL) return;   // k_gt_moments_small's
-    const int first = g.lo + (int)(it - ioff[c]) * MOM_CH;
-    const int last = min(g.hi, first + MOM_CH - 1);
-    const double cx = cm[5 * (size_t)c + 2], cy = cm[5 * (size_t)c + 3], cz = cm[5 * (size_t)c + 4];
-    constexpr bool wantO = ORDER >= 3, wantH = ORDER >= 4;
-    double Q[6] = {0, 0, 0, 0, 0, 0}, O[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double H[15] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double Bmax = 0.0;
-    for (int i = first + lane; i <= last; i += 64) {
-        const double mm = pm[i];
-        const double dx = x[i] - cx, dy = y[i] - cy, dz = z[i] - cz;
-        mom_accum<ORDER>(mm, dx, dy, dz, Q, O, H, Bmax);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        for (int k = 0; k < 6; ++k) Q[k] += __shfl_xor(Q[k], o);
-        if (wantO)
-            for (int k = 0; k < 10; ++k) O[k] += __shfl_xor(O[k], o);
-        if (wantH)
-            for (int k = 0; k < 15; ++k) H[k] += __shfl_xor(H[k], o);
-        Bmax = fmax(Bmax, __shfl_xor(Bmax, o));
-    }
-    if (lane == 0) {
-        double *p = part + (size_t)NM * it;
-        for (int k = 0; k < 6; ++k) p[k] = Q[k];
-        for (int k = 0; k < 10; ++k) p[6 + k] = O[k];
-        for (int k = 0; k < 15; ++k) p[16 + k] = H[k];
-        p[31] = Bmax;
+    constexpr int GS = gm_stride(ORDER);
+    __shared__ double lx[LMAX], ly[LMAX], lz[LMAX], nsp[SN];
+    __shared__ double lm[LMAX], lh[LMAX];
+    __shared__ int ls[LMAX], arr[SN];
+    __shared__ short posR[LMAX];
+    __shared__ short nlo[SN], nhi[SN], npar[SN], nch[SN], nsz[SN], nac[SN], npre[SN], nbp[SN];
+    __shared__ signed char ndm[SN];
+    __shared__ unsigned char lact[LMAX];
+    __shared__ short qa[3][2][LMAX / 2];  // open cells of a level: larger, smaller than 33
+    __shared__ int qn[3][2], nloc_sh, slot_sh, maxb_sh;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, half = lane >> 5, l32 = lane & 31;
+    if (A.L->err & 2) return;            // out of slots: built again
+    const int nsub = A.L->nsub;
+    for (int t = blockIdx.x; t < nsub; t += gridDim.x) {
+        const int root = A.sub[t];
+        const int glo = A.nd[root].lo, cnt = A.nd[root].hi - glo + 1, troot = A.nd[root].root;
+        for (int i = tid; i < cnt; i += SUB_T) {
+            lx[i] = A.px[glo + i];
+            ly[i] = A.py[glo + i];
+            lz[i] = A.pz[glo + i];
+            ls[i] = A.perm[glo + i];
+        }
+        if (tid == 0) {
+            nlo[0] = 0;
+            nhi[0] = (short)(cnt - 1);
+            npar[0] = nch[0] = -1;
+            ndm[0] = -1;
+            nsp[0] = 0.0;
+            nloc_sh = 1;
+            maxb_sh = 0;
+            for (int k = 0; k < 3; ++k) qn[k][0] = qn[k][1] = 0;
+            if (cnt > A.nBucket) {
+                const int big = cnt > 32 ? 0 : 1;
+                qa[0][big][0] = 0;
+                qn[0][big] = 1;
+            }
+        }
+        __syncthreads();
+        // the split cell k (range lo..hi, lower part lo..s-1): its children,
+        // queued for the next level if they may split
+        auto children = [&](int k, int lo, int hi, int s, int dim, double split, int nxt) {
+            const int c = atomicAdd(&nloc_sh, 2);
+            ndm[k] = (signed char)dim;
+            nsp[k] = split;
+            nch[k] = (short)c;
+            for (int q = 0; q < 2; ++q) {
+                const int a0 = q ? s : lo, a1 = q ? hi : s - 1, m = a1 - a0 + 1;
+                nlo[c + q] = (short)a0;
+                nhi[c + q] = (short)a1;
+                npar[c + q] = (short)k;
+                nch[c + q] = -1;
+                ndm[c + q] = -1;
+                nsp[c + q] = 0.0;
+                if (m > A.nBucket) {
+                    const int b = m > 32 ? 0 : 1;
+                    qa[nxt][b][atomicAdd(&qn[nxt][b], 1)] = (short)(c + q);
+                }
+            }
+        };
+        for (int cur = 0; qn[cur][0] + qn[cur][1] > 0;) {
+            const int nxt = cur == 2 ? 0 : cur + 1, nn2 = nxt == 2 ? 0 : nxt + 1;
+            const int nbig = qn[cur][0], nsml = qn[cur][1];
+            if (tid == 0) qn[nn2][0] = qn[nn2][1] = 0;   // the queue after the next
+            for (int b = w; b < nbig; b += SUB_T / 64) {
+                const int k = qa[cur][0][b];
+                const int lo = nlo[k], hi = nhi[k];
+                double bmin[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
+                double bmax[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+                for (int i = lo + lane; i <= hi; i += 64) {
+                    const double v[3] = {lx[i], ly[i], lz[i]};
+                    for (int d = 0; d < 3; ++d) {
+                        bmin[d] = v[d] < bmin[d] ? v[d] : bmin[d];
+                        bmax[d] = v[d] > bmax[d] ? v[d] : bmax[d];
+                    }
+                }
+                for (int o = 32; o > 0; o >>= 1)
+                    for (int d = 0; d < 3; ++d) {
+                        const double l = __shfl_xor(bmin[d], o), h = __shfl_xor(bmax[d], o);
+                        bmin[d] = l < bmin[d] ? l : bmin[d];
+                        bmax[d] = h > bmax[d] ? h : bmax[d];
+                    }
+                int dim = 0;
+                for (int q = 1; q < 3; ++q)
+                    if (bmax[q] - bmin[q] > bmax[dim] - bmin[dim]) dim = q;
+                if (!(bmax[0] > bmin[0]) && !(bmax[1] > bmin[1]) && !(bmax[2] > bmin[2])) continue;
+                const double split = 0.5 * (bmin[dim] + bmax[dim]);
+                const double *cc = dim == 0 ? lx : (dim == 1 ? ly : lz);
+                int nl = 0;
+                for (int c0 = lo; c0 <= hi; c0 += 64) {
+                    const int i = c0 + lane;
+                    nl += __popcll(__ballot(i <= hi && cc[i] < split));
+                }
+                const int s = lo + nl;
+                if (s == lo || s > hi) {   // one side empty: reported, left a bucket
+                    if (lane == 0) atomicOr(&A.L->err, 1);
+                    continue;
+                }
+                int run = 0;
+                for (int c0 = lo; c0 <= hi; c0 += 64) {   // upper positions holding a lower one
+                    const int i = c0 + lane;
+                    const bool f = i <= hi && cc[i] < split;
+                    const unsigned long long m = __ballot(f);
+                    const int ex = run + __popcll(m & ((1ull << lane) - 1));
+                    if (f && i >= s) posR[lo + (nl - 1 - ex)] = (short)i;
+                    run += __popcll(m);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                run = 0;
+                for (int c0 = lo; c0 < s; c0 += 64) {     // lower positions holding an upper one
+                    const int i = c0 + lane;
+                    const bool in = i < s, f = in && cc[i] < split;
+                    const unsigned long long m = __ballot(f);
+                    const int ex = run + __popcll(m & ((1ull << lane) - 1));
+                    if (in && !f) {
+                        const int j = posR[lo + (i - lo) - ex];
+                        double d = lx[i]; lx[i] = lx[j]; lx[j] = d;
+                        d = ly[i]; ly[i] = ly[j]; ly[j] = d;
+                        d = lz[i]; lz[i] = lz[j]; lz[j] = d;
+                        const int u = ls[i]; ls[i] = ls[j]; ls[j] = u;
+                    }
+                    run += __popcll(m);
+                }
+                if (lane == 0) children(k, lo, hi, s, dim, split, nxt);
+            }
+            for (int b = 2 * w; b < nsml; b += SUB_T / 32) {   // at most 32 particles: half a
+                const bool have = b + half < nsml;             // wavefront each
+                const int k = have ? qa[cur][1][b + half] : 0;
+                const int lo = have ? nlo[k] : 0, hi = have ? nhi[k] : -1;
+                const int i = lo + l32;
+                const bool in = i <= hi;
+                double bmin[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
+                double bmax[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+                if (in) {
+                    const double v[3] = {lx[i], ly[i], lz[i]};
+                    for (int d = 0; d < 3; ++d) {       // comparisons, as in the larger cells
+                        bmin[d] = v[d] < bmin[d] ? v[d] : bmin[d];
+                        bmax[d] = v[d] > bmax[d] ? v[d] : bmax[d];
+                    }
+                }
+                for (int o = 16; o > 0; o >>= 1)
+                    for (int d = 0; d < 3; ++d) {
+                        const double l = __shfl_xor(bmin[d], o), h = __shfl_xor(bmax[d], o);
+                        bmin[d] = l < bmin[d] ? l : bmin[d];
+                        bmax[d] = h > bmax[d] ? h : bmax[d];
+                    }
+                int dim = 0;
+                for (int q = 1; q < 3; ++q)
+                    if (bmax[q] - bmin[q] > bmax[dim] - bmin[dim]) dim = q;
+                const bool ext = have && (bmax[0] > bmin[0] || bmax[1] > bmin[1] ||
+                                          bmax[2] > bmin[2]);
+                const double split = 0.5 * (bmin[dim] + bmax[dim]);
+                const double *cc = dim == 0 ? lx : (dim == 1 ? ly : lz);
+                const bool f = ext && in && cc[i] < split;
+                const unsigned long long mm = __ballot(f);
+                const uint32_t m = (uint32_t)(mm >> (32 * half));
+                const int nl = __popc(m), s = lo + nl, ex = __popc(m & ((1u << l32) - 1));
+                const bool ok = ext && s > lo && s <= hi;
+                if (ext && !ok && l32 == 0) atomicOr(&A.L->err, 1);
+                if (ok && f && i >= s) posR[lo + (nl - 1 - ex)] = (short)i;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if (ok && i < s && !f) {
+                    const int j = posR[i - ex];
+                    double d = lx[i]; lx[i] = lx[j]; lx[j] = d;
+                    d = ly[i]; ly[i] = ly[j]; ly[j] = d;
+                    d = lz[i]; lz[i] = lz[j]; lz[j] = d;
+                    const int u = ls[i]; ls[i] = ls[j]; ls[j] = u;
+                }
+                if (ok && l32 == 0) children(k, lo, hi, s, dim, split, nxt);
+            }
+            cur = nxt;
+            __syncthreads();
+        }
+        // storage-order particles; the cells' slots
+        const int nloc = nloc_sh;
+        if (tid == 0) slot_sh = nloc > 1 ? atomicAdd(&A.L->nloc, nloc - 1) : 0;
+        for (int i = tid; i < cnt; i += SUB_T) {
+            const int s = ls[i];
+            const double mm = A.m[s], hh = A.h[s];
+            const uint32_t bt = A.bits[s];
+            lm[i] = mm;
+            lh[i] = hh;
+            lact[i] = bt & 1u;
+            A.px[glo + i] = lx[i];
+            A.py[glo + i] = ly[i];
+            A.pz[glo + i] = lz[i];
+            A.perm[glo + i] = s;
+            A.pm[glo + i] = mm;
+            A.ph[glo + i] = hh;
+            A.pact[glo + i] = bt;
+        }
+        for (int k = tid; k < nloc; k += SUB_T) arr[k] = 0;
+        __syncthreads();
+        const int used = slot_sh + nloc - 1;             // from the last slot down
+        const bool room = A.L->next + used <= A.cap;
+        if (!room && tid == 0) atomicOr(&A.L->err, 2);
+        // sizes and active buckets, climbing from the buckets
+        for (int k = tid; k < nloc; k += SUB_T) {
+            if (nch[k] >= 0) continue;
+            int na = 0;
+            for (int i = nlo[k]; i <= nhi[k]; ++i) na |= lact[i];
+            atomicMax(&maxb_sh, nhi[k] - nlo[k] + 1);
+            nsz[k] = 1;
+            nac[k] = (short)na;
+            for (int c = npar[k]; c >= 0; c = npar[c]) {
+                if (__hip_atomic_fetch_add(&arr[c], 1, __ATOMIC_ACQ_REL,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+                    break;
+                const int c0 = nch[c];
+                nsz[c] = (short)(1 + nsz[c0] + nsz[c0 + 1]);
+                nac[c] = (short)(nac[c0] + nac[c0 + 1]);
+            }
+        }
+        __syncthreads();
+        for (int k = tid; k < nloc; k += SUB_T) {        // preorder ids and bucket ranks
+            int p = 0, bp = 0;
+            for (int c = k; npar[c] >= 0; c = npar[c]) {
+                const int c0 = nch[npar[c]];
+                ++p;
+                if (c != c0) {
+                    p += nsz[c0];
+                    bp += nac[c0];
+                }
+            }
+            npre[k] = (short)p;
+            nbp[k] = (short)bp;
+            arr[k] = 0;
+        }
+        __syncthreads();
+        if (room) {
+            const int s1 = A.cap - used;                 // slot of preorder id 1
+            auto slot = [&](int k) { return k == 0 ? root : s1 + npre[k] - 1; };
+            auto get = [&](int i, double *p, double &mm, double &hh) {
+                p[0] = lx[i];
+                p[1] = ly[i];
+                p[2] = lz[i];
+                mm = lm[i];
+                hh = lh[i];
+                return lact[i] != 0;
+            };
+            for (int k = tid; k < nloc; k += SUB_T) {    // records, climbing likewise
+                if (nch[k] >= 0) continue;
+                double g[GS];
+                for (int q = 0; q < GS; ++q) g[q] = 0.0;
+                const int sk = slot(k);
+                bucket_record<ORDER>(nlo[k], nhi[k], get, g, A.bb8 + 8 * (size_t)sk);
+                double *o = A.gm + (size_t)GS * sk;
+                for (int q = 0; q < GS; ++q) o[q] = g[q];
+                for (int c = npar[k]; c >= 0; c = npar[c]) {
+                    if (__hip_atomic_fetch_add(&arr[c], 1, __ATOMIC_ACQ_REL,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+                        break;
+                    const double *c0 = A.gm + (size_t)GS * slot(nch[c]);
+                    const double *c1 = A.gm + (size_t)GS * slot(nch[c] + 1);
+                    for (int q = 0; q < GS; ++q) g[q] = 0.0;
+                    mass_children(c0, c1, g);
+                    for (int q = 0; q < 2; ++q) {
+                        const double *cq = q ? c1 : c0;
+                        const double d[3] = {cq[2] - g[2], cq[3] - g[3], cq[4] - g[4]};
+                        mom_shift<ORDER>(cq, d, g);
+                    }
+                    o = A.gm + (size_t)GS * slot(c);
+                    for (int q = 0; q < GS; ++q) o[q] = g[q];
+                }
+            }
+            __syncthreads();
+            for (int k = tid >> 4; k < nloc; k += SUB_T / 16) {   // Bmax, 16 lanes per cell
+                if (nch[k] < 0) continue;                // buckets have theirs
+                double *o = A.gm + (size_t)GS * slot(k);
+                const double cm[3] = {o[2], o[3], o[4]};
+                double b2 = 0.0;
+                for (int i = nlo[k] + (tid & 15); i <= nhi[k]; i += 16) {
+                    const double d2 = cm_d2(lx[i], ly[i], lz[i], cm);
+                    b2 = d2 > b2 ? d2 : b2;
+                }
+                for (int q = 8; q > 0; q >>= 1) {
+                    const double u = __shfl_xor(b2, q);
+                    b2 = u > b2 ? u : b2;
+                }
+                if ((tid & 15) == 0) o[GM_B] = b2;
+            }
+            for (int k = tid; k < nloc; k += SUB_T) {
+                GNode &g = A.nd[slot(k)];
+                const int c = nch[k];
+                if (k > 0) {
+                    g.lo = glo + nlo[k];
+                    g.hi = glo + nhi[k];
+                    g.root = troot;
+                    g.pre = npre[k];
+                    g.bpre = nbp[k];
+                }
+                g.dim = ndm[k];
+                g.split = nsp[k];
+                g.size = nsz[k];
+                g.nab = nac[k];
+                g.ch0 = c < 0 ? -1 : slot(c);
+                g.ch1 = c < 0 ? -1 : slot(c + 1);
+            }
+            if (tid == 0) {
+                A.subn[t] = make_int2(s1, nloc - 1);
+                atomicMax(&A.L->maxb, maxb_sh);
+            }
+        }
+        __syncthreads();
     }
 }
 
-// Cells of at most MOM_SMALL particles (most cells: the buckets and the
-// levels just above them): one thread each sums its cell's particles in
-// order, with no cross-lane reduction.  Each such cell is one item.
-template <int ORDER>
-__global__ __launch_bounds__(256) void k_gt_moments_small(int nitem, const int *__restrict__ icell,
-                                                          const GNode *__restrict__ nd,
-                                                          const double *__restrict__ cm,
-                                                          const double *__restrict__ x,
-                                                          const double *__restrict__ y,
-                                                          const double *__restrict__ z,
-                                                          const double *__restrict__ pm,
-                                                          double *__restrict__ part)
+// A closed cell above LMAX, by a pair of lanes (q 0, 1): its record and its
+// subtree's counts from its children's, or, of a bucket of coincident
+// particles, from its particles (by lane 0).
+template <int ORDER> __device__ __forceinline__ void upper_record(const TreeArgs &A, int c, int q)
 {
 #pragma clang fp contract(off)
-    const int it = blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= nitem) return;
-    const int c = icell[it];
-    const GNode &g = nd[c];
-    if (g.hi - g.lo + 1 > MOM_SMALL) return;
-    const double cx = cm[5 * (size_t)c + 2], cy = cm[5 * (size_t)c + 3], cz = cm[5 * (size_t)c + 4];
-    double Q[6] = {0, 0, 0, 0, 0, 0}, O[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double H[15] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double Bmax = 0.0;
-    for (int i = g.lo; i <= g.hi; ++i) {
-        const double mm = pm[i];
-        const double dx = x[i] - cx, dy = y[i] - cy, dz = z[i] - cz;
-        mom_accum<ORDER>(mm, dx, dy, dz, Q, O, H, Bmax);
+    constexpr int GS = gm_stride(ORDER);
+    GNode &g = A.nd[c];
+    double *o = A.gm + (size_t)GS * c;
+    double v[GS];
+    for (int k = 0; k < GS; ++k) v[k] = 0.0;
+    const bool leaf = g.dim < 0;
+    if (leaf) {
+        if (q) return;
+        const int na = bucket_record<ORDER>(
+            g.lo, g.hi,
+            [&](int i, double *p, double &m, double &h) {
+                const int s = A.perm[i];
+                p[0] = A.px[i];
+                p[1] = A.py[i];
+                p[2] = A.pz[i];
+                A.pm[i] = m = A.m[s];
+                A.ph[i] = h = A.h[s];
+                A.pact[i] = A.bits[s];
+                return (A.pact[i] & 1u) != 0;
+            },
+            v, A.bb8 + 8 * (size_t)c);
+        for (int k = 0; k < GS; ++k) o[k] = v[k];
+        g.size = 1;
+        g.nab = na > 0;
+        atomicMax(&A.L->maxb, g.hi - g.lo + 1);
+        return;
     }
-    double *p = part + (size_t)NM * it;
-    for (int k = 0; k < 6; ++k) p[k] = Q[k];
-    for (int k = 0; k < 10; ++k) p[6 + k] = O[k];
-    for (int k = 0; k < 15; ++k) p[16 + k] = H[k];
-    p[31] = Bmax;
+    const int i0 = g.ch0, i1 = g.ch1;
+    const double *c0 = A.gm + (size_t)GS * i0, *c1 = A.gm + (size_t)GS * i1;
+    mass_children(c0, c1, v);
+    const double *cq = q ? c1 : c0;
+    const double d[3] = {cq[2] - v[2], cq[3] - v[3], cq[4] - v[4]};
+    mom_shift<ORDER>(cq, d, v);
+    for (int k = GM_Q; k < GS; ++k) v[k] += __shfl_xor(v[k], 1);
+    if (q) return;
+    v[GM_B] = 0.0;
+    for (int k = 0; k < GS; ++k) o[k] = v[k];
+    const int s0 = A.nd[i0].size, a0 = A.nd[i0].nab;
+    g.sizeLo = s0;
+    g.nabLo = a0;
+    g.size = 1 + s0 + A.nd[i1].size;
+    g.nab = a0 + A.nd[i1].nab;
 }
 
-// Per cell in preorder: the parity record (iDim, pLower, pUpper, iLower,
+// What k_gt_mid closed in one unit, deepest level first (one wavefront).
+template <int ORDER> __global__ __launch_bounds__(64) void k_gt_up_unit(TreeArgs A)
+{
+    const int lane = threadIdx.x;
+    if (A.L->err & 2) return;
+    const int2 u = A.useg[blockIdx.x];
+    if (u.y == 0) return;
+    const int base = A.nd[A.unit[blockIdx.x]].lo;
+    for (int l = u.y - 1; l >= 0; --l) {
+        const int e0 = l ? A.segl[base + l - 1] : 0, e1 = A.segl[base + l];
+        for (int e = e0 + (lane >> 1); e < e1; e += 32) upper_record<ORDER>(A, A.seg[base + e], lane & 1);
+        __syncthreads();
+    }
+}
+
+// The splitting cells of one level above MID.
+template <int ORDER> __global__ __launch_bounds__(256) void k_gt_up_level(TreeArgs A, int depth)
+{
+    if (A.L->err & 2) return;
+    const int c = A.L->lv[depth] + ((blockIdx.x * 256 + threadIdx.x) >> 1);
+    if (c >= A.L->lv[depth + 1]) return;
+    const GNode &g = A.nd[c];
+    if (g.hi - g.lo < MID || g.dim < 0) return;          // a unit
+    upper_record<ORDER>(A, c, threadIdx.x & 1);
+}
+
+// One workgroup: the roots' preorder ids and first bucket ranks, and to the
+// host the cells, active buckets, largest bucket and error word.
+__global__ __launch_bounds__(256) void k_gt_totals(int nr, TreeArgs A, int *host)
+{
+    __shared__ int2 ws[4];
+    int2 run = make_int2(0, 0);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int b = 0; b < nr; b += 256) {
+        const int k = b + threadIdx.x;
+        const int sz = k < nr ? A.nd[k].size : 0, na = k < nr ? A.nd[k].nab : 0;
+        int is = sz, ia = na;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int us = __shfl_up(is, o), ua = __shfl_up(ia, o);
+            if (lane >= o) {
+                is += us;
+                ia += ua;
+            }
+        }
+        if (lane == 63) ws[w] = make_int2(is, ia);
+        __syncthreads();
+        int ps = run.x + is - sz, pa = run.y + ia - na;
+        for (int q = 0; q < 4; ++q) {
+            if (q < w) {
+                ps += ws[q].x;
+                pa += ws[q].y;
+            }
+            run.x += ws[q].x;
+            run.y += ws[q].y;
+        }
+        if (k < nr) {
+            A.nd[k].pre = ps;
+            A.nd[k].bpre = pa;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        tell_host(host + 1, run.x);
+        tell_host(host + 2, run.y);
+        tell_host(host + 3, A.L->maxb);
+        tell_host(host + 4, A.L->next);
+        tell_host(host + 5, A.L->nsub);
+        tell_host(host, A.L->err);
+    }
+}
+
+// Largest squared distances of the cells above LMAX: per unit, the cells
+// k_gt_mid closed (a wavefront each), then the unit's particles against
+// every cell above it, combined in LDS and then by one atomic a cell.
+constexpr int BM_A = 512;        // ancestors combined at a time
+template <int ORDER> __global__ __launch_bounds__(256) void k_gt_up_bmax(TreeArgs A)
+{
+    constexpr int GS = gm_stride(ORDER);
+    __shared__ unsigned long long bm[BM_A];
+    __shared__ int an[BM_A];
+    __shared__ int na_sh, next_sh;
+    if (A.L->err & 2) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int root = A.unit[blockIdx.x];
+    const int lo = A.nd[root].lo, hi = A.nd[root].hi;
+    const int2 u = A.useg[blockIdx.x];
+    for (int e = w; e < u.x; e += 4) {
+        const int c = A.seg[lo + e];
+        const int c0 = A.nd[c].lo, c1 = A.nd[c].hi;
+        double *o = A.gm + (size_t)GS * c;
+        if (A.nd[c].dim < 0) continue;
+        const double cm[3] = {o[2], o[3], o[4]};
+        double b2 = 0.0;
+        for (int i = c0 + lane; i <= c1; i += 64) {
+            const double d2 = cm_d2(A.px[i], A.py[i], A.pz[i], cm);
+            b2 = d2 > b2 ? d2 : b2;
+        }
+        for (int q = 32; q > 0; q >>= 1) {
+            const double v = __shfl_xor(b2, q);
+            b2 = v > b2 ? v : b2;
+        }
+        if (lane == 0) o[GM_B] = b2;
+    }
+    for (int c = A.nd[root].par; c >= 0; c = next_sh) {
+        if (tid == 0) {
+            int k = 0;
+            for (; c >= 0 && k < BM_A; c = A.nd[c].par) an[k++] = c;
+            na_sh = k;
+            next_sh = c;
+        }
+        for (int k = tid; k < BM_A; k += 256) bm[k] = 0;
+        __syncthreads();
+        const int na = na_sh;
+        for (int b = lo; b <= hi; b += 1024) {
+            double x[4], y[4], z[4];
+            for (int q = 0; q < 4; ++q) {                // past the end: the last particle
+                const int i = min(b + 256 * q + tid, hi);
+                x[q] = A.px[i];
+                y[q] = A.py[i];
+                z[q] = A.pz[i];
+            }
+            for (int k = 0; k < na; ++k) {
+                const double *o = A.gm + (size_t)GS * an[k];
+                const double cm[3] = {o[2], o[3], o[4]};
+                double b2 = 0.0;
+                for (int q = 0; q < 4; ++q) {
+                    const double d2 = cm_d2(x[q], y[q], z[q], cm);
+                    b2 = d2 > b2 ? d2 : b2;
+                }
+                for (int q = 32; q > 0; q >>= 1) {
+                    const double v = __shfl_xor(b2, q);
+                    b2 = v > b2 ? v : b2;
+                }
+                if (lane == 0) atomicMax(&bm[k], (unsigned long long)__double_as_longlong(b2));
+            }
+        }
+        __syncthreads();
+        for (int k = tid; k < na; k += 256)
+            atomicMax(reinterpret_cast<unsigned long long *>(A.gm + (size_t)GS * an[k] + GM_B),
+                      bm[k]);
+        __syncthreads();
+    }
+}
+
+// What the walk and the parity tools read, in preorder.
+struct EmitArgs {
+    int iOpenType;
+    double dCrit;
+    int *tint;
+    double *tdbl;
+    WalkNode *wn;
+    double *cell, *momOH;
+    int *bucket, *broot;
+    double *bbox;
+};
+
+// Preorder id and first bucket rank of a cell above LMAX or of a subtree of
+// k_gt_sub, up the parents.
+__device__ __forceinline__ int2 climb(const GNode *__restrict__ nd, int c)
+{
+    int p = 0, b = 0;
+    for (int up = nd[c].par; up >= 0;) {
+        const GNode &g = nd[up];
+        ++p;
+        if (g.ch1 == c) {
+            p += g.sizeLo;
+            b += g.nabLo;
+        }
+        c = up;
+        up = g.par;
+    }
+    return make_int2(p + nd[c].pre, b + nd[c].bpre);
+}
+
+// Per cell at preorder id c: the parity record (iDim, pLower, pUpper, iLower,
 // iNext, 0; mass, softening, c.o.m., fOpen2, Bmax, fSplit), the walk record,
-// the cell record and O/H: moments summed over the cell's items in order,
-// traceless Q as the walk stores it (walk.c:41-48), fOpen2 by pkdCalcOpen
-// (pkd.c:2228-2264).
-// Cells of more than one moment item (one wavefront per cell): lane j sums
-// the items j, j + 64, ..., a fixed butterfly combines the lanes, and the
-// total replaces the cell's first item.
-__global__ __launch_bounds__(256) void k_gt_combine(int nn, int nv,
-                                                    const int64_t *__restrict__ ioff,
-                                                    double *__restrict__ part)
-{
-    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (b >= nn) return;
-    const int64_t i0 = ioff[b], i1 = ioff[b + 1];
-    if (i1 - i0 < 2) return;
-    double M[31];
-    for (int k = 0; k < 31; ++k) M[k] = 0.0;
-    double Bmax = 0.0;
-    for (int64_t it = i0 + lane; it < i1; it += 64) {
-        const double *p = part + (size_t)NM * it;
-        for (int k = 0; k < nv; ++k) M[k] += p[k];
-        Bmax = fmax(Bmax, p[31]);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        for (int k = 0; k < nv; ++k) M[k] += __shfl_xor(M[k], o);
-        Bmax = fmax(Bmax, __shfl_xor(Bmax, o));
-    }
-    if (lane) return;
-    double *p = part + (size_t)NM * i0;
-    for (int k = 0; k < nv; ++k) p[k] = M[k];
-    p[31] = Bmax;
-}
-
-__global__ void k_gt_emit(int nn, int iOrder, int iOpenType, double dCrit,
-                          const GNode *__restrict__ nd, const double *__restrict__ cm,
-                          const int64_t *__restrict__ ioff, const double *__restrict__ part,
-                          int *__restrict__ tint, double *__restrict__ tdbl,
-                          WalkNode *__restrict__ wn, double *__restrict__ cell,
-                          double *__restrict__ momOH)
+// the cell record (traceless Q as the walk stores it, walk.c:41-48) and the
+// reduced O/H; fOpen2 by pkdCalcOpen (pkd.c:2228-2264).  Of a bucket with
+// active particles also its entry of the bucket list (rank bk).
+template <int ORDER>
+__device__ __forceinline__ void emit_cell(const TreeArgs &A, const EmitArgs &E, int slot, int c,
+                                          int bk)
 {
 #pragma clang fp contract(off)
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nn) return;
-    const GNode &g = nd[b];
-    const int c = g.pre;
-    const double *q = cm + 5 * (size_t)b;
-    const double *M = part + (size_t)NM * ioff[b];
-    const double Bmax = M[31];
+    constexpr int GS = gm_stride(ORDER);
+    const GNode &g = A.nd[slot];
+    const double *M = A.gm + (size_t)GS * slot;
+    const double Bmax = sqrt(M[GM_B]);
     double dOpen;
-    if (iOpenType == 1) {
-        dOpen = 2 / sqrt(3.0) * Bmax / dCrit;
+    if (E.iOpenType == 1) {
+        dOpen = 2 / sqrt(3.0) * Bmax / E.dCrit;
         if (dOpen < Bmax) dOpen = Bmax;
     } else {
         dOpen = Bmax;
     }
-    const double fOpen2 = g.hi >= g.lo ? dOpen * dOpen : 0.0;
-    const GNode &rt = nd[g.root];
-    const int end = rt.pre + rt.size;
-    const int first = g.ch0 >= 0 ? nd[g.ch0].pre : -1;
-    const int second = g.ch1 >= 0 ? nd[g.ch1].pre : -1;
-    const int next = c + g.size < end ? c + g.size : -1;
-    int *ti = tint + 6 * (size_t)c;   // iLower: the first child is c + 1 in preorder
+    const double fOpen2 = dOpen * dOpen;
+    const GNode &rt = A.nd[g.root];
+    const int next = c + g.size < rt.pre + rt.size ? c + g.size : -1;
+    const int second = g.ch1 >= 0 ? c + 1 + A.nd[g.ch0].size : -1;
+    int *ti = E.tint + 6 * (size_t)c;   // iLower: the first child is c + 1 in preorder
     ti[0] = g.dim;
     ti[1] = g.lo;
     ti[2] = g.hi;
     ti[3] = g.dim >= 0 ? c + 1 : -1;
     ti[4] = next;
     ti[5] = 0;
-    double *td = tdbl + 8 * (size_t)c;
-    for (int k = 0; k < 5; ++k) td[k] = q[k];
+    double *td = E.tdbl + 8 * (size_t)c;
+    for (int k = 0; k < 5; ++k) td[k] = M[k];
     td[5] = fOpen2;
     td[6] = Bmax;
     td[7] = g.split;
     WalkNode w;
-    w.cx = q[2];
-    w.cy = q[3];
-    w.cz = q[4];
+    w.cx = M[2];
+    w.cy = M[3];
+    w.cz = M[4];
     w.fOpen2 = fOpen2;
-    w.fSoft = q[1];
+    w.fSoft = M[1];
     w.pLower = g.lo;
     w.pUpper = g.hi;
-    w.iLower = first;
+    w.iLower = g.dim >= 0 ? c + 1 : -1;
     w.iNext = next;
     w.iUpper = second;
     w.pad1 = 0;
-    wn[c] = w;
-    double *r = cell + (size_t)CR_N * c;
-    r[CR_M] = q[0];
-    for (int d = 0; d < 3; ++d) r[CR_X + d] = q[2 + d];
-    r[CR_H] = q[1];
-    for (int k = 0; k < 6; ++k) r[CR_QR + k] = M[k];
-    const double tr = M[0] + M[1] + M[2];
-    r[CR_QT] = M[0] - tr / 3.0;
-    r[CR_QT + 1] = M[1] - tr / 3.0;
-    r[CR_QT + 2] = M[2] - tr / 3.0;
-    r[CR_QT + 3] = M[3];
-    r[CR_QT + 4] = M[4];
-    r[CR_QT + 5] = M[5];
-    if (iOrder >= 3)
-        for (int k = 0; k < 25; ++k) momOH[(size_t)OH_N * c + k] = M[6 + k];
-}
-
-// Buckets with an active particle: flag by preorder id; bounds of the
-// active particles, largest softening, active count (pkd.c:2916-2937,
-// walk.c:319-324); the largest bucket, active or not (the fused walk maps a
-// bucket's targets, and an opened bucket's particles, onto one wavefront).
-__global__ void k_gt_bucket(int nn, const GNode *__restrict__ nd, const double *__restrict__ x,
-                            const double *__restrict__ y, const double *__restrict__ z,
-                            const double *__restrict__ ph, const uint32_t *__restrict__ pact,
-                            int *__restrict__ flag, double *__restrict__ bb8,
-                            int *__restrict__ maxb)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nn) return;
-    const GNode &g = nd[b];
-    const int c = g.pre;
-    if (g.dim >= 0 || g.lo > g.hi) {
-        flag[c] = 0;
-        return;
-    }
-    double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    int na = 0;
-    double fsm = 0.0;
-    for (int i = g.lo; i <= g.hi; ++i) {
-        if (ph[i] > fsm) fsm = ph[i];
-        if (!(pact[i] & 1u)) continue;
-        ++na;
-        const double r[3] = {x[i], y[i], z[i]};
-        for (int d = 0; d < 3; ++d) {
-            if (r[d] < lo[d]) lo[d] = r[d];
-            if (r[d] > hi[d]) hi[d] = r[d];
+    E.wn[c] = w;
+    double *r = E.cell + (size_t)CR_N * c;
+    r[CR_M] = M[0];
+    for (int d = 0; d < 3; ++d) r[CR_X + d] = M[2 + d];
+    r[CR_H] = M[1];
+    const double *Q = M + GM_Q;
+    for (int k = 0; k < 6; ++k) r[CR_QR + k] = Q[k];
+    const double tr = Q[0] + Q[1] + Q[2];
+    for (int k = 0; k < 3; ++k) r[CR_QT + k] = Q[k] - tr / 3.0;
+    for (int k = 3; k < 6; ++k) r[CR_QT + k] = Q[k];
+    if constexpr (ORDER >= 3) {
+        double *o = E.momOH + (size_t)OH_N * c;
+        const double *T = M + GM_T;
+        const double tx = T[0] + T[1] + T[7], ty = T[2] + T[3] + T[8], tz = T[4] + T[5] + T[9];
+        o[0] = T[0] - 0.6 * tx;
+        o[1] = T[1] - 0.2 * tx;
+        o[2] = T[2] - 0.2 * ty;
+        o[3] = T[3] - 0.6 * ty;
+        o[4] = T[4] - 0.2 * tz;
+        o[5] = T[5] - 0.2 * tz;
+        o[6] = T[6];
+        o[7] = T[7] - 0.2 * tx;
+        o[8] = T[8] - 0.2 * ty;
+        o[9] = T[9] - 0.6 * tz;
+        if constexpr (ORDER >= 4) {
+            const double *F = M + GM_F;
+            const double sxx = F[0] + F[6] + F[9], syy = F[6] + F[3] + F[12];
+            const double szz = F[9] + F[12] + F[14], sxy = F[2] + F[1] + F[10];
+            const double sxz = F[4] + F[8] + F[11], syz = F[7] + F[5] + F[13];
+            const double s4 = sxx + syy + szz;
+            o[10] = F[0] - 6.0 / 7.0 * (sxx - 0.1 * s4);
+            o[11] = F[1] - 3.0 / 7.0 * sxy;
+            o[12] = F[2] - 3.0 / 7.0 * sxy;
+            o[13] = F[3] - 6.0 / 7.0 * (syy - 0.1 * s4);
+            o[14] = F[4] - 3.0 / 7.0 * sxz;
+            o[15] = F[5] - 3.0 / 7.0 * syz;
+            o[16] = F[6] - 1.0 / 7.0 * (sxx + syy - 0.2 * s4);
+            o[17] = F[7] - 1.0 / 7.0 * syz;
+            o[18] = F[8] - 1.0 / 7.0 * sxz;
+            o[19] = F[9] - 1.0 / 7.0 * (sxx + szz - 0.2 * s4);
+            o[20] = F[10] - 1.0 / 7.0 * sxy;
+            o[21] = F[11] - 3.0 / 7.0 * sxz;
+            o[22] = F[12] - 1.0 / 7.0 * (syy + szz - 0.2 * s4);
+            o[23] = F[13] - 3.0 / 7.0 * syz;
+            o[24] = F[14] - 6.0 / 7.0 * (szz - 0.1 * s4);
         }
     }
-    flag[c] = na > 0;
-    atomicMax(maxb, g.hi - g.lo + 1);
-    double *o = bb8 + 8 * (size_t)c;
-    for (int d = 0; d < 3; ++d) {
-        o[d] = lo[d];
-        o[3 + d] = hi[d];
+    if (g.dim < 0 && g.nab) {
+        E.bucket[bk] = c;
+        E.broot[bk] = rt.pre;
+        for (int d = 0; d < 8; ++d) E.bbox[8 * (size_t)bk + d] = A.bb8[8 * (size_t)slot + d];
     }
-    o[6] = fsm;
-    o[7] = (double)na;
 }
 
-__global__ void k_gt_bucket_list(int nn, const int *__restrict__ flag,
-                                 const int64_t *__restrict__ pos, const double *__restrict__ bb8,
-                                 const int *__restrict__ rootOf, int *__restrict__ bucket,
-                                 double *__restrict__ bbox, int *__restrict__ broot)
+// Blocks below nub: a thread per slot above LMAX.  The others: a wavefront
+// per subtree of k_gt_sub, its cells in preorder (consecutive slots and ids).
+template <int ORDER>
+__global__ __launch_bounds__(256) void k_gt_emit(int nub, int nup, int nsub, TreeArgs A, EmitArgs E)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nn || !flag[c]) return;
-    const int k = (int)pos[c];
-    bucket[k] = c;
-    for (int d = 0; d < 8; ++d) bbox[8 * (size_t)k + d] = bb8[8 * (size_t)c + d];
-    broot[k] = rootOf[c];
-}
-
-__global__ void k_gt_rootof(int nn, const GNode *__restrict__ nd, int *__restrict__ rootOf)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nn) return;
-    rootOf[nd[b].pre] = nd[nd[b].root].pre;
+    if ((int)blockIdx.x < nub) {
+        const int c = blockIdx.x * 256 + threadIdx.x;
+        if (c >= nup) return;
+        const GNode &g = A.nd[c];
+        if (g.hi - g.lo < LMAX) return;                  // with its subtree
+        const int2 p = climb(A.nd, c);
+        emit_cell<ORDER>(A, E, c, p.x, p.y);
+        return;
+    }
+    const int t = (blockIdx.x - nub) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= nsub) return;
+    const int root = A.sub[t];
+    const int2 s = A.subn[t], p = climb(A.nd, root);
+    for (int k = lane; k <= s.y; k += 64) {
+        const int slot = k ? s.x + k - 1 : root;
+        emit_cell<ORDER>(A, E, slot, p.x + k, p.y + (k ? A.nd[slot].bpre : 0));
+    }
 }
 
 }  // namespace
@@ -1487,13 +1707,13 @@ static int gt_partition(GravDev &G, hipStream_t st, const TileArgs &A, int grid,
     return GG_OK;
 }
 
-int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenType, double dCrit,
-                int iOrder)
+// One build with slots for cap cells; *room tells whether they were enough.
+static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenType,
+                     double dCrit, int iOrder, int cap, bool *room)
 {
     GravDev &G = pkd->grav;
     hipStream_t st = pkd->stream;
     const int n = pkd->nLocal;
-    G.built = 0;
     // roots: the non-empty systems
     std::vector<int> rlo;
     int maxRoot = 0;
@@ -1504,11 +1724,11 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
         }
     const int nr = (int)rlo.size();
     for (int k = 0; k < nr; ++k) rlo.push_back(k + 1 < nr ? rlo[k + 1] - 1 : n - 1);
-    const size_t n1 = (size_t)std::max(n, 1);
-    const size_t cap = 2 * n1 + 2;   // cells at most: every split has two children
+    const size_t n1 = (size_t)n;
     const int ts = tile_size(n);
-    const size_t mtile = n1 / ts + n1 / MID + std::max(nr, 1) + 1;   // tiles of a level, at most
+    const size_t mtile = n1 / ts + n1 / MID + nr + 1;                // tiles of a level, at most
     const size_t mbox = std::max<size_t>(2 * (n1 / MID) + 2, nr);    // its cells
+    const int order = iOrder >= 4 ? 4 : (iOrder == 3 ? 3 : 2);
     GG_TRY(G.px.reserve(sizeof(double) * n1));
     GG_TRY(G.py.reserve(sizeof(double) * n1));
     GG_TRY(G.pz.reserve(sizeof(double) * n1));
@@ -1518,286 +1738,212 @@ int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenTy
     GG_TRY(G.perm.reserve(sizeof(int) * n1));
     GG_TRY(G.acc.reserve(sizeof(double) * 5 * n1));
     GG_TRY(G.gposR.reserve(sizeof(int) * n1));
-    GG_TRY(G.gnode.reserve(sizeof(GNode) * cap));
+    GG_TRY(G.gnode.reserve(sizeof(GNode) * (size_t)cap));
+    GG_TRY(G.gm.reserve(sizeof(double) * gm_stride(order) * (size_t)cap));
+    GG_TRY(G.gbb8.reserve(sizeof(double) * 8 * (size_t)cap));
     GG_TRY(G.gbox.reserve(sizeof(unsigned long long) * 12 * mbox));
     GG_TRY(G.gtile.reserve(sizeof(int4) * mtile));
     GG_TRY(G.gflag.reserve(sizeof(unsigned long long) * mtile * (ts / 64)));
     GG_TRY(G.gtcnt.reserve(sizeof(int) * 2 * mtile));
-    GG_TRY(G.gunit.reserve(sizeof(int) * cap));
+    GG_TRY(G.gunit.reserve((sizeof(int) + sizeof(int2)) * (size_t)n));
+    GG_TRY(G.gsub.reserve((sizeof(int) + sizeof(int2)) * (size_t)n));
+    GG_TRY(G.gseg.reserve(sizeof(int) * 2 * n1));
     GG_TRY(G.glev.reserve(sizeof(GLevel)));
-    GG_TRY(G.gnit.reserve(sizeof(int) * cap));
-    GG_TRY(G.gioff.reserve(sizeof(int64_t) * (cap + 1)));
-    GG_TRY(G.gchoff.reserve(sizeof(int64_t) * (cap + 1)));
-    GG_TRY(G.groot.reserve(sizeof(int) * 2 * std::max(nr, 1)));
+    GG_TRY(G.groot.reserve(sizeof(int) * 2 * nr));
     if (!G.hst)
         GG_HIP(hipHostMalloc((void **)&G.hst, sizeof(int) * GravDev::NHST, hipHostMallocDefault));
     GLevel *L = G.glev.as<GLevel>();
-    GNode *nd = G.gnode.as<GNode>();
-    int nn = 0;
-    std::vector<std::pair<int, int>> depths;
-    if (nr > 0) {
-        const int *rl = G.groot.as<int>(), *rh = rl + nr;
-        unsigned long long *box[2];
-        box[0] = G.gbox.as<unsigned long long>();
-        box[1] = box[0] + 6 * mbox;
-        volatile int *hv = G.hst;
-        for (int k = 0; k < 8; ++k) hv[k] = -1;
+    TreeArgs T;
+    T.nBucket = nBucket;
+    T.cap = cap;
+    T.L = L;
+    T.nd = G.gnode.as<GNode>();
+    T.gm = G.gm.as<double>();
+    T.bb8 = G.gbb8.as<double>();
+    T.px = G.px.as<double>();
+    T.py = G.py.as<double>();
+    T.pz = G.pz.as<double>();
+    T.pm = G.pm.as<double>();
+    T.ph = G.ph.as<double>();
+    T.pact = G.pact.as<uint32_t>();
+    T.perm = G.perm.as<int>();
+    T.m = pkd->f[GG_MASS].as<double>();
+    T.h = pkd->f[GG_SOFT].as<double>();
+    T.bits = pkd->f[GG_IACTIVE].as<uint32_t>();
+    // a unit, or a cell left to k_gt_sub, holds a particle: at most n of each
+    int2 *subn = G.gsub.as<int2>(), *useg = G.gunit.as<int2>();
+    int *sub = reinterpret_cast<int *>(subn + n), *unit = reinterpret_cast<int *>(useg + n);
+    int *seg = G.gseg.as<int>(), *segl = seg + n;
+    T.sub = sub;
+    T.subn = subn;
+    T.unit = unit;
+    T.useg = useg;
+    T.seg = seg;
+    T.segl = segl;
+    const int *rl = G.groot.as<int>(), *rh = rl + nr;
+    unsigned long long *box[2];
+    box[0] = G.gbox.as<unsigned long long>();
+    box[1] = box[0] + 6 * mbox;
+    volatile int *hv = G.hst;
+    for (int k = 0; k < 16; ++k) hv[k] = -1;
+    if (nr > 1)   // (a single root is the whole store)
         GG_HIP(hipMemcpyAsync(G.groot.p, rlo.data(), sizeof(int) * 2 * nr, hipMemcpyHostToDevice,
                               st));
-        hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, nr, rl, rh, nd,
-                           box[0], G.gunit.as<int>(), L);
-        hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, n, nr, rl,
-                           pkd->f[GG_R].as<double>(), pkd->f[GG_IACTIVE].as<uint32_t>(),
-                           G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
-                           G.perm.as<int>(), box[0], L);
-        hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need[1], G.hst + 3);
-        GG_HIP(hipGetLastError());
-        TileArgs A;
-        A.ts = ts;
-        A.mask = 0;
-        A.L = L;
-        A.tiles = G.gtile.as<int4>();
-        A.nd = nd;
-        A.x = G.px.as<double>();
-        A.y = G.py.as<double>();
-        A.z = G.pz.as<double>();
-        A.src = G.perm.as<int>();
-        A.bits = pkd->f[GG_IACTIVE].as<uint32_t>();
-        A.flag = G.gflag.as<unsigned long long>();
-        A.tcnt = G.gtcnt.as<int>();
-        A.tpre = A.tcnt + mtile;
-        A.posR = G.gposR.as<int>();
-        A.err = &L->err;
-        const int grid = (int)mtile;
-        auto ctl = [&](int mode, int depth, int *host) {
-            hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, mode, ts, depth, L, nd,
-                               box[depth & 1], box[(depth & 1) ^ 1], G.gtile.as<int4>(),
-                               G.gunit.as<int>(), host);
-        };
-        // msrBuildTree's active-type orders (master.c:4262).  A particle with
-        // the second order's bit has one of the first's, so where all have it
-        // both orders leave everything in place.
-        int lack = 0;
-        GG_TRY(host_word(st, G.hst + 3, &lack));
-        if (lack) {
-            ctl(1, 0, G.hst + 4);
-            A.mask = GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE;
-            GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
-            A.mask = GG_TYPE_TREEACTIVE;
-            GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
-        }
-        int nunit = nr, nng = nr, nlev = 1;
-        if (maxRoot > MID) {
-            // The levels.  The host learns a level's tile count while its
-            // partition runs, in time to queue the next level behind it.
-            for (int depth = 0;; ++depth) {
-                GG_CHECK(depth < DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
-                int *h = G.hst + 8 + 4 * (depth & 3);
-                for (int k = 0; k < 3; ++k) ((volatile int *)h)[k] = -1;
-                ctl(0, depth, h);
-                GG_TRY(gt_partition<0>(G, st, A, grid, box[(depth & 1) ^ 1]));
-                int nt = 0;
-                GG_TRY(host_word(st, h, &nt));
-                if (nt == 0) {
-                    GG_TRY(host_word(st, h + 1, &nunit));
-                    GG_TRY(host_word(st, h + 2, &nng));
-                    nlev = depth + 1;
-                    break;
-                }
+    hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, n, nr, rl, rh, T.nd,
+                       box[0], unit, L);
+    hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, n, nr, rl,
+                       pkd->f[GG_R].as<double>(), T.bits, T.px, T.py, T.pz, T.perm, box[0], L);
+    hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need[1], G.hst);
+    GG_HIP(hipGetLastError());
+    TileArgs A;
+    A.ts = ts;
+    A.mask = 0;
+    A.L = L;
+    A.tiles = G.gtile.as<int4>();
+    A.nd = T.nd;
+    A.x = T.px;
+    A.y = T.py;
+    A.z = T.pz;
+    A.src = T.perm;
+    A.bits = T.bits;
+    A.flag = G.gflag.as<unsigned long long>();
+    A.tcnt = G.gtcnt.as<int>();
+    A.tpre = A.tcnt + mtile;
+    A.posR = G.gposR.as<int>();
+    A.err = &L->err;
+    const int grid = (int)mtile;
+    auto ctl = [&](int mode, int depth, int *host) {
+        hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, mode, ts, depth, cap, L, T.nd,
+                           box[depth & 1], box[(depth & 1) ^ 1], G.gtile.as<int4>(), unit, host);
+    };
+    // msrBuildTree's active-type orders (master.c:4262).  A particle with
+    // the second order's bit has one of the first's, so where all have it
+    // both orders leave everything in place.
+    int lack = 0;
+    GG_TRY(host_word(st, G.hst, &lack));
+    if (lack) {
+        ctl(1, 0, G.hst + 1);
+        A.mask = GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE;
+        GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
+        A.mask = GG_TYPE_TREEACTIVE;
+        GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
+    }
+    int nunit = nr, nlev = 0;
+    if (maxRoot > MID) {
+        // The levels.  The host learns a level's tile count while its
+        // partition runs, in time to queue the next level behind it.
+        for (int depth = 0;; ++depth) {
+            GG_CHECK(depth < DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
+            int *h = G.hst + 16 + 4 * (depth & 3);
+            for (int k = 0; k < 2; ++k) ((volatile int *)h)[k] = -1;
+            ctl(0, depth, h);
+            GG_TRY(gt_partition<0>(G, st, A, grid, box[(depth & 1) ^ 1]));
+            int nt = 0;
+            GG_TRY(host_word(st, h, &nt));
+            if (nt == 0) {
+                GG_TRY(host_word(st, h + 1, &nunit));
+                nlev = depth;            // levels with a splitting cell
+                break;
             }
         }
-        if (nunit > 0)
-            hipLaunchKernelGGL(k_gt_mid, dim3(nunit), dim3(MID_T), 0, st, G.gunit.as<int>(), L,
-                               nBucket, nd, G.px.as<double>(), G.py.as<double>(),
-                               G.pz.as<double>(), G.perm.as<int>(), &L->err);
-        GG_HIP(hipGetLastError());
-        GLevel hl;
-        GG_HIP(hipMemcpyAsync(&hl, L, sizeof hl, hipMemcpyDeviceToHost, st));
-        GG_HIP(hipStreamSynchronize(st));
-        GG_CHECK(!hl.err, GG_EUNSUP,
-                 "a cell split leaves one side empty (positions differ in the last bit only)");
-        nng = hl.next;
-        // cells of at most LMAX particles: their subtrees in one launch, each
-        // in node slots reserved after the cells above them
-        GG_TRY(G.gbflag.reserve(sizeof(int) * (size_t)nng));
-        hipLaunchKernelGGL(k_gt_lmark, dim3(nblk(nng, 256)), dim3(256), 0, st, nng, nd,
-                           G.gbflag.as<int>(), G.gnit.as<int>());
-        int64_t nloc = 0, nres = 0;
-        GG_TRY(exclusive_scan_i64(st, G.gbflag.as<int>(), G.gchoff.as<int64_t>(), nng, G.scan,
-                                  &nloc));
-        GG_TRY(exclusive_scan_i64(st, G.gnit.as<int>(), G.gioff.as<int64_t>(), nng, G.scan, &nres));
-        GG_CHECK((size_t)nng + (size_t)nres <= cap, GG_EHIP, "tree cell capacity exceeded");
-        nn = nng;
-        if (nloc > 0) {
-            GG_TRY(G.glroot.reserve(sizeof(int) * (size_t)nloc));
-            GG_TRY(G.glused.reserve(sizeof(int) * (size_t)nloc));
-            GG_TRY(G.glbase.reserve(sizeof(int64_t) * ((size_t)nloc + 1)));
-            GG_TRY(G.gscr.reserve(sizeof(GNode) * (size_t)std::max<int64_t>(nres, 1)));
-            hipLaunchKernelGGL(k_gt_lcompact, dim3(nblk(nng, 256)), dim3(256), 0, st, nng,
-                               G.gbflag.as<int>(), G.gchoff.as<int64_t>(), G.glroot.as<int>());
-            hipLaunchKernelGGL(k_gt_local, dim3((unsigned)nloc), dim3(256), 0, st,
-                               G.glroot.as<int>(), G.gioff.as<int64_t>(), nBucket, nd,
-                               G.gscr.as<GNode>(), G.glused.as<int>(), G.px.as<double>(),
-                               G.py.as<double>(), G.pz.as<double>(), G.perm.as<int>(),
-                               &L->err);
-            GG_HIP(hipGetLastError());
-            int64_t nused = 0;
-            GG_TRY(exclusive_scan_i64(st, G.glused.as<int>(), G.glbase.as<int64_t>(), (int)nloc,
-                                      G.scan, &nused));
-            int err = 0;
-            GG_HIP(hipMemcpyAsync(&err, &L->err, sizeof(int), hipMemcpyDeviceToHost, st));
-            GG_HIP(hipStreamSynchronize(st));
-            GG_CHECK(!err, GG_EUNSUP,
-                     "a cell split leaves one side empty (positions differ in the last bit only)");
-            nn = nng + (int)nused;
-            hipLaunchKernelGGL(k_gt_lcopy, dim3((unsigned)nloc), dim3(256), 0, st,
-                               G.glroot.as<int>(), G.gioff.as<int64_t>(), G.glused.as<int>(),
-                               G.glbase.as<int64_t>(), nng, nd, G.gscr.as<GNode>());
-            GG_HIP(hipGetLastError());
-        }
-        // nodes by depth
-        const int ndep = std::max(nlev, hl.maxdep + 1) + LMAX + 1;
-        GG_CHECK(ndep <= DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
-        GG_TRY(G.gdcnt.reserve(sizeof(int) * 2 * (size_t)ndep));
-        GG_TRY(G.gdlist.reserve(sizeof(int) * (size_t)nn));
-        GG_HIP(hipMemsetAsync(G.gdcnt.p, 0, sizeof(int) * ndep, st));
-        hipLaunchKernelGGL(k_gt_depth_count, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, ndep, nd,
-                           G.gdcnt.as<int>());
-        std::vector<int> dcnt((size_t)ndep), doff((size_t)ndep + 1, 0);
-        GG_HIP(hipMemcpyAsync(dcnt.data(), G.gdcnt.p, sizeof(int) * ndep, hipMemcpyDeviceToHost,
-                              st));
-        GG_HIP(hipStreamSynchronize(st));
-        int nd_used = 0;
-        for (int d = 0; d < ndep; ++d) {
-            doff[d + 1] = doff[d] + dcnt[d];
-            if (dcnt[d]) nd_used = d + 1;
-        }
-        GG_HIP(hipMemcpyAsync(G.gdcnt.as<int>() + ndep, doff.data(), sizeof(int) * ndep,
-                              hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_gt_depth_list, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, ndep, nd,
-                           G.gdcnt.as<int>() + ndep, G.gdlist.as<int>());
-        depths.clear();
-        for (int d = 0; d < nd_used; ++d) depths.push_back({doff[d], dcnt[d]});
-        const int *dl = G.gdlist.as<int>();
-        // preorder numbering from subtree sizes
-        for (int d = (int)depths.size() - 1; d >= 0; --d)
-            if (depths[d].second)
-                hipLaunchKernelGGL(k_gt_size, dim3(nblk(depths[d].second, 256)), dim3(256), 0, st,
-                                   depths[d].second, dl + depths[d].first, nd);
-        std::vector<GNode> roots((size_t)nr);
-        GG_HIP(hipMemcpyAsync(roots.data(), nd, sizeof(GNode) * nr, hipMemcpyDeviceToHost, st));
-        GG_HIP(hipStreamSynchronize(st));
-        int pre = 0;
-        for (int k = 0; k < nr; ++k) {
-            roots[k].pre = pre;
-            pre += roots[k].size;
-        }
-        GG_HIP(hipMemcpyAsync(nd, roots.data(), sizeof(GNode) * nr, hipMemcpyHostToDevice, st));
-        for (size_t d = 0; d < depths.size(); ++d)
-            if (depths[d].second)
-                hipLaunchKernelGGL(k_gt_pre, dim3(nblk(depths[d].second, 256)), dim3(256), 0, st,
-                                   depths[d].second, dl + depths[d].first, nd);
-        GG_HIP(hipGetLastError());
-        GG_HIP(hipStreamSynchronize(st));
     }
-    const bool empty = nn == 0;
-    const int nNodes = empty ? 1 : nn;
-    // storage-order particle fields
-    if (n > 0)
-        hipLaunchKernelGGL(k_gt_gather, dim3(nblk(n, 256)), dim3(256), 0, st, n,
-                           G.perm.as<int>(), pkd->f[GG_MASS].as<double>(),
-                           pkd->f[GG_SOFT].as<double>(), pkd->f[GG_IACTIVE].as<uint32_t>(),
-                           G.pm.as<double>(), G.ph.as<double>(), G.pact.as<uint32_t>());
-    GG_TRY(G.wnode.reserve(sizeof(WalkNode) * nNodes));
-    GG_TRY(G.cell.reserve(sizeof(double) * CR_N * nNodes));
-    GG_TRY(G.momOH.reserve(sizeof(double) * OH_N * (iOrder >= 3 ? nNodes : 1)));
-    GG_TRY(G.tint.reserve(sizeof(int) * 6 * nNodes));
-    GG_TRY(G.tdbl.reserve(sizeof(double) * 8 * nNodes));
-    GG_TRY(G.gcm.reserve(sizeof(double) * 5 * nNodes));
-    int nb = 0;
-    if (empty) {   // an empty store: one empty bucket (pkd.c:2684-2712)
+    // the units and the subtrees below them, then the records upwards
+    int *ht = G.hst + 4;
+    if (nunit > 0)
+        hipLaunchKernelGGL(k_gt_mid, dim3(nunit), dim3(MID_T), 0, st, unit, cap, L, T.nd, T.px,
+                           T.py, T.pz, T.perm, sub, seg, segl, useg);
+    const int gsub = std::min(std::max(n / 64, 1), 2048);
+#define GG_BY_ORDER(K, GRID, BLOCK, ...)                                                          \
+    do {                                                                                          \
+        if (order == 4) hipLaunchKernelGGL(K<4>, GRID, BLOCK, 0, st, __VA_ARGS__);                \
+        else if (order == 3) hipLaunchKernelGGL(K<3>, GRID, BLOCK, 0, st, __VA_ARGS__);           \
+        else hipLaunchKernelGGL(K<2>, GRID, BLOCK, 0, st, __VA_ARGS__);                           \
+    } while (0)
+    GG_BY_ORDER(k_gt_sub, dim3(gsub), dim3(SUB_T), T);
+    if (nunit > 0) GG_BY_ORDER(k_gt_up_unit, dim3(nunit), dim3(64), T);
+    for (int d = nlev - 1; d >= 0; --d)
+        GG_BY_ORDER(k_gt_up_level, dim3(nblk(2 * mbox, 256)), dim3(256), T, d);
+    hipLaunchKernelGGL(k_gt_totals, dim3(1), dim3(256), 0, st, nr, T, ht);
+    if (nunit > 0) GG_BY_ORDER(k_gt_up_bmax, dim3(nunit), dim3(256), T);
+    GG_HIP(hipGetLastError());
+    int tot[6];   // error word, cells, active buckets, largest bucket, slots above LMAX, subtrees
+    for (int k = 0; k < 6; ++k) GG_TRY(host_word(st, ht + k, tot + k));
+    const int err = tot[0], nn = tot[1], nb = tot[2], nup = tot[4], nsub = tot[5];
+    GG_CHECK(!(err & 1), GG_EUNSUP,
+             "a cell split leaves one side empty (positions differ in the last bit only)");
+    *room = !(err & 2);
+    if (!*room) return GG_OK;
+    G.maxBucket = tot[3];     // > 64 only for cells of coincident particles (pkd.c:2489)
+    GG_TRY(G.wnode.reserve(sizeof(WalkNode) * (size_t)nn));
+    GG_TRY(G.cell.reserve(sizeof(double) * CR_N * (size_t)nn));
+    GG_TRY(G.momOH.reserve(sizeof(double) * OH_N * (size_t)(iOrder >= 3 ? nn : 1)));
+    GG_TRY(G.tint.reserve(sizeof(int) * 6 * (size_t)nn));
+    GG_TRY(G.tdbl.reserve(sizeof(double) * 8 * (size_t)nn));
+    GG_TRY(G.bucket.reserve(sizeof(int) * std::max(nb, 1)));
+    GG_TRY(G.broot.reserve(sizeof(int) * std::max(nb, 1)));
+    GG_TRY(G.bbox.reserve(sizeof(double) * 8 * (size_t)std::max(nb, 1)));
+    EmitArgs E;
+    E.iOpenType = iOpenType;
+    E.dCrit = dCrit;
+    E.tint = G.tint.as<int>();
+    E.tdbl = G.tdbl.as<double>();
+    E.wn = G.wnode.as<WalkNode>();
+    E.cell = G.cell.as<double>();
+    E.momOH = G.momOH.as<double>();
+    E.bucket = G.bucket.as<int>();
+    E.broot = G.broot.as<int>();
+    E.bbox = G.bbox.as<double>();
+    const int nub = nblk(nup, 256);
+    GG_BY_ORDER(k_gt_emit, dim3(nub + nblk(nsub, 4)), dim3(256), nub, nup, nsub, T, E);
+#undef GG_BY_ORDER
+    GG_HIP(hipGetLastError());
+    G.nNodes = nn;
+    G.nb = nb;
+    return GG_OK;
+}
+
+int gtree_build(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iOpenType, double dCrit,
+                int iOrder)
+{
+    GravDev &G = pkd->grav;
+    hipStream_t st = pkd->stream;
+    const int n = pkd->nLocal;
+    G.built = 0;
+    if (n == 0) {   // an empty store: one empty bucket (pkd.c:2684-2712)
         const int ti[6] = {-1, 0, -1, -1, -1, 0};
         const double td[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         WalkNode w{};
         w.pLower = 0;
         w.pUpper = -1;
         w.iLower = w.iNext = w.iUpper = -1;
+        GG_TRY(G.wnode.reserve(sizeof w));
+        GG_TRY(G.tint.reserve(sizeof ti));
+        GG_TRY(G.tdbl.reserve(sizeof td));
         GG_HIP(hipMemcpyAsync(G.tint.p, ti, sizeof ti, hipMemcpyHostToDevice, st));
         GG_HIP(hipMemcpyAsync(G.tdbl.p, td, sizeof td, hipMemcpyHostToDevice, st));
         GG_HIP(hipMemcpyAsync(G.wnode.p, &w, sizeof w, hipMemcpyHostToDevice, st));
         GG_HIP(hipStreamSynchronize(st));
+        G.nNodes = 1;
+        G.nb = G.maxBucket = 0;
     } else {
-        // mass, softening, c.o.m.: deepest level first
-        for (int d = (int)depths.size() - 1; d >= 0; --d)
-            if (depths[d].second)
-                hipLaunchKernelGGL(k_gt_mass, dim3(nblk(depths[d].second, 256)), dim3(256), 0, st,
-                                   depths[d].second, G.gdlist.as<int>() + depths[d].first, nd,
-                                   G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
-                                   G.pm.as<double>(), G.ph.as<double>(), G.gcm.as<double>());
-        // moments: work items of MOM_CH particles per cell
-        hipLaunchKernelGGL(k_gt_items, dim3(nblk(nn, 256)), dim3(256), 0, st, 0, nn, MOM_CH, 0,
-                           nd, G.gnit.as<int>());
-        int64_t nitem = 0;
-        GG_TRY(exclusive_scan_i64(st, G.gnit.as<int>(), G.gioff.as<int64_t>(), nn, G.scan, &nitem));
-        GG_TRY(G.gpart.reserve(sizeof(double) * NM * std::max<int64_t>(nitem, 1)));
-        GG_TRY(G.gicell.reserve(sizeof(int) * std::max<int64_t>(nitem, 1)));
-        hipLaunchKernelGGL(k_gt_itemcell, dim3(nblk(nn, 256)), dim3(256), 0, st, nn,
-                           G.gioff.as<int64_t>(), G.gicell.as<int>());
-        if (nitem > 0) {
-            auto mom = iOrder >= 4 ? k_gt_moments<4> : (iOrder >= 3 ? k_gt_moments<3>
-                                                                      : k_gt_moments<2>);
-            hipLaunchKernelGGL(mom, dim3(nblk(nitem, 4)), dim3(256), 0, st, (int)nitem,
-                               G.gicell.as<int>(), G.gioff.as<int64_t>(), nd, G.gcm.as<double>(),
-                               G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
-                               G.pm.as<double>(), G.gpart.as<double>());
-            auto small = iOrder >= 4 ? k_gt_moments_small<4>
-                                     : (iOrder >= 3 ? k_gt_moments_small<3> : k_gt_moments_small<2>);
-            hipLaunchKernelGGL(small, dim3(nblk(nitem, 256)), dim3(256), 0, st, (int)nitem,
-                               G.gicell.as<int>(), nd, G.gcm.as<double>(), G.px.as<double>(),
-                               G.py.as<double>(), G.pz.as<double>(), G.pm.as<double>(),
-                               G.gpart.as<double>());
-        }
-        const int nv = iOrder >= 4 ? 31 : (iOrder >= 3 ? 16 : 6);
-        hipLaunchKernelGGL(k_gt_combine, dim3(nblk(nn, 4)), dim3(256), 0, st, nn, nv,
-                           G.gioff.as<int64_t>(), G.gpart.as<double>());
-        hipLaunchKernelGGL(k_gt_emit, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, iOrder,
-                           iOpenType, dCrit, nd, G.gcm.as<double>(), G.gioff.as<int64_t>(),
-                           G.gpart.as<double>(), G.tint.as<int>(), G.tdbl.as<double>(),
-                           G.wnode.as<WalkNode>(), G.cell.as<double>(), G.momOH.as<double>());
-        // active buckets in preorder
-        GG_TRY(G.gbflag.reserve(sizeof(int) * nn));
-        GG_TRY(G.gbb8.reserve(sizeof(double) * 8 * nn));
-        GG_TRY(G.grootof.reserve(sizeof(int) * nn));
-        hipLaunchKernelGGL(k_gt_bucket, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, nd,
-                           G.px.as<double>(), G.py.as<double>(), G.pz.as<double>(),
-                           G.ph.as<double>(), G.pact.as<uint32_t>(), G.gbflag.as<int>(),
-                           G.gbb8.as<double>(), &L->maxb);
-        hipLaunchKernelGGL(k_gt_rootof, dim3(nblk(nn, 256)), dim3(256), 0, st, nn, nd,
-                           G.grootof.as<int>());
-        int64_t nb64 = 0;
-        GG_TRY(exclusive_scan_i64(st, G.gbflag.as<int>(), G.gchoff.as<int64_t>(), nn, G.scan,
-                                  &nb64));
-        nb = (int)nb64;
-        int maxb = 0;
-        GG_HIP(hipMemcpyAsync(&maxb, &L->maxb, sizeof(int), hipMemcpyDeviceToHost,
-                              st));
-        GG_HIP(hipStreamSynchronize(st));
-        G.maxBucket = maxb;     // > 64 only for cells of coincident particles (pkd.c:2489)
-        GG_TRY(G.bucket.reserve(sizeof(int) * std::max(nb, 1)));
-        GG_TRY(G.broot.reserve(sizeof(int) * std::max(nb, 1)));
-        GG_TRY(G.bbox.reserve(sizeof(double) * 8 * std::max(nb, 1)));
-        hipLaunchKernelGGL(k_gt_bucket_list, dim3(nblk(nn, 256)), dim3(256), 0, st, nn,
-                           G.gbflag.as<int>(), G.gchoff.as<int64_t>(), G.gbb8.as<double>(),
-                           G.grootof.as<int>(), G.bucket.as<int>(), G.bbox.as<double>(),
-                           G.broot.as<int>());
-        GG_HIP(hipGetLastError());
+        // Slots: buckets of nBucket hold about 0.65 nBucket particles, so
+        // 3 n / nBucket cells; twice that fits all but odd distributions,
+        // which build again with the most a tree can have.
+        const int64_t most = 2 * (int64_t)n + 2;
+        const int64_t guess = 6 * (int64_t)n / nBucket + 2 * (int64_t)nSys + 4096;
+        GG_CHECK(most <= INT_MAX, GG_EINVAL, "%d particles: too many for one tree", n);
+        bool room = false;
+        GG_TRY(gtree_try(pkd, nSys, sysOff, nBucket, iOpenType, dCrit, iOrder,
+                         (int)std::min(most, guess), &room));
+        if (!room)
+            GG_TRY(gtree_try(pkd, nSys, sysOff, nBucket, iOpenType, dCrit, iOrder, (int)most,
+                             &room));
+        GG_CHECK(room, GG_EHIP, "tree cell capacity exceeded");
     }
+    const int nb = G.nb;
     GG_TRY(G.cnt.reserve(sizeof(int) * 3 * std::max(nb, 1)));
     GG_TRY(G.off.reserve(sizeof(int64_t) * (3 * (size_t)std::max(nb, 1) + 1)));
-    GG_HIP(hipStreamSynchronize(st));
-    G.nb = nb;
     G.n = n;
-    G.nNodes = nNodes;
     G.iRoot = 0;
     G.nSys = nSys;
     G.iOrder = iOrder;

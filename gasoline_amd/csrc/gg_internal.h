@@ -79,10 +79,9 @@ struct GravDev {
     DevBuf broot;          // per active bucket: the root of its tree
     DevBuf tint, tdbl;     // per node: 6 ints, 8 doubles (gg_tree_info's layout)
     // tree build scratch
-    DevBuf gposR, gnode, gbox, gtile, gflag, gtcnt, gunit, glev, gchoff, groot, gcm;
+    DevBuf gposR, gnode, gm, gbox, gtile, gflag, gtcnt, gunit, gsub, gseg, glev, groot, gbb8;
     static constexpr int NHST = 32;
     int *hst = nullptr;             // pinned words the build's kernels tell the host
-    DevBuf gnit, gioff, gicell, gpart, gbflag, gbb8, grootof, glroot, gdcnt, gdlist, glused, glbase, gscr;
     DevBuf ewt, emom, ewh;          // Ewald: moment partials, root moments, k-space table
     DevBuf ewl;                     // Ewald: real-space terms per slot (for fWeight)
     int64_t ewLoops = 0;            // real-space terms of the last Ewald pass
@@ -103,8 +102,8 @@ struct GravDev {
     {
         DevBuf *all[] = {&px, &py, &pz, &pm, &ph, &pact, &perm, &wnode, &cell, &momOH, &bucket,
                          &bbox, &cnt, &off, &ent, &acc, &stats, &scan, &werr, &broot, &tint,
-                         &tdbl, &gposR, &gnode, &gbox, &gtile, &gflag, &gtcnt, &gunit, &glev,
-                         &gchoff, &groot, &gcm, &gnit, &gioff, &gicell, &gpart, &gbflag, &gbb8, &grootof, &glroot, &gdcnt, &gdlist, &glused, &glbase, &gscr,
+                         &tdbl, &gposR, &gnode, &gm, &gbox, &gtile, &gflag, &gtcnt, &gunit, &gsub,
+                         &gseg, &glev, &groot, &gbb8,
                          &ewt, &emom, &ewh, &ewl, &qorder, &qbin, &qhist, &qnext};
         for (DevBuf *b : all) b->release();
         if (hst) (void)hipHostFree(hst);

@@ -77,6 +77,17 @@ def test_tree_large_coincident_bucket(gpu, clump):
     check(gpu, r, m, np.full(n, 0.01), 16, 4)
 
 
+def test_tree_with_many_more_cells_than_usual(gpu):
+    # groups of 30 particles at 2^-k beside 64 coincident ones: buckets of one
+    # particle though they may hold 64, six times the usual number of cells
+    g, k = 300, np.arange(30)
+    one = np.zeros((94, 3))
+    one[:30, 0] = 2.0 ** -k
+    r = np.concatenate([one + [4.0 * (i % 20), 4.0 * (i // 20), 0.0] for i in range(g)])
+    m = np.full(len(r), 1.0 / len(r))
+    check(gpu, r, m, np.full(len(r), 0.01), 64, 4)
+
+
 def test_forest_of_large_and_small_systems(gpu):
     sizes = [1, 4096, 0, 9000, 17, 4097, 300, 700]
     off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
