@@ -215,6 +215,7 @@ extern "C" int gg_finish(GGPKD pkd)
     (void)hipStreamSynchronize(pkd->stream);
     for (auto &b : pkd->f) b.release();
     pkd->red.release();
+    if (pkd->redHost) (void)hipHostFree(pkd->redHost);
     GravDev &G = pkd->grav;
     G.release_all();
     if (G.gexec) (void)hipGraphExecDestroy(G.gexec);

@@ -1673,10 +1673,8 @@ __global__ __launch_bounds__(256) void k_gt_emit(int nub, int nup, int nsub, Tre
 
 }  // namespace
 
-// Waits until the kernels queued on the stream have written *p (pinned,
-// tell_host; -1 before).  The stream running dry without it is an error, so
-// the wait always ends.
-static int host_word(hipStream_t st, const int *p, int *v)
+// The stream running dry without the word is an error, so the wait always ends.
+int host_word(hipStream_t st, const int *p, int *v)
 {
     for (unsigned it = 0;; ++it) {
         *v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
@@ -1686,7 +1684,7 @@ static int host_word(hipStream_t st, const int *p, int *v)
         if (e == hipErrorNotReady) continue;
         GG_HIP(e);
         *v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
-        GG_CHECK(*v != -1, GG_EHIP, "the tree build's device state never arrived");
+        GG_CHECK(*v != -1, GG_EHIP, "a device word never reached the host");
         return GG_OK;
     }
 }

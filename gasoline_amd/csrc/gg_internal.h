@@ -250,9 +250,14 @@ struct gg_pkd_s {
     gg::Timers tm;
     gg::AosStage aos;
     gg::DevBuf red;                // reductions of the elementwise updates
+    unsigned *redHost = nullptr;   // their words on the host (pinned)
+    int redZero = 0;               // the device words are zero
 };
 
 namespace gg {
+// Waits until the kernels queued on the stream have written the pinned word
+// *p (a system-scope release store; -1 before): GG_OK and its value in *v.
+int host_word(hipStream_t st, const int *p, int *v);
 int field_width(int field);                 // values per particle
 int field_is32(int field);                  // 32-bit integer field (iActive, iRung)
 int ensure_field(GGPKD pkd, int field);     // allocate (zeroed) if missing

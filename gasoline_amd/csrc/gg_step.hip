@@ -11,7 +11,6 @@
 #include <cfloat>
 #include <cstring>
 #include <initializer_list>
-#include <vector>
 
 #pragma clang fp contract(off)
 
@@ -63,24 +62,70 @@ __global__ void k_kick(KickArgs K)
     }
 }
 
+// Kernels that count or reduce over the store run at most MAXB blocks of TB
+// threads, each over every gridDim-th chunk, and add up a block's lanes in LDS
+// first: one atomic a wavefront on one address is served at about 10 ns each,
+// which was most of gg_active_type's 201 us at 1M particles (20 us so).
+constexpr int TB = 512, MAXB = 512;
+int red_grid(size_t n)
+{
+    const size_t b = (n + TB - 1) / TB;
+    return (int)(b < (size_t)MAXB ? b : (size_t)MAXB);
+}
+
+template <class T, class F>
+__device__ __forceinline__ T block_red(T v, F f)
+{
+    __shared__ T part[TB / 64];
+    for (int o = 32; o > 0; o >>= 1) v = f(v, __shfl_xor(v, o));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = part[0];
+    for (int k = 1; k < TB / 64; ++k) v = f(v, part[k]);
+    __syncthreads();
+    return v;
+}
+
+// A call's counts and its blocks' tickets in one 64-bit word: bits 0..33 a
+// count (<= 3n), 34..43 and 44..53 numbers of blocks, 54..63 the ticket (<=
+// MAXB each).  The block that adds last therefore holds the totals: it hands
+// them to the host (pinned words h[1], h[2], then the flag h[0]) and clears
+// the word for the next call, all inside the kernel that counts.
+constexpr int TK_A = 34, TK_B = 44, TK_T = 54;
+static_assert(MAXB < 1 << (TK_B - TK_A) && MAXB < 1 << (64 - TK_T), "blocks fit their fields");
+
+__device__ __forceinline__ void hand_over(unsigned long long mine, unsigned *red, unsigned *h)
+{
+    unsigned long long *w = (unsigned long long *)red;
+    mine += 1ull << TK_T;
+    const unsigned long long tot = atomicAdd(w, mine) + mine;
+    if ((int)(tot >> TK_T) != (int)gridDim.x) return;
+    atomicExch(w, 0ull);
+    __hip_atomic_store(h + 1, (unsigned)tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(h + 2, (unsigned)(tot >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(h, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // r += dDelta v, wrapped into [c - L/2, c + L/2) when periodic.
 __global__ void k_drift(int n, double dt, int per, double c0, double c1, double c2, double L0,
                         double L1, double L2, const double *__restrict__ v, double *__restrict__ r,
-                        unsigned *__restrict__ out)
+                        unsigned *__restrict__ red, unsigned *__restrict__ h)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double c[3] = {c0, c1, c2}, L[3] = {L0, L1, L2};
-    for (int j = 0; j < 3; ++j) {
-        const size_t e = 3 * (size_t)i + j;
+    const size_t n3 = 3 * (size_t)n, step = (size_t)gridDim.x * TB;
+    unsigned long long out = 0;
+    for (size_t e = (size_t)blockIdx.x * TB + threadIdx.x; e < n3; e += step) {
         double x = r[e] + dt * v[e];
         if (per) {
-            if (x >= c[j] + 0.5 * L[j]) x -= L[j];
-            if (x < c[j] - 0.5 * L[j]) x += L[j];
-            if (!(x >= c[j] - 0.5 * L[j] && x < c[j] + 0.5 * L[j])) atomicAdd(out, 1u);
+            const int j = (int)(e % 3);
+            const double c = j == 0 ? c0 : j == 1 ? c1 : c2, L = j == 0 ? L0 : j == 1 ? L1 : L2;
+            if (x >= c + 0.5 * L) x -= L;
+            if (x < c - 0.5 * L) x += L;
+            if (!(x >= c - 0.5 * L && x < c + 0.5 * L)) ++out;
         }
         r[e] = x;
     }
+    out = block_red(out, [](auto a, auto b) { return a + b; });
+    if (threadIdx.x == 0) hand_over(out, red, h);
 }
 
 // pkdKickVpred, NOCOOLING: gas particles only; bad counts uPred < 0
@@ -89,19 +134,25 @@ __global__ void k_kick_vpred(int n, double vf1, double vf2, double du, int bGasU
                              const uint32_t *__restrict__ bits, const double *__restrict__ a,
                              const double *__restrict__ udpdv, const double *__restrict__ udav,
                              const double *__restrict__ uddif, double *__restrict__ vpred,
-                             double *__restrict__ upred, unsigned *__restrict__ bad)
+                             double *__restrict__ upred, unsigned *__restrict__ red,
+                             unsigned *__restrict__ h)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !(bits[i] & GG_TYPE_GAS)) return;
-    for (int j = 0; j < 3; ++j) {
-        const size_t e = 3 * (size_t)i + j;
-        vpred[e] = vpred[e] * vf1 + a[e] * vf2;
+    unsigned long long bad = 0;
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB) {
+        if (!(bits[i] & GG_TYPE_GAS)) continue;
+        for (int j = 0; j < 3; ++j) {
+            const size_t e = 3 * i + j;
+            vpred[e] = vpred[e] * vf1 + a[e] * vf2;
+        }
+        if (bGasU) {
+            const double u = upred[i] + (udpdv[i] + udav[i] + uddif[i]) * du;
+            upred[i] = u;
+            if (!(u >= 0.0)) ++bad;
+        }
     }
-    if (bGasU) {
-        const double u = upred[i] + (udpdv[i] + udav[i] + uddif[i]) * du;
-        upred[i] = u;
-        if (!(u >= 0.0)) atomicAdd(bad, 1u);
-    }
+    bad = block_red(bad, [](auto p, auto q) { return p + q; });
+    if (threadIdx.x == 0) hand_over(bad, red, h);
 }
 
 __global__ void k_init_dt(int n, double dDelta, const uint32_t *__restrict__ bits,
@@ -114,16 +165,21 @@ __global__ void k_init_dt(int n, double dDelta, const uint32_t *__restrict__ bit
 // pkdGravStep: dt = min(dt, dEta/sqrt(dtGrav)); bad counts dtGrav <= 0.
 __global__ void k_grav_step(int n, double dEta, const uint32_t *__restrict__ bits,
                             const double *__restrict__ dtg, double *__restrict__ dt,
-                            unsigned *__restrict__ bad)
+                            unsigned *__restrict__ red, unsigned *__restrict__ h)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !(bits[i] & GG_TYPE_ACTIVE)) return;
-    if (!(dtg[i] > 0.0)) {
-        atomicAdd(bad, 1u);
-        return;
+    unsigned long long bad = 0;
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB) {
+        if (!(bits[i] & GG_TYPE_ACTIVE)) continue;
+        if (!(dtg[i] > 0.0)) {
+            ++bad;
+            continue;
+        }
+        const double d = dEta / sqrt(dtg[i]);
+        if (d < dt[i]) dt[i] = d;
     }
-    const double d = dEta / sqrt(dtg[i]);
-    if (d < dt[i]) dt[i] = d;
+    bad = block_red(bad, [](auto p, auto q) { return p + q; });
+    if (threadIdx.x == 0) hand_over(bad, red, h);
 }
 
 // pkdAccelStep: the acceleration criterion (softening, or h for gas) and
@@ -175,15 +231,16 @@ struct SphStepArgs {
     const uint32_t *bits;
     const double *fb2, *c, *u, *udpdv, *udav, *uddif, *rho, *diff;
     double *dtNew, *dt;
-    unsigned long long *minKey;      // smallest dt of the gas, as dkey
+    unsigned long long *minKey;      // largest ~dkey of the gas: its smallest dt (0: no gas)
 };
 
 // pkdSphStep, NOCOOLING without THERMALCOND/TWOPHASE/UNONCOOL.
 __global__ void k_sph_step(SphStepArgs A)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     unsigned long long key = ~0ull;
-    if (i < A.n && (A.bits[i] & GG_TYPE_GAS)) {
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)A.n;
+         i += (size_t)gridDim.x * TB) {
+        if (!(A.bits[i] & GG_TYPE_GAS)) continue;
         if (A.bits[i] & GG_TYPE_ACTIVE) {
             const double ph = sqrt(0.25 * A.fb2[i]);
             double dT = A.dtNew[i];
@@ -210,13 +267,11 @@ __global__ void k_sph_step(SphStepArgs A)
             }
             if (dT < A.dt[i]) A.dt[i] = dT;
         }
-        key = dkey(A.dt[i]);
+        const unsigned long long k = dkey(A.dt[i]);
+        key = k < key ? k : key;
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long k2 = __shfl_xor(key, o);
-        key = k2 < key ? k2 : key;
-    }
-    if ((threadIdx.x & 63) == 0 && key != ~0ull) atomicMin(A.minKey, key);
+    key = block_red(key, [](auto p, auto q) { return q < p ? q : p; });
+    if (threadIdx.x == 0 && key != ~0ull) atomicMax(A.minKey, ~key);
 }
 
 // pkdOneParticleDtToRung (pkd.c:4704-4726)
@@ -269,9 +324,9 @@ __global__ void k_dt_to_rung(int n, int iRung, double dDelta, int iMaxRung, int 
                              const double *__restrict__ dt, int *__restrict__ rung,
                              double *__restrict__ dtOld, int *__restrict__ red)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     int top = -1, ideal = 0;
-    if (i < n) {
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB) {
         int r = rung[i];
         if (r >= iRung) {
             if (!(bits[i] & GG_TYPE_ACTIVE)) {
@@ -282,7 +337,7 @@ __global__ void k_dt_to_rung(int n, int iRung, double dDelta, int iMaxRung, int 
                     atomicAdd(&red[0], 1);
                 } else {
                     int t = one_dt_to_rung(iRung, dDelta, d);
-                    ideal = t + 1;
+                    ideal = max(ideal, t + 1);
                     if (t >= iMaxRung) t = iMaxRung - 1;
                     r = t;
                     dtOld[i] = d;
@@ -292,13 +347,11 @@ __global__ void k_dt_to_rung(int n, int iRung, double dDelta, int iMaxRung, int 
             }
             rung[i] = r;
         }
-        top = r;
+        top = max(top, r);
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        top = max(top, __shfl_xor(top, o));
-        ideal = max(ideal, __shfl_xor(ideal, o));
-    }
-    if ((threadIdx.x & 63) == 0) {
+    top = block_red(top, [](auto p, auto q) { return max(p, q); });
+    ideal = block_red(ideal, [](auto p, auto q) { return max(p, q); });
+    if (threadIdx.x == 0) {
         if (top >= 0) atomicMax(&red[1], top);
         if (ideal > 0) atomicMax(&red[2], ideal);
     }
@@ -313,20 +366,20 @@ __global__ void k_dt_to_rung(int n, int iRung, double dDelta, int iMaxRung, int 
 //   TB_RESET   (pkdResetType): iSetMask cleared on the matching ones.
 // Tests: TT_ANY bits & iTestMask nonzero (TYPETest), TT_EXACT (bits &
 // iFilterMask) == iTestMask (TYPEFilter), TT_ALL every particle.
-// count[0] = matching particles, count[1] = particles whose TYPE_ACTIVE bit
-// changed, count[2] = particles whose TYPE_GAS bit changed.
+// With red it hands over the matching particles and, as the fields A and B,
+// the blocks where a TYPE_ACTIVE and a TYPE_GAS bit changed.
 enum { TB_ACTIVE = 0, TB_SET = 1, TB_RESET = 2 };
 enum { TT_ANY = 0, TT_EXACT = 1, TT_ALL = 2 };
 __global__ void k_type_bits(int n, int op, int test, uint32_t iFilterMask, uint32_t iTestMask,
                             uint32_t iSetMask, int bRung, int iRung, int bGreater,
                             const int *__restrict__ rung, uint32_t *__restrict__ bits,
-                            int *__restrict__ count)
+                            unsigned *__restrict__ red, unsigned *__restrict__ h)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool on = false, dAct = false, dGas = false;
-    if (i < n) {
+    unsigned cnt = 0, diff = 0;
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB) {
         const uint32_t b = bits[i];
-        on = test == TT_ALL ? true
+        bool on = test == TT_ALL ? true
              : test == TT_EXACT ? (b & iFilterMask) == iTestMask : (b & iTestMask) != 0;
         if (bRung) {
             const int r = rung[i];
@@ -335,25 +388,42 @@ __global__ void k_type_bits(int n, int op, int test, uint32_t iFilterMask, uint3
         uint32_t nb = b;
         if (op == TB_ACTIVE) nb = on ? (b | iSetMask) : (b & ~iSetMask);
         else if (on) nb = op == TB_SET ? (b | iSetMask) : (b & ~iSetMask);
-        dAct = ((nb ^ b) & GG_TYPE_ACTIVE) != 0;
-        dGas = ((nb ^ b) & GG_TYPE_GAS) != 0;
         if (nb != b) bits[i] = nb;
+        cnt += on;
+        diff |= nb ^ b;
     }
-    const int c0 = __popcll(__ballot(on)), c1 = __popcll(__ballot(dAct)),
-              c2 = __popcll(__ballot(dGas));
-    if ((threadIdx.x & 63) == 0) {
-        if (c0) atomicAdd(count, c0);
-        if (c1) atomicAdd(count + 1, c1);
-        if (c2) atomicAdd(count + 2, c2);
-    }
+    if (!red) return;
+    cnt = block_red(cnt, [](auto p, auto q) { return p + q; });
+    diff = block_red(diff, [](auto p, auto q) { return p | q; });
+    if (threadIdx.x) return;
+    hand_over((unsigned long long)cnt | (unsigned long long)!!(diff & GG_TYPE_ACTIVE) << TK_A |
+                  (unsigned long long)!!(diff & GG_TYPE_GAS) << TK_B,
+              red, h);
 }
 
 __global__ void k_rung_count(int n, const int *__restrict__ rung, int *__restrict__ red)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool on = i < n && rung[i] == red[1];
-    const int c = __popcll(__ballot(on));
-    if ((threadIdx.x & 63) == 0 && c) atomicAdd(&red[3], c);
+    const int top = red[1];
+    int c = 0;
+    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB)
+        c += rung[i] == top;
+    c = block_red(c, [](auto p, auto q) { return p + q; });
+    if (threadIdx.x == 0 && c) atomicAdd(&red[3], c);
+}
+
+// Hands red[0..n) to the host (pinned words h[1..n], then the flag h[0]) and
+// leaves them zero for the next call.
+__global__ void k_red_tell(int n, unsigned *__restrict__ red, unsigned *__restrict__ h)
+{
+    const int t = threadIdx.x;
+    if (t < n) {
+        __hip_atomic_store(h + 1 + t, red[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        red[t] = 0;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(h, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace
@@ -362,6 +432,60 @@ __global__ void k_rung_count(int n, const int *__restrict__ rung, int *__restric
 using namespace gg;
 
 namespace {
+// The reductions of the calls below: words that the kernels count into.  They
+// are zero when a call begins (hand_over and k_red_tell leave them so) and
+// come back through pinned memory that the host polls, in place of a fill
+// before the work and a copy and a stream synchronisation behind it, which
+// took longer than the work itself on the stores these calls are made for
+// most often: at 50k particles gg_active_type 33 -> 16 us a call, gg_drift 27 -> 16.
+constexpr int NRED = 64;
+
+int red_begin(GGPKD pkd, unsigned **red)
+{
+    if (!pkd->redHost)
+        GG_HIP(hipHostMalloc((void **)&pkd->redHost, sizeof(unsigned) * (NRED + 1),
+                             hipHostMallocDefault));
+    GG_TRY(pkd->red.reserve(sizeof(unsigned) * NRED));
+    if (!pkd->redZero)
+        GG_HIP(hipMemsetAsync(pkd->red.p, 0, sizeof(unsigned) * NRED, pkd->stream));
+    pkd->redZero = 0;   // until red_end has seen the words come back
+    *red = pkd->red.as<unsigned>();
+    __atomic_store_n(pkd->redHost, ~0u, __ATOMIC_RELEASE);
+    return GG_OK;
+}
+
+// Waits for the kernel that hands the words over; out[0..n) are they.
+int red_wait(GGPKD pkd, int n, unsigned *out)
+{
+    unsigned *h = pkd->redHost;
+    int flag = 0;
+    GG_TRY(host_word(pkd->stream, (const int *)h, &flag));
+    pkd->redZero = 1;
+    for (int k = 0; k < n; ++k) out[k] = h[1 + k];
+    return GG_OK;
+}
+
+// The same for words that no kernel hands over by itself.
+int red_end(GGPKD pkd, int n, unsigned *out)
+{
+    hipLaunchKernelGGL(k_red_tell, dim3(1), dim3(64), 0, pkd->stream, n,
+                       pkd->red.as<unsigned>(), pkd->redHost);
+    GG_HIP(hipGetLastError());
+    return red_wait(pkd, n, out);
+}
+
+// The count of the kernel that handed over.
+int red_count(GGPKD pkd, unsigned long long *cnt, int *a, int *b)
+{
+    unsigned w[2];
+    GG_TRY(red_wait(pkd, 2, w));
+    const unsigned long long t = (unsigned long long)w[1] << 32 | w[0];
+    *cnt = t & ((1ull << TK_A) - 1);
+    if (a) *a = (int)(t >> TK_A & ((1u << (TK_B - TK_A)) - 1));
+    if (b) *b = (int)(t >> TK_B & ((1u << (TK_T - TK_B)) - 1));
+    return GG_OK;
+}
+
 int need_fields(GGPKD pkd, std::initializer_list<int> f)
 {
     for (int k : f) GG_TRY(ensure_field(pkd, k));
@@ -426,33 +550,23 @@ extern "C" int gg_drift(GGPKD pkd, double dDelta, const double *fCenter, int bPe
     if (n == 0) return GG_OK;
     GG_CHECK(pkd->f[GG_R].p, GG_ESTATE, "positions must be put before gg_drift");
     GG_TRY(ensure_field(pkd, GG_V));
-    DevBuf bad;
-    GG_TRY(bad.reserve(sizeof(unsigned)));
+    unsigned *red;
+    unsigned long long nb = 0;
+    GG_TRY(red_begin(pkd, &red));
     const double c[3] = {bPeriodic ? fCenter[0] : 0, bPeriodic ? fCenter[1] : 0,
                          bPeriodic ? fCenter[2] : 0};
     const double L[3] = {bPeriodic ? fPeriod[0] : 0, bPeriodic ? fPeriod[1] : 0,
                          bPeriodic ? fPeriod[2] : 0};
-    unsigned nb = 0;
-    int rc = GG_OK;
-    if (hipMemsetAsync(bad.p, 0, sizeof(unsigned), pkd->stream) != hipSuccess) rc = GG_EHIP;
-    if (rc == GG_OK) {
-        hipLaunchKernelGGL(k_drift, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, dDelta,
-                           bPeriodic, c[0], c[1], c[2], L[0], L[1], L[2],
-                           pkd->f[GG_V].as<double>(), pkd->f[GG_R].as<double>(),
-                           bad.as<unsigned>());
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(&nb, bad.p, sizeof(unsigned), hipMemcpyDeviceToHost, pkd->stream) !=
-                hipSuccess ||
-            hipStreamSynchronize(pkd->stream) != hipSuccess)
-            rc = GG_EHIP;
-    }
-    bad.release();
-    GG_CHECK(rc == GG_OK, rc, "gg_drift: HIP launch or copy failed");
+    hipLaunchKernelGGL(k_drift, dim3(red_grid(3 * (size_t)n)), dim3(TB), 0, pkd->stream, n, dDelta,
+                       bPeriodic, c[0], c[1], c[2], L[0], L[1], L[2],
+                       pkd->f[GG_V].as<double>(), pkd->f[GG_R].as<double>(), red, pkd->redHost);
+    GG_HIP(hipGetLastError());
+    GG_TRY(red_count(pkd, &nb, nullptr, nullptr));
     pkd->sph.built = 0;    // the trees describe the old positions
     pkd->sph.listValid = 0;
     pkd->grav.built = 0;
     // pkdDrift asserts that every particle ends inside the box (pkd.c:3760)
-    GG_CHECK(nb == 0, GG_EINVAL, "%u coordinates left the periodic box in one drift", nb);
+    GG_CHECK(nb == 0, GG_EINVAL, "%llu coordinates left the periodic box in one drift", nb);
     return GG_OK;
 }
 
@@ -464,19 +578,17 @@ extern "C" int gg_kick_vpred(GGPKD pkd, double dvFacOne, double dvFacTwo, double
     if (n == 0) return GG_OK;
     GG_TRY(need_fields(pkd, {GG_VPRED, GG_A, GG_UPRED, GG_UDOTPDV, GG_UDOTAV, GG_UDOTDIFF,
                              GG_IACTIVE}));
-    GG_TRY(pkd->red.reserve(sizeof(unsigned)));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0, sizeof(unsigned), pkd->stream));
-    hipLaunchKernelGGL(k_kick_vpred, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, dvFacOne,
+    unsigned *red;
+    unsigned long long bad = 0;
+    GG_TRY(red_begin(pkd, &red));
+    hipLaunchKernelGGL(k_kick_vpred, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n, dvFacOne,
                        dvFacTwo, duDelta, !bIsothermal, pkd->f[GG_IACTIVE].as<uint32_t>(),
                        pkd->f[GG_A].as<double>(), pkd->f[GG_UDOTPDV].as<double>(),
                        pkd->f[GG_UDOTAV].as<double>(), pkd->f[GG_UDOTDIFF].as<double>(),
-                       pkd->f[GG_VPRED].as<double>(), pkd->f[GG_UPRED].as<double>(),
-                       pkd->red.as<unsigned>());
+                       pkd->f[GG_VPRED].as<double>(), pkd->f[GG_UPRED].as<double>(), red, pkd->redHost);
     GG_HIP(hipGetLastError());
-    unsigned bad = 0;
-    GG_HIP(hipMemcpyAsync(&bad, pkd->red.p, sizeof(unsigned), hipMemcpyDeviceToHost, pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
-    GG_CHECK(bad == 0, GG_EINVAL, "gg_kick_vpred: %u gas particles with uPred < 0", bad);
+    GG_TRY(red_count(pkd, &bad, nullptr, nullptr));
+    GG_CHECK(bad == 0, GG_EINVAL, "gg_kick_vpred: %llu gas particles with uPred < 0", bad);
     return GG_OK;
 }
 
@@ -499,16 +611,15 @@ extern "C" int gg_grav_step(GGPKD pkd, double dEta)
     const int n = pkd->nLocal;
     if (n == 0) return GG_OK;
     GG_TRY(need_fields(pkd, {GG_DT, GG_DTGRAV, GG_IACTIVE}));
-    GG_TRY(pkd->red.reserve(sizeof(unsigned)));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0, sizeof(unsigned), pkd->stream));
-    hipLaunchKernelGGL(k_grav_step, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, dEta,
+    unsigned *red;
+    unsigned long long bad = 0;
+    GG_TRY(red_begin(pkd, &red));
+    hipLaunchKernelGGL(k_grav_step, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n, dEta,
                        pkd->f[GG_IACTIVE].as<uint32_t>(), pkd->f[GG_DTGRAV].as<double>(),
-                       pkd->f[GG_DT].as<double>(), pkd->red.as<unsigned>());
+                       pkd->f[GG_DT].as<double>(), red, pkd->redHost);
     GG_HIP(hipGetLastError());
-    unsigned bad = 0;
-    GG_HIP(hipMemcpyAsync(&bad, pkd->red.p, sizeof(unsigned), hipMemcpyDeviceToHost, pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
-    GG_CHECK(bad == 0, GG_EINVAL, "gg_grav_step: %u active particles with dtGrav <= 0", bad);
+    GG_TRY(red_count(pkd, &bad, nullptr, nullptr));
+    GG_CHECK(bad == 0, GG_EINVAL, "gg_grav_step: %llu active particles with dtGrav <= 0", bad);
     return GG_OK;
 }
 
@@ -557,8 +668,8 @@ extern "C" int gg_sph_step(GGPKD pkd, double dCosmoFac, double dEtaCourant, doub
     if (n == 0) return GG_OK;
     GG_TRY(need_fields(pkd, {GG_DT, GG_DTNEW, GG_FBALL2, GG_C, GG_U, GG_UDOTPDV, GG_UDOTAV,
                              GG_UDOTDIFF, GG_DENSITY, GG_DIFF, GG_IACTIVE}));
-    GG_TRY(pkd->red.reserve(sizeof(unsigned long long)));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0xff, sizeof(unsigned long long), pkd->stream));
+    unsigned *red, w[2];
+    GG_TRY(red_begin(pkd, &red));
     SphStepArgs A;
     A.n = n;
     A.dtFacCourant = dEtaCourant * dCosmoFac * 2 / 1.6;   // pkdDtFacCourant, pkd.c:5893-5895
@@ -578,12 +689,11 @@ extern "C" int gg_sph_step(GGPKD pkd, double dCosmoFac, double dEtaCourant, doub
     A.diff = pkd->f[GG_DIFF].as<double>();
     A.dtNew = pkd->f[GG_DTNEW].as<double>();
     A.dt = pkd->f[GG_DT].as<double>();
-    A.minKey = pkd->red.as<unsigned long long>();
-    hipLaunchKernelGGL(k_sph_step, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, A);
+    A.minKey = (unsigned long long *)red;
+    hipLaunchKernelGGL(k_sph_step, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, A);
     GG_HIP(hipGetLastError());
-    unsigned long long key = ~0ull;
-    GG_HIP(hipMemcpyAsync(&key, pkd->red.p, sizeof(key), hipMemcpyDeviceToHost, pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
+    GG_TRY(red_end(pkd, 2, w));
+    const unsigned long long key = ~((unsigned long long)w[1] << 32 | w[0]);
     if (key != ~0ull) {   // undo the order-preserving map
         const unsigned long long b = (key >> 63) ? (key & 0x7fffffffffffffffull) : ~key;
         std::memcpy(pdtMinGas, &b, sizeof(double));
@@ -601,25 +711,23 @@ extern "C" int gg_dt_to_rung(GGPKD pkd, int iRung, double dDelta, int iMaxRung, 
     *pnMaxRung = *piMaxRungIdeal = *piMaxRungOut = 0;
     if (n == 0) return GG_OK;
     GG_TRY(need_fields(pkd, {GG_IRUNG, GG_DT, GG_DTOLD, GG_SOFT, GG_IACTIVE}));
-    GG_TRY(pkd->red.reserve(4 * sizeof(int)));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0, 4 * sizeof(int), pkd->stream));
-    hipLaunchKernelGGL(k_dt_to_rung, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, iRung,
+    unsigned *words, red[4];
+    GG_TRY(red_begin(pkd, &words));
+    hipLaunchKernelGGL(k_dt_to_rung, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n, iRung,
                        dDelta, iMaxRung, bAll, pkd->f[GG_IACTIVE].as<uint32_t>(),
                        pkd->f[GG_SOFT].as<double>(), pkd->f[GG_DT].as<double>(),
                        pkd->f[GG_IRUNG].as<int>(), pkd->f[GG_DTOLD].as<double>(),
-                       pkd->red.as<int>());
-    hipLaunchKernelGGL(k_rung_count, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n,
-                       pkd->f[GG_IRUNG].as<int>(), pkd->red.as<int>());
+                       (int *)words);
+    hipLaunchKernelGGL(k_rung_count, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n,
+                       pkd->f[GG_IRUNG].as<int>(), (int *)words);
     GG_HIP(hipGetLastError());
-    int red[4];
-    GG_HIP(hipMemcpyAsync(red, pkd->red.p, sizeof(red), hipMemcpyDeviceToHost, pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
+    GG_TRY(red_end(pkd, 4, red));
     GG_CHECK(red[0] == 0, GG_EINVAL,
              "gg_dt_to_rung: %d particles on rung >= %d are inactive or have fSoft <= 0, dt <= 0 "
-             "or dDelta/dt >= 2.1e9 (rungs are undefined)", red[0], iRung);
-    *piMaxRungOut = red[1];
-    *pnMaxRung = red[3];
-    *piMaxRungIdeal = red[2];
+             "or dDelta/dt >= 2.1e9 (rungs are undefined)", (int)red[0], iRung);
+    *piMaxRungOut = (int)red[1];
+    *pnMaxRung = (int)red[3];
+    *piMaxRungIdeal = (int)red[2];
     return GG_OK;
 }
 
@@ -636,22 +744,25 @@ static int type_bits(GGPKD pkd, int op, int test, unsigned iFilterMask, unsigned
     if (n == 0) return GG_OK;
     if (bRung) GG_TRY(need_fields(pkd, {GG_IRUNG, GG_IACTIVE}));
     else GG_TRY(need_fields(pkd, {GG_IACTIVE}));
-    GG_TRY(pkd->red.reserve(3 * sizeof(int)));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0, 3 * sizeof(int), pkd->stream));
-    hipLaunchKernelGGL(k_type_bits, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, op, test,
+    // Counts are taken only where the caller or a tree asks for them.
+    const int cnt = pn || (iSetMask & (GG_TYPE_ACTIVE | GG_TYPE_GAS));
+    unsigned *red = nullptr;
+    unsigned long long c = 0;
+    int dAct = 0, dGas = 0;
+    if (cnt) GG_TRY(red_begin(pkd, &red));
+    hipLaunchKernelGGL(k_type_bits, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n, op, test,
                        (uint32_t)iFilterMask, (uint32_t)iTestMask, (uint32_t)iSetMask, bRung,
                        iRung, bGreater, bRung ? pkd->f[GG_IRUNG].as<int>() : (const int *)nullptr,
-                       pkd->f[GG_IACTIVE].as<uint32_t>(), pkd->red.as<int>());
+                       pkd->f[GG_IACTIVE].as<uint32_t>(), red, pkd->redHost);
     GG_HIP(hipGetLastError());
-    int c[3] = {0, 0, 0};
-    GG_HIP(hipMemcpyAsync(c, pkd->red.p, sizeof(c), hipMemcpyDeviceToHost, pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
-    if (c[1]) pkd->grav.built = 0;
-    if (c[2]) {
+    if (cnt) GG_TRY(red_count(pkd, &c, &dAct, &dGas));
+    else GG_HIP(hipStreamSynchronize(pkd->stream));
+    if (dAct) pkd->grav.built = 0;
+    if (dGas) {
         pkd->sph.gasMaskValid = 0;
         pkd->sph.built = 0;
     }
-    if (pn) *pn = c[0];
+    if (pn) *pn = (int)c;
     return GG_OK;
 }
 
@@ -668,22 +779,20 @@ extern "C" int gg_emergency_adjust(GGPKD pkd, int iRung, int iMaxRung, double dD
     if (n == 0) return GG_OK;
     GG_TRY(need_fields(pkd, {GG_IRUNG, GG_DT, GG_DTNEW, GG_V, GG_VPRED, GG_IACTIVE}));
     const int nred = 3 + iMaxRung;
-    GG_TRY(pkd->red.reserve(sizeof(int) * nred));
-    GG_HIP(hipMemsetAsync(pkd->red.p, 0, sizeof(int) * nred, pkd->stream));
+    static_assert(3 + 60 <= NRED, "one word per rung");
+    unsigned *words, red[NRED];
+    GG_TRY(red_begin(pkd, &words));
     hipLaunchKernelGGL(k_emergency, dim3(nblk(n, 256)), dim3(256), 0, pkd->stream, n, iRung,
                        iMaxRung, dDelta, dDeltaThresh, pkd->f[GG_IACTIVE].as<uint32_t>(),
                        pkd->f[GG_DTNEW].as<double>(), pkd->f[GG_DT].as<double>(),
                        pkd->f[GG_IRUNG].as<int>(), pkd->f[GG_VPRED].as<double>(),
-                       pkd->f[GG_V].as<double>(), pkd->red.as<int>());
+                       pkd->f[GG_V].as<double>(), (int *)words);
     GG_HIP(hipGetLastError());
-    std::vector<int> red(nred);
-    GG_HIP(hipMemcpyAsync(red.data(), pkd->red.p, sizeof(int) * nred, hipMemcpyDeviceToHost,
-                          pkd->stream));
-    GG_HIP(hipStreamSynchronize(pkd->stream));
-    *pnUn = red[0];
-    *piMaxRungOut = red[1];
-    *piMaxRungIdeal = red[2];
-    *pnMaxRung = red[0] ? red[3 + red[1]] : 0;
+    GG_TRY(red_end(pkd, nred, red));
+    *pnUn = (int)red[0];
+    *piMaxRungOut = (int)red[1];
+    *piMaxRungIdeal = (int)red[2];
+    *pnMaxRung = red[0] ? (int)red[3 + red[1]] : 0;
     return GG_OK;
 }
 
