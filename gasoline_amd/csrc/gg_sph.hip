@@ -630,6 +630,10 @@ __device__ int wave_bfs(const QArgs &A, Test test, int *fr, int FC, int *bf, int
 }
 
 constexpr int QB = 512;   // buckets per single-query search
+// The error words, and behind them the kNN's search counters (distances,
+// 64 bits; passes; largest group) in NSTAT copies a cache line apart:
+// wavefronts adding to one line queue up at about 10 ns each.
+constexpr int ERRW = 16, NSTAT = 64;
 
 // LDS of a single-query search.
 struct QLds {
@@ -794,6 +798,21 @@ __global__ __launch_bounds__(64) void k_query(QArgs A)
     const int lane = threadIdx.x;
     if (A.nq) {
         const int nq = (int)*A.nq;
+        if (blockIdx.x == 0) {     // the search counters of k_knn_bucket into the error words
+            const unsigned *st = A.err + ERRW + lane * 16;
+            unsigned long long c = *reinterpret_cast<const unsigned long long *>(st);
+            unsigned np = st[2], mx = st[3];
+            for (int o = 32; o > 0; o >>= 1) {
+                c += __shfl_xor(c, o);
+                np += __shfl_xor(np, o);
+                mx = max(mx, (unsigned)__shfl_xor(mx, o));
+            }
+            if (lane == 0) {
+                A.err[5] = mx;
+                A.err[6] = np;
+                *reinterpret_cast<unsigned long long *>(A.err + 8) = c;
+            }
+        }
         for (int b = blockIdx.x; b < nq; b += gridDim.x) {
             query_one(A, A.qlist[b], S, lane);
             wave_sync();
@@ -805,7 +824,7 @@ __global__ __launch_bounds__(64) void k_query(QArgs A)
 
 // ---------------------------------------------- kNN by bucket groups
 // Group of a bucket: every bucket within a group radius RL of the bucket's
-// box.  k_knn_bucket, one wavefront per bucket, finds the group (a
+// box.  k_knn_bucket, one or more wavefronts per bucket, finds the group (a
 // breadth-first descent of the radix tree, whose waits on the child records
 // other wavefronts' selections fill) into LDS, then settles the bucket's
 // queries against it, holding the group's bucket boxes and ranges in LDS.
@@ -828,12 +847,27 @@ constexpr int KL_FC = 512;             // descent frontier per wavefront
 struct KLArgs {
     QArgs Q;
     int nb;                            // buckets
+    int lsp;                           // log2 of the wavefronts per bucket
     const int *bfirst, *bcnt;
     int *gnb;                          // buckets in the group, -1: too large
     double *grl2;                      // group radius^2
     int *retry;
     unsigned *nretry;
 };
+
+// log2 of the wavefronts that share a bucket's queries (each takes every
+// 2^lsp-th one after a group descent of its own).  A bucket's queries are a
+// serial chain of about 6 us each, so few buckets leave the chip idle (its
+// 1024 SIMDs hold 3 of these wavefronts each) for as long as one bucket takes;
+// on a large store the extra descents only cost.  Measured (us, 1 / 2 / 4 / 8
+// / 16 wavefronts per bucket, K 32): 185 buckets 191 / 108 / 61 / 41 / 31,
+// 530: 187 / 107 / 67 / 69 / 71, 1059: 208 / 127 / 117 / 106 / 131, 2109: 228 /
+// 195 / 172 / 189 / 252, 6577: 439 / 398 / 428 / 518 / 718, 14352: 812 / 790 /
+// 900, 22083: 1193 / 1215 / 1394.
+static int knn_split(int nb)
+{
+    return nb > 16384 ? 0 : nb > 4096 ? 1 : nb > 1536 ? 2 : nb > 384 ? 3 : 4;
+}
 
 // Squared gap between two boxes, minimised over periodic images of a.
 __device__ __forceinline__ double boxbox_d2(const double *a, const double *b, int per,
@@ -1146,7 +1180,7 @@ __device__ __forceinline__ double readlane_d(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// One wavefront per bucket.
+// 2^lsp wavefronts per bucket (knn_split).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_knn_bucket(KLArgs KA)
 {
     const QArgs &A = KA.Q;
@@ -1161,9 +1195,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     double *bd = reinterpret_cast<double *>(ubuf + KL_SB * 8);
     int *bs = reinterpret_cast<int *>(ubuf + KL_SB * 8 + CAP * 8);
     const int lane = threadIdx.x;
-    const int g = xcd_block(blockIdx.x, gridDim.x);
+    const int gp = xcd_block(blockIdx.x, gridDim.x);
+    const int g = gp >> KA.lsp, part = gp & ((1 << KA.lsp) - 1);
     const int s0 = KA.bfirst[g], nq = KA.bcnt[g];
     const int K = A.K;
+    // this wavefront's queries of the bucket; without any the group is not
+    // needed
+    const bool isq = lane < nq && A.qflag[s0 + lane] != 0;
+    const bool mine = isq && (lane & ((1 << KA.lsp) - 1)) == part;
+    if (!__ballot(mine)) return;
+    const bool first = __ffsll((long long)__ballot(isq)) == __ffsll((long long)__ballot(mine));
+    unsigned *stat = A.err + ERRW + (gp & (NSTAT - 1)) * 16;
     // the group radius: from the queries' fBall2 hints, else the bucket's
     // density estimate
     double qg = 0, RL2;
@@ -1192,14 +1234,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         if (lane == 0) {   // for the retries
             KA.gnb[g] = nbg;
             KA.grl2[g] = R2;
-            if (nbg >= 0) atomicMax(&A.err[5], (unsigned)nbg);
+            if (nbg >= 0) atomicMax(stat + 3, (unsigned)nbg);
         }
         nb = nbg;
         RL2 = R2;
     }
     if (nb < 0) {          // group too large: every query retries
-        if (lane == 0) atomicAdd(&A.err[2], 1u);
-        if (lane < nq && A.qflag[s0 + lane]) {
+        if (lane == 0 && first) atomicAdd(&A.err[2], 1u);
+        if (mine) {
             const unsigned p = atomicAdd(KA.nretry, 1u);
             KA.retry[p] = s0 + lane;
         }
@@ -1207,12 +1249,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     }
     // the bucket's queries, one per lane, broadcast as each is served
     double qx = 0, qy = 0, qz = 0;
-    int qf = 0;
-    if (lane < nq) {
+    if (mine) {
         qx = A.sx[s0 + lane];
         qy = A.sy[s0 + lane];
         qz = A.sz[s0 + lane];
-        qf = A.qflag[s0 + lane] != 0;
     }
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (int k = lane; k < nb; k += 64) {
@@ -1250,9 +1290,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     G.lcnt = lcnt;
     G.nb = nb;
     unsigned npass = 0, ncand = 0;     // search work: passes (uniform), distances (per lane)
-    for (int j = 0; j < nq; ++j) {
-        if (!__builtin_amdgcn_readlane(qf, j)) continue;
-        const int q = s0 + j;
+    for (unsigned long long todo = __ballot(mine); todo; todo &= todo - 1) {
+        const int j = __ffsll((long long)todo) - 1, q = s0 + j;
         const double x = readlane_d(qx, j), y = readlane_d(qy, j), z = readlane_d(qz, j),
                      gq = readlane_d(qg, j);
         // first ball: slack * fBall2 from the hint, else 0.8 RL^2 (~1.6K expected)
@@ -1268,8 +1307,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     }
     for (int o = 32; o > 0; o >>= 1) ncand += __shfl_xor(ncand, o);
     if (lane == 0) {
-        if (npass) atomicAdd(&A.err[6], npass);
-        atomicAdd(reinterpret_cast<unsigned long long *>(A.err + 8), (unsigned long long)ncand);
+        if (npass) atomicAdd(stat + 2, npass);
+        atomicAdd(reinterpret_cast<unsigned long long *>(stat), (unsigned long long)ncand);
     }
 }
 
@@ -2621,8 +2660,8 @@ extern "C" int gg_smooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPeriodi
     GG_TRY(make_flags(pkd, GG_TYPE_SMOOTHACTIVE));
     GG_TRY(S.nbr.reserve(sizeof(int) * (size_t)K * n));
     GG_TRY(S.fb2s.reserve(sizeof(double) * n));
-    GG_TRY(S.err.reserve(sizeof(unsigned) * 12));
-    GG_HIP(hipMemsetAsync(S.err.p, 0, sizeof(unsigned) * 12, st));
+    GG_TRY(S.err.reserve(sizeof(unsigned) * (ERRW + 16 * NSTAT)));
+    GG_HIP(hipMemsetAsync(S.err.p, 0, sizeof(unsigned) * (ERRW + 16 * NSTAT), st));
     const bool hint = S.seedSlack > 0.0;
     if (hint) GG_TRY(gather_field(pkd, GG_FBALL2, 1, 0, S.guess));
     GG_TRY(S.retry.reserve(sizeof(int) * n));
@@ -2631,6 +2670,7 @@ extern "C" int gg_smooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPeriodi
     KL.Q.guess = hint ? S.guess.as<double>() : nullptr;
     KL.Q.nbr = S.nbr.as<int>();
     KL.nb = S.nb;
+    KL.lsp = knn_split(S.nb);
     KL.bfirst = S.bfirst.as<int>();
     KL.bcnt = S.bcnt.as<int>();
     GG_TRY(S.grpn.reserve(sizeof(int) * S.nb));
@@ -2641,7 +2681,7 @@ extern "C" int gg_smooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPeriodi
     KL.nretry = S.err.as<unsigned>() + 10;   // err[10]: retries (zeroed above)
     timer_mark(pkd, 0);
     timer_mark(pkd, 1);   // the group lists are found inside k_knn_bucket
-    hipLaunchKernelGGL(k_knn_bucket, dim3(S.nb), dim3(64), 0, st, KL);
+    hipLaunchKernelGGL(k_knn_bucket, dim3(S.nb << KL.lsp), dim3(64), 0, st, KL);
     timer_mark(pkd, 2);
     GG_HIP(hipGetLastError());
     {   // queries the leaf groups could not settle; their number stays on the device
