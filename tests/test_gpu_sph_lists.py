@@ -1,14 +1,17 @@
 """The SPH lists where their kernels change course: the wavefronts that share
 a bucket's queries in the kNN (by the number of buckets, with all or few of
-the particles searching).
+the particles searching), and the extras lists' sorting networks (short, long
+and beyond them).
 
 Bars: neighbour sets equal a k-d tree's (random positions: no ties) and
 fBall2 to 4 ulp (the tree forms the distance in another order); forces FP64
-within 1e-12 of the oracle's or of the gathered balls' (sums in another
-order); a repeated call bit for bit."""
+within 1e-12 of the oracle's; a repeated call bit for bit."""
 import numpy as np
 import pytest
 from scipy.spatial import cKDTree
+
+from gasoline_amd import ics
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -18,6 +21,10 @@ def put_gas(pk, d):
     pk.put("fMass", d["m"])
     pk.put("vPred", d["v"])
     pk.put("uPred", d["u"])
+
+
+def scaled(a, b):
+    return np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300)
 
 
 @pytest.mark.parametrize("part", [1.0, 0.05])
@@ -38,3 +45,47 @@ def test_knn_wavefronts_per_bucket(gpu, n, part):
     d, j = cKDTree(r).query(r[on], k=K)
     assert np.array_equal(np.sort(nbr[on], axis=1), np.sort(j, axis=1))
     assert np.allclose(fb2[on], d[:, -1] ** 2, rtol=4 * 2.3e-16, atol=0)
+
+
+def clump(nc, nh, seed):
+    """A clump inside a thin halo: the halo's balls reach into the clump,
+    whose own balls do not reach out."""
+    rng = np.random.default_rng(seed)
+    h = rng.normal(size=(nh, 3))
+    h *= (rng.uniform(0.9, 1.1, nh) / np.linalg.norm(h, axis=1))[:, None]
+    r = np.concatenate([rng.normal(0, 0.02, (nc, 3)), h])
+    n = nc + nh
+    return dict(r=r, m=np.full(n, 1.0 / n), v=rng.normal(0, 0.1, (n, 3)),
+                u=rng.uniform(0.5, 1.0, n))
+
+
+def extras(d, fb2):
+    dist2 = ((d["r"][:, None] - d["r"][None]) ** 2).sum(2)
+    return ((dist2 <= fb2[:, None]) & ~(dist2.T <= fb2[None, :])).sum(0)
+
+
+@pytest.mark.parametrize("K,nc,nh,lo,hi", [(16, 30, 80, 2, 16), (40, 30, 40, 17, 32),
+                                           (40, 60, 40, 33, 48), (40, 110, 40, 49, 64),
+                                           (64, 60, 200, 65, 400)])
+def test_extras_sorted(gpu, K, nc, nh, lo, hi):
+    d = clump(nc, nh, 3)
+    nbr, fb2, ties = O.knn(d["r"], K)
+    assert ties == 0
+    assert lo <= extras(d, fb2).max() <= hi
+    smf = O.default_smf()
+    lists = O.ball_gather(d["r"], fb2)
+    den = O.dendvdx(d["m"], d["v"], d["u"], fb2, lists, smf)
+    pr2, c, dt = O.gas_pressure(d["u"], den["rho"], fb2, smf)
+    hyd = O.sph_pressure_sym(d["m"], d["v"], d["u"], den["rho"], pr2, c, den["balsara"],
+                             den["diff"], dt, fb2, lists, smf)
+    out = []
+    for _ in range(2):
+        with gpu.Pkd(len(d["m"]), prec=gpu.PREC_FP64) as pk:
+            put_gas(pk, d)
+            pk.build_local()
+            pk.smooth(gpu.Smf.default(), K, False)
+            pk.gas_pressure(gpu.Smf.default())
+            pk.resmooth(gpu.Smf.default(), K, False)
+            out.append(pk.get("a"))
+    assert scaled(out[0], hyd["acc"]) < 1e-12
+    assert np.array_equal(out[0], out[1])
