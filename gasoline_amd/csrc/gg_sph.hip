@@ -2068,13 +2068,17 @@ __global__ void k_gather_comp(int n, const int *__restrict__ order, const double
     dst[s] = src[(size_t)width * order[s] + comp];
 }
 
-__global__ void k_count_diff(int n, const double *__restrict__ a, const double *__restrict__ b,
-                             const uint32_t *__restrict__ qa, const uint32_t *__restrict__ qb,
-                             unsigned *__restrict__ out)
+// Which kNN lists (flags qb, radii b) serve the queries qa with radii a:
+// out[0] is set when some query has no list of its radius, out[1] when some
+// list belongs to no query.
+__global__ void k_list_diff(int n, const double *__restrict__ a, const double *__restrict__ b,
+                            const uint32_t *__restrict__ qa, const uint32_t *__restrict__ qb,
+                            unsigned *__restrict__ out)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    if (qa[s] != qb[s] || (qa[s] && a[s] != b[s])) atomicAdd(out, 1u);
+    if (qa[s] && (!qb[s] || a[s] != b[s])) out[0] = 1u;   // every writer stores the same flag
+    if (!qa[s] && qb[s]) out[1] = 1u;
 }
 
 template <typename T>
@@ -2911,16 +2915,21 @@ extern "C" int gg_resmooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPerio
     GG_TRY(gather_field(pkd, GG_FBALL2, 1, 0, S.fb2s));
     GG_TRY(S.err.reserve(sizeof(unsigned) * 12));
     GG_HIP(hipMemsetAsync(S.err.p, 0, sizeof(unsigned) * 12, st));
-    // reuse the kNN lists when they are exactly the ball lists of the
-    // stored radii (same queries, same fBall2, no boundary ties)
-    bool reuse = false;
+    // reuse the kNN lists when each query has one that is exactly its ball
+    // (same fBall2, no boundary ties): the queries may be fewer than the kNN's,
+    // as in a block step, which smooths all the gas and re-smooths the
+    // neighbours of the active particles.  Gathering the balls again took
+    // 200 us of a 16k-particle re-smooth (two passes of one wavefront per slot
+    // and the host's wait for their total).  Only equal query sets (exact)
+    // have the extras the density pass found.
+    bool reuse = false, exact = false;
     if (S.listValid) {
-        GG_TRY(S.diffcnt.reserve(sizeof(unsigned)));
-        GG_HIP(hipMemsetAsync(S.diffcnt.p, 0, sizeof(unsigned), st));
-        hipLaunchKernelGGL(k_count_diff, dim3(nblk(n, 256)), dim3(256), 0, st, n,
+        GG_TRY(S.diffcnt.reserve(2 * sizeof(unsigned)));
+        GG_HIP(hipMemsetAsync(S.diffcnt.p, 0, 2 * sizeof(unsigned), st));
+        hipLaunchKernelGGL(k_list_diff, dim3(nblk(n, 256)), dim3(256), 0, st, n,
                            S.fb2s.as<double>(), S.fb2knn.as<double>(), S.qf.as<uint32_t>(),
                            S.qfknn.as<uint32_t>(), S.diffcnt.as<unsigned>());
-        GG_TRY(rb_queue(pkd, S.diffcnt.p, 1, 0));
+        GG_TRY(rb_queue(pkd, S.diffcnt.p, 2, 0));
     }
     timer_mark(pkd, 1);
     // the force pass's per-particle records in slot order (they do not depend
@@ -2949,7 +2958,8 @@ extern "C" int gg_resmooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPerio
     timer_mark(pkd, 2);
     if (S.listValid) {
         GG_TRY(rb_wait(pkd));
-        reuse = (S.rb[0] == 0);
+        reuse = S.rb[0] == 0;
+        exact = reuse && S.rb[1] == 0;
     }
     const int64_t *off;
     const int *idx;
@@ -2987,12 +2997,12 @@ extern "C" int gg_resmooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPerio
         timer_mark(pkd, 5);
         GG_TRY(rb_wait(pkd));
         // the extras belong to the kNN lists only when those were the lists
-        S.exValid = reuse && S.rb[7] == 0;
+        S.exValid = exact && S.rb[7] == 0;
         const int ph[5] = {5, 8, 5, 4, 8};
         timer_collect(pkd, 0, 5, ph);
         return GG_OK;
     }
-    const bool fixedExtras = reuse && S.exValid;
+    const bool fixedExtras = exact && S.exValid;
     if (fixedExtras) {   // the density pass found them: sort each list
         GG_TRY(S.nxd.reserve(sizeof(int64_t) * nblk(n, 256)));
         hipLaunchKernelGGL(k_rev_sort_fixed, dim3(nblk(n, 256)), dim3(256), 0, st, n, ECAP,

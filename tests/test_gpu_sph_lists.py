@@ -1,11 +1,13 @@
 """The SPH lists where their kernels change course: the wavefronts that share
 a bucket's queries in the kNN (by the number of buckets, with all or few of
-the particles searching), and the extras lists' sorting networks (short, long
-and beyond them).
+the particles searching), the extras lists' sorting networks (short, long and
+beyond them), and the re-smooth of fewer particles than were smoothed, which
+takes the kNN's lists.
 
 Bars: neighbour sets equal a k-d tree's (random positions: no ties) and
 fBall2 to 4 ulp (the tree forms the distance in another order); forces FP64
-within 1e-12 of the oracle's; a repeated call bit for bit."""
+within 1e-12 of the oracle's or of the gathered balls' (sums in another
+order); a repeated call bit for bit."""
 import numpy as np
 import pytest
 from scipy.spatial import cKDTree
@@ -89,3 +91,33 @@ def test_extras_sorted(gpu, K, nc, nh, lo, hi):
             out.append(pk.get("a"))
     assert scaled(out[0], hyd["acc"]) < 1e-12
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n,part", [(60, 0.5), (3000, 0.02), (30000, 0.3), (30000, 0.0)])
+def test_resmooth_of_fewer_particles(gpu, n, part):
+    K = 32
+    d = ics.evrard(n, seed=6) if n > 100 else clump(30, n - 30, 5)
+    n = len(d["m"])
+    rng = np.random.default_rng(n)
+    on = rng.uniform(size=n) < part
+    smf = gpu.Smf.default()
+    out = []
+    with gpu.Pkd(n, prec=gpu.PREC_FP64) as pk:
+        put_gas(pk, d)
+        pk.put("iActive", np.where(on, 7 + 16, 7).astype(np.uint32) | gpu.TYPE_GAS)
+        pk.build_local()
+        pk.smooth(smf, K, False)
+        pk.gas_pressure(smf)
+        assert pk.smooth_stats()["ties"] == 0
+        fb2 = pk.get("fBall2")
+        assert pk.active_type(16, gpu.TYPE_SMOOTHACTIVE) == on.sum()
+        # the kNN's lists; then the balls gathered: radii an ulp larger hold the
+        # same particles
+        for f in (fb2, np.nextafter(fb2, np.inf)):
+            pk.put("fBall2", f)
+            for k, w in (("a", 3), ("uDotPdV", 1), ("mumax", 1)):
+                pk.put(k, np.zeros((n, w)) if w > 1 else np.zeros(n))
+            pk.resmooth(smf, K, False)
+            out.append([pk.get(k) for k in ("a", "uDotPdV", "mumax")])
+    for x, y in zip(*out):
+        assert (not y.any() and not x.any()) if not on.any() else scaled(x, y) < 1e-12
