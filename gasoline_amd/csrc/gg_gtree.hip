@@ -93,11 +93,16 @@ __device__ __forceinline__ double ord_val(unsigned long long k)
     return __longlong_as_double(b < 0 ? (b & 0x7fffffffffffffffll) : ~b);
 }
 
+// A cell's bounds while its particles are still being scanned: six keys, each
+// in a 128-byte line of its own.  Every tile of a cell adds to its six, and
+// atomics on one line are served one after another: side by side they made
+// k_gt_swap take 53 us on the root of 2^21 particles, 35 in lines of their own.
+constexpr int BOX_S = 16, BOX_N = 6 * BOX_S;
 __device__ __forceinline__ void box_init(unsigned long long *b)
 {
     for (int d = 0; d < 3; ++d) {
-        b[d] = ~0ull;
-        b[3 + d] = 0ull;
+        b[BOX_S * d] = ~0ull;
+        b[BOX_S * (3 + d)] = 0ull;
     }
 }
 
@@ -135,7 +140,7 @@ __global__ void k_gt_roots(int n, int nr, const int *__restrict__ rlo,
     g.ch0 = g.ch1 = -1;
     g.dim = -1;
     g.split = 0.0;
-    box_init(box + 6 * (size_t)k);
+    box_init(box + BOX_N * (size_t)k);
     unit[k] = k;
 }
 
@@ -199,11 +204,11 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
                 hi[d] = v[d] > hi[d] ? v[d] : hi[d];
             }
         } else {
-            unsigned long long *b = box + 6 * (size_t)root_of(i, nr, rlo);
+            unsigned long long *b = box + BOX_N * (size_t)root_of(i, nr, rlo);
             for (int d = 0; d < 3; ++d) {
                 if (v[d] != v[d]) continue;
-                atomicMin(b + d, ord_key(v[d]));
-                atomicMax(b + 3 + d, ord_key(v[d]));
+                atomicMin(b + BOX_S * d, ord_key(v[d]));
+                atomicMax(b + BOX_S * (3 + d), ord_key(v[d]));
             }
         }
     }
@@ -214,9 +219,9 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
     }
     if (r0 != r1) return;
     const unsigned long long k = block_box(lo, hi, sm);
-    unsigned long long *b = box + 6 * (size_t)r0;
-    if (threadIdx.x < 3) atomicMin(b + threadIdx.x, k);
-    else if (threadIdx.x < 6) atomicMax(b + threadIdx.x, k);
+    unsigned long long *b = box + BOX_N * (size_t)r0 + BOX_S * threadIdx.x;
+    if (threadIdx.x < 3) atomicMin(b, k);
+    else if (threadIdx.x < 6) atomicMax(b, k);
 }
 
 // The host's copy of a device word (pinned memory, -1 until written).
@@ -265,11 +270,11 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
             } else if (cnt <= MID) {
                 un = 1;
             } else {
-                const unsigned long long *k = box + 6 * (size_t)(c - a);
+                const unsigned long long *k = box + BOX_N * (size_t)(c - a);
                 double bmin[3], bmax[3];
                 for (int d = 0; d < 3; ++d) {
-                    bmin[d] = ord_val(k[d]);
-                    bmax[d] = ord_val(k[3 + d]);
+                    bmin[d] = ord_val(k[BOX_S * d]);
+                    bmax[d] = ord_val(k[BOX_S * (3 + d)]);
                 }
                 bool extent = false;
                 for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
@@ -331,7 +336,7 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
                 h.ch0 = h.ch1 = -1;
                 h.dim = -1;
                 h.split = 0.0;
-                box_init(kbox + 6 * (size_t)(kid + q));
+                box_init(kbox + BOX_N * (size_t)(kid + q));
             }
         }
         if (un) unit[nunit0 + nun + pu + iu - 1] = c;
@@ -497,7 +502,7 @@ template <int MODE> __global__ __launch_bounds__(256) void k_gt_rank(TileArgs A)
 // upper particle (counted up from lo) <-> posR[lo + k], each pair swapped
 // by its lower member.  Every particle passes through registers once, so
 // the children's bounds are taken on the way (mode 0).  It moves 24-28 bytes
-// a particle and 56 a swapped one.  Measured per level: 31 us on a 2^21
+// a particle and 56 a swapped one.  Measured per level: 25 us on a 2^21
 // Plummer sphere (count 6.3, rank 4.6, control 5.9) and 14 us on 3 10^5
 // particles (4.3, 3.9, 5.4), where the chain of loads and the bounds'
 // reduction bound it rather than the bytes.
@@ -512,7 +517,9 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
     const int4 T = A.tiles[t];
     tile_flags(A, t, A.tpre[t], fw, fp);
     const GNode &g = A.nd[T.x];
-    const int hi = g.hi, s = g.s, ch0 = g.ch0;
+    const int lo = g.lo, hi = g.hi, s = g.s, ch0 = g.ch0;
+    // a child that goes to k_gt_mid takes its bounds there
+    const bool need[2] = {MODE == 0 && s - lo > MID, MODE == 0 && hi - s + 1 > MID};
     const int last = min(hi, T.y + A.ts - 1);
     double bl[2][3], bh[2][3];
     for (int q = 0; q < 2; ++q)
@@ -554,13 +561,14 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
             else grow(1, v);
         }
     }
-    if (MODE == 1) return;
+    if (!need[0] && !need[1]) return;
     const int kid = ch0 - A.L->a;        // the children's level starts at L->a now
     for (int q = 0; q < 2; ++q) {
+        if (!need[q]) continue;
         const unsigned long long k = block_box(bl[q], bh[q], sm[q]);
-        unsigned long long *b = kbox + 6 * (size_t)(kid + q);
-        if (threadIdx.x < 3) atomicMin(b + threadIdx.x, k);
-        else if (threadIdx.x < 6) atomicMax(b + threadIdx.x, k);
+        unsigned long long *b = kbox + BOX_N * (size_t)(kid + q) + BOX_S * threadIdx.x;
+        if (threadIdx.x < 3) atomicMin(b, k);
+        else if (threadIdx.x < 6) atomicMax(b, k);
     }
 }
 
@@ -1739,7 +1747,7 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     GG_TRY(G.gnode.reserve(sizeof(GNode) * (size_t)cap));
     GG_TRY(G.gm.reserve(sizeof(double) * gm_stride(order) * (size_t)cap));
     GG_TRY(G.gbb8.reserve(sizeof(double) * 8 * (size_t)cap));
-    GG_TRY(G.gbox.reserve(sizeof(unsigned long long) * 12 * mbox));
+    GG_TRY(G.gbox.reserve(sizeof(unsigned long long) * 2 * BOX_N * mbox));
     GG_TRY(G.gtile.reserve(sizeof(int4) * mtile));
     GG_TRY(G.gflag.reserve(sizeof(unsigned long long) * mtile * (ts / 64)));
     GG_TRY(G.gtcnt.reserve(sizeof(int) * 2 * mtile));
@@ -1781,7 +1789,7 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     const int *rl = G.groot.as<int>(), *rh = rl + nr;
     unsigned long long *box[2];
     box[0] = G.gbox.as<unsigned long long>();
-    box[1] = box[0] + 6 * mbox;
+    box[1] = box[0] + BOX_N * mbox;
     volatile int *hv = G.hst;
     for (int k = 0; k < 16; ++k) hv[k] = -1;
     if (nr > 1)   // (a single root is the whole store)
