@@ -47,7 +47,7 @@ struct GNode {
     int ch0, ch1, dim, s;        // children (-1), split axis (-1: bucket), split position
     int size, nab;               // cells and buckets with active particles of the subtree
     int pre, bpre;               // preorder id and bucket rank (within the subtree of
-                                 // k_gt_sub; absolute for a root)
+                                 // k_gt_sub; absolute for the cells of the level loop)
     int sizeLo, nabLo;           // the lower child's, above LMAX
     double split;
 };
@@ -1393,26 +1393,33 @@ template <int ORDER> __global__ __launch_bounds__(64) void k_gt_up_unit(TreeArgs
     }
 }
 
-// The splitting cells of one level above MID.
-template <int ORDER> __global__ __launch_bounds__(256) void k_gt_up_level(TreeArgs A, int depth)
+// One workgroup: the splitting cells of the levels above MID from the deepest
+// up, then the roots' preorder ids and first bucket ranks, then those of the
+// level's children downwards; to the host the cells, active buckets, largest
+// bucket and error word.  A level holds at most 2 n / MID cells, usually a
+// few, so what it costs is one record's chain of loads: about 2 us between
+// barriers against 4.7 us for a launch of its own (18 of them on a galaxy of
+// 50k particles, 26 on 2^21).
+constexpr int TOP_T = 512;
+template <int ORDER>
+__global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs A, int *host)
 {
-    if (A.L->err & 2) return;
-    const int c = A.L->lv[depth] + ((blockIdx.x * 256 + threadIdx.x) >> 1);
-    if (c >= A.L->lv[depth + 1]) return;
-    const GNode &g = A.nd[c];
-    if (g.hi - g.lo < MID || g.dim < 0) return;          // a unit
-    upper_record<ORDER>(A, c, threadIdx.x & 1);
-}
-
-// One workgroup: the roots' preorder ids and first bucket ranks, and to the
-// host the cells, active buckets, largest bucket and error word.
-__global__ __launch_bounds__(256) void k_gt_totals(int nr, TreeArgs A, int *host)
-{
-    __shared__ int2 ws[4];
+    __shared__ int2 ws[TOP_T / 64];
     int2 run = make_int2(0, 0);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int b = 0; b < nr; b += 256) {
-        const int k = b + threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lev = A.L->err & 2 ? 0 : nlev;
+    auto splits = [&](int c) {                           // (the others are units)
+        const GNode &g = A.nd[c];
+        return g.hi - g.lo >= MID && g.dim >= 0;
+    };
+    for (int d = lev - 1; d >= 0; --d) {
+        const int c1 = A.L->lv[d + 1];
+        for (int c = A.L->lv[d] + (tid >> 1); c < c1; c += TOP_T / 2)
+            if (splits(c)) upper_record<ORDER>(A, c, tid & 1);
+        __syncthreads();
+    }
+    for (int b = 0; b < nr; b += TOP_T) {
+        const int k = b + tid;
         const int sz = k < nr ? A.nd[k].size : 0, na = k < nr ? A.nd[k].nab : 0;
         int is = sz, ia = na;
         for (int o = 1; o < 64; o <<= 1) {
@@ -1425,7 +1432,7 @@ __global__ __launch_bounds__(256) void k_gt_totals(int nr, TreeArgs A, int *host
         if (lane == 63) ws[w] = make_int2(is, ia);
         __syncthreads();
         int ps = run.x + is - sz, pa = run.y + ia - na;
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < TOP_T / 64; ++q) {
             if (q < w) {
                 ps += ws[q].x;
                 pa += ws[q].y;
@@ -1439,7 +1446,7 @@ __global__ __launch_bounds__(256) void k_gt_totals(int nr, TreeArgs A, int *host
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         tell_host(host + 1, run.x);
         tell_host(host + 2, run.y);
         tell_host(host + 3, A.L->maxb);
@@ -1447,65 +1454,92 @@ __global__ __launch_bounds__(256) void k_gt_totals(int nr, TreeArgs A, int *host
         tell_host(host + 5, A.L->nsub);
         tell_host(host, A.L->err);
     }
+    for (int d = 0; d < lev; ++d) {
+        const int c1 = A.L->lv[d + 1];
+        for (int c = A.L->lv[d] + tid; c < c1; c += TOP_T) {
+            if (!splits(c)) continue;
+            const GNode &g = A.nd[c];
+            GNode &l = A.nd[g.ch0], &u = A.nd[g.ch1];
+            l.pre = g.pre + 1;
+            l.bpre = g.bpre;
+            u.pre = g.pre + 1 + g.sizeLo;
+            u.bpre = g.bpre + g.nabLo;
+        }
+        __syncthreads();
+    }
 }
 
-// Largest squared distances of the cells above LMAX: per unit, the cells
-// k_gt_mid closed (a wavefront each), then the unit's particles against
-// every cell above it, combined in LDS and then by one atomic a cell.
-constexpr int BM_A = 512;        // ancestors combined at a time
-template <int ORDER> __global__ __launch_bounds__(256) void k_gt_up_bmax(TreeArgs A)
+// Largest squared distances of the cells above LMAX: per unit, those of the
+// cells k_gt_mid closed, and the unit's particles against every cell above
+// it, by one atomic a cell.  The workgroup holds the unit's particles in
+// registers, four a thread, 256 in a row to a wavefront, and takes the cells
+// from a list in LDS; a wavefront passes over cells it has no particle of.
+// With a wavefront to each closed cell its latest loads were waited for one
+// after another: 43 us for 4096 particles, 66 us with 18 cells above a unit;
+// 18 and 28 us this way.
+constexpr int BM_T = 1024, BM_E = 4, BM_A = 256;         // BM_A: cells of the list
+template <int ORDER> __global__ __launch_bounds__(BM_T) void k_gt_up_bmax(TreeArgs A)
 {
     constexpr int GS = gm_stride(ORDER);
     __shared__ unsigned long long bm[BM_A];
-    __shared__ int an[BM_A];
-    __shared__ int na_sh, next_sh;
+    __shared__ double cx[BM_A], cy[BM_A], cz[BM_A];
+    __shared__ int cell[BM_A], first[BM_A], last[BM_A];
+    __shared__ int na_sh, up_sh;
     if (A.L->err & 2) return;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int root = A.unit[blockIdx.x];
     const int lo = A.nd[root].lo, hi = A.nd[root].hi;
-    const int2 u = A.useg[blockIdx.x];
-    for (int e = w; e < u.x; e += 4) {
-        const int c = A.seg[lo + e];
-        const int c0 = A.nd[c].lo, c1 = A.nd[c].hi;
-        double *o = A.gm + (size_t)GS * c;
-        if (A.nd[c].dim < 0) continue;
-        const double cm[3] = {o[2], o[3], o[4]};
-        double b2 = 0.0;
-        for (int i = c0 + lane; i <= c1; i += 64) {
-            const double d2 = cm_d2(A.px[i], A.py[i], A.pz[i], cm);
-            b2 = d2 > b2 ? d2 : b2;
+    const int nclosed = A.useg[blockIdx.x].x;
+    int up = A.nd[root].par;
+    for (int done = 0; done < nclosed || up >= 0;) {
+        const int nc = min(BM_A, nclosed - done);
+        if (tid < nc) {                                  // closed cells
+            const int c = A.seg[lo + done + tid];
+            const bool leaf = A.nd[c].dim < 0;           // buckets have theirs
+            cell[tid] = c;
+            first[tid] = leaf ? 1 : A.nd[c].lo;
+            last[tid] = leaf ? 0 : A.nd[c].hi;
         }
-        for (int q = 32; q > 0; q >>= 1) {
-            const double v = __shfl_xor(b2, q);
-            b2 = v > b2 ? v : b2;
-        }
-        if (lane == 0) o[GM_B] = b2;
-    }
-    for (int c = A.nd[root].par; c >= 0; c = next_sh) {
-        if (tid == 0) {
-            int k = 0;
-            for (; c >= 0 && k < BM_A; c = A.nd[c].par) an[k++] = c;
+        if (tid == BM_T - 64) {                          // cells above
+            int k = nc;
+            for (; up >= 0 && k < BM_A; up = A.nd[up].par) {
+                cell[k] = up;
+                first[k] = lo;
+                last[k++] = hi;
+            }
             na_sh = k;
-            next_sh = c;
+            up_sh = up;
         }
-        for (int k = tid; k < BM_A; k += 256) bm[k] = 0;
         __syncthreads();
         const int na = na_sh;
-        for (int b = lo; b <= hi; b += 1024) {
-            double x[4], y[4], z[4];
-            for (int q = 0; q < 4; ++q) {                // past the end: the last particle
-                const int i = min(b + 256 * q + tid, hi);
+        up = up_sh;
+        if (tid < na) {
+            const double *o = A.gm + (size_t)GS * cell[tid];
+            cx[tid] = o[2];
+            cy[tid] = o[3];
+            cz[tid] = o[4];
+            bm[tid] = 0;
+        }
+        __syncthreads();
+        for (int b = lo; b <= hi; b += BM_T * BM_E) {
+            const int wlo = b + w * 64 * BM_E, whi = min(hi, wlo + 64 * BM_E - 1);
+            if (wlo > hi) continue;
+            double x[BM_E], y[BM_E], z[BM_E];
+            for (int q = 0; q < BM_E; ++q) {
+                const int i = min(hi, wlo + 64 * q + lane);
                 x[q] = A.px[i];
                 y[q] = A.py[i];
                 z[q] = A.pz[i];
             }
             for (int k = 0; k < na; ++k) {
-                const double *o = A.gm + (size_t)GS * an[k];
-                const double cm[3] = {o[2], o[3], o[4]};
+                const int c0 = first[k], c1 = last[k];
+                if (c0 > whi || c1 < wlo) continue;
+                const double cm[3] = {cx[k], cy[k], cz[k]};
                 double b2 = 0.0;
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < BM_E; ++q) {
+                    const int i = wlo + 64 * q + lane;
                     const double d2 = cm_d2(x[q], y[q], z[q], cm);
-                    b2 = d2 > b2 ? d2 : b2;
+                    b2 = i >= c0 && i <= c1 && d2 > b2 ? d2 : b2;
                 }
                 for (int q = 32; q > 0; q >>= 1) {
                     const double v = __shfl_xor(b2, q);
@@ -1515,9 +1549,12 @@ template <int ORDER> __global__ __launch_bounds__(256) void k_gt_up_bmax(TreeArg
             }
         }
         __syncthreads();
-        for (int k = tid; k < na; k += 256)
-            atomicMax(reinterpret_cast<unsigned long long *>(A.gm + (size_t)GS * an[k] + GM_B),
-                      bm[k]);
+        if (tid < na) {
+            double *o = A.gm + (size_t)GS * cell[tid] + GM_B;
+            if (tid >= nc) atomicMax(reinterpret_cast<unsigned long long *>(o), bm[tid]);
+            else if (first[tid] <= last[tid]) *o = __longlong_as_double((long long)bm[tid]);
+        }
+        done += nc;
         __syncthreads();
     }
 }
@@ -1535,11 +1572,13 @@ struct EmitArgs {
 };
 
 // Preorder id and first bucket rank of a cell above LMAX or of a subtree of
-// k_gt_sub, up the parents.
-__device__ __forceinline__ int2 climb(const GNode *__restrict__ nd, int c)
+// k_gt_sub, up the parents to a cell of the levels above MID (those before
+// ntop), which has its own.
+__device__ __forceinline__ int2 climb(const GNode *__restrict__ nd, int ntop, int c)
 {
     int p = 0, b = 0;
-    for (int up = nd[c].par; up >= 0;) {
+    while (c >= ntop) {
+        const int up = nd[c].par;
         const GNode &g = nd[up];
         ++p;
         if (g.ch1 == c) {
@@ -1547,7 +1586,6 @@ __device__ __forceinline__ int2 climb(const GNode *__restrict__ nd, int c)
             b += g.nabLo;
         }
         c = up;
-        up = g.par;
     }
     return make_int2(p + nd[c].pre, b + nd[c].bpre);
 }
@@ -1665,14 +1703,14 @@ __global__ __launch_bounds__(256) void k_gt_emit(int nub, int nup, int nsub, Tre
         if (c >= nup) return;
         const GNode &g = A.nd[c];
         if (g.hi - g.lo < LMAX) return;                  // with its subtree
-        const int2 p = climb(A.nd, c);
+        const int2 p = climb(A.nd, A.L->b, c);
         emit_cell<ORDER>(A, E, c, p.x, p.y);
         return;
     }
     const int t = (blockIdx.x - nub) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= nsub) return;
     const int root = A.sub[t];
-    const int2 s = A.subn[t], p = climb(A.nd, root);
+    const int2 s = A.subn[t], p = climb(A.nd, A.L->b, root);
     for (int k = lane; k <= s.y; k += 64) {
         const int slot = k ? s.x + k - 1 : root;
         emit_cell<ORDER>(A, E, slot, p.x + k, p.y + (k ? A.nd[slot].bpre : 0));
@@ -1867,10 +1905,8 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     } while (0)
     GG_BY_ORDER(k_gt_sub, dim3(gsub), dim3(SUB_T), T);
     if (nunit > 0) GG_BY_ORDER(k_gt_up_unit, dim3(nunit), dim3(64), T);
-    for (int d = nlev - 1; d >= 0; --d)
-        GG_BY_ORDER(k_gt_up_level, dim3(nblk(2 * mbox, 256)), dim3(256), T, d);
-    hipLaunchKernelGGL(k_gt_totals, dim3(1), dim3(256), 0, st, nr, T, ht);
-    if (nunit > 0) GG_BY_ORDER(k_gt_up_bmax, dim3(nunit), dim3(256), T);
+    GG_BY_ORDER(k_gt_up_top, dim3(1), dim3(TOP_T), nr, nlev, T, ht);
+    if (nunit > 0) GG_BY_ORDER(k_gt_up_bmax, dim3(nunit), dim3(BM_T), T);
     GG_HIP(hipGetLastError());
     int tot[6];   // error word, cells, active buckets, largest bucket, slots above LMAX, subtrees
     for (int k = 0; k < 6; ++k) GG_TRY(host_word(st, ht + k, tot + k));
