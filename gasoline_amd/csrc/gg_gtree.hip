@@ -144,22 +144,42 @@ __global__ void k_gt_roots(int n, int nr, const int *__restrict__ rlo,
     unit[k] = k;
 }
 
+// Min/max of a wavefront's lo/hi.  Lanes 0, 8, 16 return the lower bounds x,
+// y, z, lanes 32, 40, 48 the upper ones.  The lanes share the six values out
+// as the reduction goes (three, two, one each), so it takes 9 exchanges of a
+// double; one butterfly per value takes 36, and k_gt_mid spent a quarter of
+// its time in the LDS pipe on them.
+__device__ __forceinline__ bool box_lane(int lane) { return !(lane & 7) && (lane & 24) != 24; }
+__device__ __forceinline__ double wave_box(const double *lo, const double *hi, int lane)
+{
+    const bool h = lane & 32, r = lane & 16, e = lane & 8;
+    double a[3];                             // minima of lo, or of -hi
+    for (int d = 0; d < 3; ++d) {
+        const double t = __shfl_xor(h ? lo[d] : -hi[d], 32);
+        a[d] = h ? -hi[d] : lo[d];
+        a[d] = t < a[d] ? t : a[d];
+    }
+    const double t0 = __shfl_xor(r ? a[0] : a[2], 16), t1 = __shfl_xor(a[1], 16);
+    double k0 = r ? a[2] : a[0], k1 = a[1];
+    k0 = t0 < k0 ? t0 : k0;
+    k1 = t1 < k1 ? t1 : k1;
+    double v = r || !e ? k0 : k1;
+    const double t2 = __shfl_xor(r || e ? k0 : k1, 8);
+    v = t2 < v ? t2 : v;
+    for (int o = 4; o > 0; o >>= 1) {
+        const double t = __shfl_xor(v, o);
+        v = t < v ? t : v;
+    }
+    return h ? -v : v;
+}
+
 // Min/max of a workgroup's lo/hi (256 threads), left to threads 0..5 as
 // order keys: thread d < 3 the lower bound d, 3 + d the upper.
 __device__ __forceinline__ unsigned long long block_box(double *lo, double *hi, double (*sm)[6])
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int o = 32; o > 0; o >>= 1)
-        for (int d = 0; d < 3; ++d) {
-            const double l = __shfl_xor(lo[d], o), h = __shfl_xor(hi[d], o);
-            lo[d] = l < lo[d] ? l : lo[d];
-            hi[d] = h > hi[d] ? h : hi[d];
-        }
-    if (lane == 0)
-        for (int d = 0; d < 3; ++d) {
-            sm[w][d] = lo[d];
-            sm[w][3 + d] = hi[d];
-        }
+    const double x = wave_box(lo, hi, lane);
+    if (box_lane(lane)) sm[w][(lane >> 5) * 3 + ((lane >> 3) & 3)] = x;
     __syncthreads();
     if (threadIdx.x >= 6) return 0;
     double v = sm[0][threadIdx.x];
@@ -579,8 +599,10 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
 // particle on, level by level, with the levels' ends in segl and their
 // numbers in useg, for the upward pass.
 // At most MID / LMAX parts are open at a time, so a level is a handful of
-// wavefront passes over the particles between barriers (7 us measured on one
-// full cell) instead of four launches.  Flags are bits, 64 particles a word, and ranks come
+// wavefront passes over the particles between barriers instead of four
+// launches.  Its barriers and LDS round trips bound it: 88 us for a cell of 4096
+// Plummer particles (160 with a butterfly per bound, the flags' prefix left to
+// one wavefront and the slots' atomics waited for in every level).  Flags are bits, 64 particles a word, and ranks come
 // from a prefix over the 64 words.  MID is what the LDS holds: 124 KB, one
 // workgroup per CU.
 constexpr int MID_T = 1024, MID_O = MID / LMAX, MID_W = MID / 64;
@@ -597,8 +619,8 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     __shared__ double lx[MID], ly[MID], lz[MID];
     __shared__ int ls[MID];
     __shared__ unsigned short posR[MID];
-    __shared__ unsigned long long fbits[MID_W + 1];
-    __shared__ int wpre[MID_W + 1];
+    __shared__ unsigned long long fbits[MID_W];
+    __shared__ int subl[MID], sub0_sh, nsub_sh;
     __shared__ int olo[2][MID_O], ohi[2][MID_O], onode[2][MID_O];
     __shared__ unsigned long long cb[MID_O][6];
     __shared__ double csplit[MID_O];
@@ -631,21 +653,14 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
         onode[0][0] = rootId;
         nopen[0] = 1;
         full = 0;
-        fbits[MID_W] = 0;
     }
+    if (tid < 6 * MID_O) cb[tid / 6][tid % 6] = tid % 6 < 3 ? ~0ull : 0ull;
     __syncthreads();
-    // flags of positions below i
-    auto F = [&](int i) {
-        return wpre[i >> 6] + __popcll(fbits[i >> 6] & ((1ull << (i & 63)) - 1));
-    };
     const int w0 = w * (MID / (MID_T / 64));             // this wavefront's particles
     constexpr int WN = MID / MID_T;                      // its words
-    int cur = 0, depth = 0, nseg = 0;
+    int cur = 0, depth = 0, nseg = 0, nsubl = 0;        // (the counts: wavefront 0)
     for (; nopen[cur] > 0; ++depth) {
         const int no = nopen[cur];
-        if (tid < 6 * no) cb[tid / 6][tid % 6] = tid % 6 < 3 ? ~0ull : 0ull;
-        if (tid == 0) nopen[cur ^ 1] = 0;
-        __syncthreads();
         for (int q = 0; q < no; ++q) {                   // bounds
             const int lo = olo[cur][q], hi = ohi[cur][q];
             if (hi < w0 || lo >= w0 + 64 * WN) continue;
@@ -659,68 +674,86 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
                     bh[d] = v[d] > bh[d] ? v[d] : bh[d];
                 }
             }
-            for (int o = 32; o > 0; o >>= 1)
-                for (int d = 0; d < 3; ++d) {
-                    const double l = __shfl_xor(bl[d], o), h = __shfl_xor(bh[d], o);
-                    bl[d] = l < bl[d] ? l : bl[d];
-                    bh[d] = h > bh[d] ? h : bh[d];
-                }
-            if (lane == 0)
-                for (int d = 0; d < 3; ++d) {
-                    atomicMin(&cb[q][d], ord_key(bl[d]));
-                    atomicMax(&cb[q][3 + d], ord_key(bh[d]));
-                }
+            const double v = wave_box(bl, bh, lane);
+            if (box_lane(lane)) {
+                unsigned long long *k = &cb[q][(lane >> 5) * 3 + ((lane >> 3) & 3)];
+                if (lane < 32) atomicMin(k, ord_key(v));
+                else atomicMax(k, ord_key(v));
+            }
         }
         __syncthreads();
-        if (tid < no) {                                  // split decisions
-            double bmin[3], bmax[3];
+        int got = 0;                                     // the level's first slot (lane 0)
+        if (w == 0) {                                    // split decisions
             bool extent = false;
-            for (int d = 0; d < 3; ++d) {
-                bmin[d] = ord_val(cb[tid][d]);
-                bmax[d] = ord_val(cb[tid][3 + d]);
-                extent |= bmax[d] > bmin[d];
+            if (lane < no) {
+                double bmin[3], bmax[3];
+                for (int d = 0; d < 3; ++d) {
+                    bmin[d] = ord_val(cb[lane][d]);
+                    bmax[d] = ord_val(cb[lane][3 + d]);
+                    extent |= bmax[d] > bmin[d];
+                }
+                int d = 0;
+                for (int k = 1; k < 3; ++k)
+                    if (bmax[k] - bmin[k] > bmax[d] - bmin[d]) d = k;
+                cdim[lane] = extent ? d : -1;            // -1: coincident, a bucket
+                csplit[lane] = 0.5 * (bmin[d] + bmax[d]);
             }
-            int d = 0;
-            for (int k = 1; k < 3; ++k)
-                if (bmax[k] - bmin[k] > bmax[d] - bmin[d]) d = k;
-            cdim[tid] = extent ? d : -1;                 // -1: coincident, a bucket
-            csplit[tid] = 0.5 * (bmin[d] + bmax[d]);
-        }
-        __syncthreads();
-        for (int k = 0; k < WN; ++k) {                   // lower-part flags
-            const int i = w0 + 64 * k + lane;
-            bool f = false;
-            for (int q = 0; q < no; ++q)
-                if (i >= olo[cur][q] && i <= ohi[cur][q] && cdim[q] >= 0)
-                    f = (cdim[q] == 0 ? lx[i] : (cdim[q] == 1 ? ly[i] : lz[i])) < csplit[q];
-            const unsigned long long m = __ballot(f);
-            if (lane == 0) fbits[(w0 >> 6) + k] = m;
-        }
-        __syncthreads();
-        if (w == 0) {
-            const int c = __popcll(fbits[lane]);
-            int inc = c;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int u = __shfl_up(inc, o);
-                if (lane >= o) inc += u;
+            const unsigned long long me = __ballot(extent);
+            if (lane == 0) {
+                nopen[cur ^ 1] = 0;
+                if (me) got = atomicAdd(&L->next, 2 * __popcll(me));   // waited for below
             }
-            wpre[lane] = inc - c;
-            if (lane == 63) wpre[MID_W] = inc;
         }
         __syncthreads();
-        int part[WN];                                    // swap partner's rank slot, -1: none
+        bool f[WN];                                      // lower-part flags
+        for (int k = 0; k < WN; ++k) f[k] = false;
+        for (int q = 0; q < no; ++q) {
+            const int lo = olo[cur][q], hi = ohi[cur][q], dim = cdim[q];
+            if (hi < w0 || lo >= w0 + 64 * WN || dim < 0) continue;
+            const double *v = dim == 0 ? lx : (dim == 1 ? ly : lz), split = csplit[q];
+            for (int k = 0; k < WN; ++k) {
+                const int i = w0 + 64 * k + lane;
+                if (i >= lo && i <= hi) f[k] = v[i] < split;
+            }
+        }
+        unsigned long long fm[WN];
         for (int k = 0; k < WN; ++k) {
-            const int i = w0 + 64 * k + lane;
+            fm[k] = __ballot(f[k]);
+            if (lane == 0) fbits[(w0 >> 6) + k] = fm[k];
+        }
+        __syncthreads();
+        // every wavefront: lane l holds word l of the flags and those before it
+        const unsigned long long word = fbits[lane];
+        int inc = __popcll(word);
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o);
+            if (lane >= o) inc += u;
+        }
+        const int pre = inc - __popcll(word), all = __builtin_amdgcn_readlane(inc, 63);
+        auto F = [&](int i) {                            // flags of positions below i
+            const int l = min(i >> 6, MID_W - 1);
+            const int n = __shfl(pre, l) + __popcll(__shfl(word, l) & ((1ull << (i & 63)) - 1));
+            return i >= MID ? all : n;
+        };
+        int part[WN], Fi[WN];                            // swap partner's rank slot, -1: none
+        for (int k = 0; k < WN; ++k) {
             part[k] = -1;
-            for (int q = 0; q < no; ++q) {
-                const int lo = olo[cur][q], hi = ohi[cur][q];
-                if (i < lo || i > hi || cdim[q] < 0) continue;
-                const int F0 = F(lo), nl = F(hi + 1) - F0, Fi = F(i) - F0;
-                const bool f = (fbits[i >> 6] >> (i & 63)) & 1;
-                if (i >= lo + nl && f) posR[lo + nl - 1 - Fi] = (unsigned short)i;
-                if (i < lo + nl && !f) part[k] = i - Fi;
+            Fi[k] = __builtin_amdgcn_readlane(pre, (w0 >> 6) + k) +
+                    __popcll(fm[k] & ((1ull << lane) - 1));
+        }
+        for (int q = 0; q < no; ++q) {
+            const int lo = olo[cur][q], hi = ohi[cur][q];
+            if (hi < w0 || lo >= w0 + 64 * WN || cdim[q] < 0) continue;
+            const int F0 = F(lo), nl = F(hi + 1) - F0;
+            for (int k = 0; k < WN; ++k) {
+                const int i = w0 + 64 * k + lane;
+                if (i < lo || i > hi) continue;
+                if (i >= lo + nl && f[k])
+                    posR[lo + nl - 1 - (Fi[k] - F0)] = (unsigned short)i;
+                if (i < lo + nl && !f[k]) part[k] = i - (Fi[k] - F0);
             }
         }
+        __syncthreads();
         if (w == 0) {                                    // nodes of the two parts
             const bool in = lane < no;
             int lo = 0, hi = -1, s = 0;
@@ -728,9 +761,12 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
             if (in) {
                 lo = olo[cur][lane];
                 hi = ohi[cur][lane];
+            }
+            const int nl = F(hi + 1) - F(lo);
+            if (in) {
                 s = lo;
                 if (cdim[lane] >= 0) {
-                    s = lo + F(hi + 1) - F(lo);
+                    s = lo + nl;
                     sp = s > lo && s <= hi;
                     if (!sp) atomicOr(&L->err, 1);       // one side empty: reported
                 }
@@ -738,13 +774,10 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
             const bool sub0 = sp && s - lo <= LMAX, sub1 = sp && hi - s + 1 <= LMAX;
             const unsigned long long ms = __ballot(sp), u0 = __ballot(sub0), u1 = __ballot(sub1);
             const unsigned long long below = (1ull << lane) - 1;
-            int got = 0;                                 // slots (lane 0), list places (lane 1)
-            if (lane < 2) {
-                const int want = lane ? __popcll(u0) + __popcll(u1) : 2 * __popcll(ms);
-                if (want) got = atomicAdd(lane ? &L->nsub : &L->next, want);
-            }
             const int id0 = __shfl(got, 0) + 2 * __popcll(ms & below);
-            const int su0 = __shfl(got, 1) + __popcll(u0 & below) + __popcll(u1 & below);
+            const int su0 = nsubl + __popcll(u0 & below) + __popcll(u1 & below);
+            nsubl += __popcll(u0) + __popcll(u1);        // at most one per particle
+            if (lane < 6 * MID_O) cb[lane / 6][lane % 6] = lane % 6 < 3 ? ~0ull : 0ull;
             if (__shfl(got, 0) + 2 * __popcll(ms) > cap) {   // out of slots: built again
                 sp = false;
                 if (lane == 0) {
@@ -752,8 +785,8 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
                     full = 1;
                 }
             }
-            if (sp && sub0) sub[su0] = id0;
-            if (sp && sub1) sub[su0 + sub0] = id0 + 1;
+            if (sp && sub0) subl[su0] = id0;
+            if (sp && sub1) subl[su0 + sub0] = id0 + 1;
             const int me = in ? onode[cur][lane] : 0;
             if (in) seg[glo + nseg + lane] = me;
             nseg += no;
@@ -792,8 +825,6 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
         }
-        __syncthreads();
-        if (full) return;
         for (int k = 0; k < WN; ++k) {                   // the swaps
             if (part[k] < 0) continue;
             const int i = w0 + 64 * k + lane, j = posR[part[k]];
@@ -804,8 +835,15 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
         }
         cur ^= 1;
         __syncthreads();
+        if (full) return;
     }
-    if (tid == 0) useg[blockIdx.x] = make_int2(nseg, depth);
+    if (tid == 0) {
+        useg[blockIdx.x] = make_int2(nseg, depth);
+        sub0_sh = nsubl ? atomicAdd(&L->nsub, nsubl) : 0;
+        nsub_sh = nsubl;
+    }
+    __syncthreads();
+    for (int k = tid; k < nsub_sh; k += MID_T) sub[sub0_sh + k] = subl[k];
     for (int i = tid; i < cnt; i += MID_T) {
         px[glo + i] = lx[i];
         py[glo + i] = ly[i];
