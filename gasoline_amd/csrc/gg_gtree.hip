@@ -207,17 +207,45 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
     const int r0 = root_of(first, nr, rlo), r1 = root_of(last, nr, rlo);
     double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
     bool lack0 = false, lack1 = false;
+    const int lane = threadIdx.x & 63;
     for (int e = 0; e < INIT_E; ++e) {
-        const int i = first + e * 256 + threadIdx.x;
-        if (i > last) break;
-        const double v[3] = {r[3 * (size_t)i], r[3 * (size_t)i + 1], r[3 * (size_t)i + 2]};
-        x[i] = v[0];
-        y[i] = v[1];
-        z[i] = v[2];
-        src[i] = i;
-        const uint32_t t = bits[i];
-        lack0 |= !(t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
-        lack1 |= !(t & GG_TYPE_TREEACTIVE);
+        const int i = first + e * 256 + threadIdx.x, i0 = i - lane;   // i0: the wavefront's first
+        if (i0 > last) break;
+        const bool in = i <= last;
+        double v[3] = {0.0, 0.0, 0.0};
+        if (in) {
+            for (int d = 0; d < 3; ++d) v[d] = r[3 * (size_t)i + d];
+            x[i] = v[0];
+            y[i] = v[1];
+            z[i] = v[2];
+            src[i] = i;
+            const uint32_t t = bits[i];
+            lack0 |= !(t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
+            lack1 |= !(t & GG_TYPE_TREEACTIVE);
+        }
+        if (r0 != r1) {
+            // a block over several systems: 64 particles of one share their
+            // atomics (one per particle made a forest of 48 systems of 1024 to
+            // 16384 particles take 150 us here, 27 this way)
+            const int q0 = root_of(i0, nr, rlo), q1 = root_of(min(i0 + 63, last), nr, rlo);
+            if (q0 == q1) {
+                double l[3], h[3];
+                for (int d = 0; d < 3; ++d) {
+                    const bool ok = in && v[d] == v[d];
+                    l[d] = ok ? v[d] : DBL_MAX;
+                    h[d] = ok ? v[d] : -DBL_MAX;
+                }
+                const double k = wave_box(l, h, lane);
+                if (box_lane(lane)) {
+                    unsigned long long *b = box + BOX_N * (size_t)q0 +
+                                            BOX_S * ((lane >> 5) * 3 + ((lane >> 3) & 3));
+                    if (lane < 32) atomicMin(b, ord_key(k));
+                    else atomicMax(b, ord_key(k));
+                }
+                continue;
+            }
+        }
+        if (!in) continue;
         if (r0 == r1) {
             for (int d = 0; d < 3; ++d) {
                 lo[d] = v[d] < lo[d] ? v[d] : lo[d];
@@ -602,9 +630,9 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
 // wavefront passes over the particles between barriers instead of four
 // launches.  Its barriers and LDS round trips bound it: 88 us for a cell of 4096
 // Plummer particles (160 with a butterfly per bound, the flags' prefix left to
-// one wavefront and the slots' atomics waited for in every level).  Flags are bits, 64 particles a word, and ranks come
-// from a prefix over the 64 words.  MID is what the LDS holds: 124 KB, one
-// workgroup per CU.
+// one wavefront and the slots' atomics waited for in every level).  Flags are
+// bits, 64 particles a word, and ranks come from a prefix over the 64 words.
+// MID is what the LDS holds: 140 KB, one workgroup per CU.
 constexpr int MID_T = 1024, MID_O = MID / LMAX, MID_W = MID / 64;
 static_assert(MID_O <= 64, "one lane per open part");
 static_assert(MID_W == 64, "one wavefront scans the flag words");
