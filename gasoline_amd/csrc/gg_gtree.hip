@@ -634,7 +634,7 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
 // bits, 64 particles a word, and ranks come from a prefix over the 64 words.
 // MID is what the LDS holds: 140 KB, one workgroup per CU.
 constexpr int MID_T = 1024, MID_O = MID / LMAX, MID_W = MID / 64;
-static_assert(MID_O <= 64, "one lane per open part");
+static_assert(6 * MID_O <= 64, "one lane per bound of an open part");
 static_assert(MID_W == 64, "one wavefront scans the flag words");
 __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, int cap,
                                                   GLevel *L, GNode *__restrict__ nd,
@@ -1159,12 +1159,11 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                         bmax[d] = v[d] > bmax[d] ? v[d] : bmax[d];
                     }
                 }
-                for (int o = 32; o > 0; o >>= 1)
-                    for (int d = 0; d < 3; ++d) {
-                        const double l = __shfl_xor(bmin[d], o), h = __shfl_xor(bmax[d], o);
-                        bmin[d] = l < bmin[d] ? l : bmin[d];
-                        bmax[d] = h > bmax[d] ? h : bmax[d];
-                    }
+                const double bx = wave_box(bmin, bmax, lane);
+                for (int d = 0; d < 3; ++d) {
+                    bmin[d] = __shfl(bx, 8 * d);
+                    bmax[d] = __shfl(bx, 32 + 8 * d);
+                }
                 int dim = 0;
                 for (int q = 1; q < 3; ++q)
                     if (bmax[q] - bmin[q] > bmax[dim] - bmin[dim]) dim = q;
