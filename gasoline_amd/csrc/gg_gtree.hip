@@ -1095,7 +1095,11 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
     __shared__ short qa[3][2][LMAX / 2];  // open cells of a level: larger, smaller than 33
     __shared__ int qn[3][2], nloc_sh, slot_sh, maxb_sh;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, half = lane >> 5, l32 = lane & 31;
-    if (A.L->err & 2) return;            // out of slots: built again
+    // No early exit when slots have run out: other workgroups of this launch
+    // set that bit while this one starts, so its wavefronts could read it
+    // differently and part of them leave the rest to LDS they never filled.
+    // Every listed subtree is valid whatever the bit; room, one value for the
+    // workgroup, guards the writes past the slots.
     const int nsub = A.L->nsub;
     for (int t = blockIdx.x; t < nsub; t += gridDim.x) {
         const int root = A.sub[t];

@@ -94,3 +94,23 @@ def test_forest_of_large_and_small_systems(gpu):
     r, v, m = ics.plummer(off[-1], seed=9)
     act = np.where(np.arange(off[-1]) % 5 == 0, 1, 3).astype(np.uint32)
     check(gpu, r, m, np.full(off[-1], 0.01), 16, 2, act=act, off=off)
+
+
+def groups(g, chain, same, span):
+    """g groups, each of `same` coincident particles and a chain of `chain`
+    at span * 0.4^k beside them, of which every split takes one away: two
+    cells a particle, whatever a bucket may hold."""
+    x = np.concatenate([span * 0.4 ** np.arange(chain), np.zeros(same)])
+    r = np.zeros((g, len(x), 3))
+    r[:, :, 0] = x
+    r[:, :, 1] = 4.0 * (np.arange(g) % 64)[:, None]
+    r[:, :, 2] = 4.0 * (np.arange(g) // 64)[:, None]
+    return r.reshape(-1, 3)
+
+
+def test_out_of_slots_while_subtrees_wait_for_the_chip(gpu):
+    # about a thousand subtrees, twice what the chip holds at once, of which
+    # the first ones already use up the slots of the first try
+    r = groups(4000, 30, 64, 1.0)
+    m = np.full(len(r), 1.0 / len(r))
+    check(gpu, r, m, np.full(len(r), 0.01), 64, 2)
