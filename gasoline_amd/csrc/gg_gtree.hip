@@ -305,6 +305,7 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int a = L->a, b = L->b, nunit0 = L->nunit;
     const bool bad = L->err != 0;
+    __syncthreads();                     // (read before any wavefront below sets it)
     int nsp = 0, ntl = 0, nun = 0;       // splits, tiles and units so far
     for (int base = a; base < b && !bad; base += CTL_T) {
         const int c = base + tid;

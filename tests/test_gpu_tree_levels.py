@@ -114,3 +114,12 @@ def test_out_of_slots_while_subtrees_wait_for_the_chip(gpu):
     r = groups(4000, 30, 64, 1.0)
     m = np.full(len(r), 1.0 / len(r))
     check(gpu, r, m, np.full(len(r), 0.01), 64, 2)
+
+
+@pytest.mark.parametrize("g,same", [(6, 4200), (8, 600)])
+def test_out_of_slots_above_the_subtrees(gpu, g, same):
+    # chains that use up the slots of the first try in the levels above 4096
+    # particles, and in the cells between 4096 and 512
+    r = groups(g, 700, same, 1.0)
+    m = np.full(len(r), 1.0 / len(r))
+    check(gpu, r, m, np.full(len(r), 0.01), 64, 4)
