@@ -1477,7 +1477,10 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
     __shared__ int2 ws[TOP_T / 64];
     int2 run = make_int2(0, 0);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int lev = A.L->err & 2 ? 0 : nlev;
+    // A build that failed has cells without a record: the host gets zeros for
+    // its totals (a word of -1 would read as not yet written).
+    const int err = A.L->err, lev = err ? 0 : nlev;
+    if (err) nr = 0;
     auto splits = [&](int c) {                           // (the others are units)
         const GNode &g = A.nd[c];
         return g.hi - g.lo >= MID && g.dim >= 0;
@@ -1522,7 +1525,7 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
         tell_host(host + 3, A.L->maxb);
         tell_host(host + 4, A.L->next);
         tell_host(host + 5, A.L->nsub);
-        tell_host(host, A.L->err);
+        tell_host(host, err);
     }
     for (int d = 0; d < lev; ++d) {
         const int c1 = A.L->lv[d + 1];

@@ -123,3 +123,23 @@ def test_out_of_slots_above_the_subtrees(gpu, g, same):
     r = groups(g, 700, same, 1.0)
     m = np.full(len(r), 1.0 / len(r))
     check(gpu, r, m, np.full(len(r), 0.01), 64, 4)
+
+
+@pytest.mark.parametrize("n", [20, 100, 600, 5000, 30000])
+def test_split_with_an_empty_side_is_refused(gpu, n):
+    # two positions whose midpoint rounds to the lower one, in a cell of each
+    # stage's size; the handle builds again afterwards
+    r, v, m = ics.plummer(n, seed=n)
+    bad = np.ones((n, 3))
+    bad[n // 2:, 0] = np.nextafter(1.0, 2.0)
+    with gpu.Pkd(n, prec=gpu.PREC_FP64) as pk:
+        pk.put("fMass", m)
+        pk.put("fSoft", np.full(n, 0.01))
+        for _ in range(2):
+            pk.put("r", bad)
+            with pytest.raises(gpu.GGError, match="one side empty"):
+                pk.build_binary(16, 1, 0.7, 2)
+            pk.put("r", r)
+            pk.build_binary(16, 1, 0.7, 2)
+            T = O.Tree(r, m, np.full(n, 0.01), nBucket=16, dTheta=0.7, iOrder=2)
+            assert np.array_equal(pk.tree_info()[1], T.perm())
