@@ -29,6 +29,7 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace gg {
@@ -37,6 +38,7 @@ namespace {
 int nblk(int64_t n, int b) { return (int)((n + b - 1) / b); }
 
 constexpr int LMAX = 512;        // cells of at most LMAX particles finish in one workgroup
+constexpr int LSML = 128;        // systems of at most LSML particles finish in one wavefront
 constexpr int MID = 4096;        // cells of at most MID particles reach LMAX in one workgroup
 constexpr int DMAX = 2048;       // levels above MID a tree may have
 
@@ -106,7 +108,7 @@ __device__ __forceinline__ void box_init(unsigned long long *b)
     }
 }
 
-// The last root whose first position is <= i.
+// The last of nr ascending first positions (or tiles) that is <= i.
 __device__ __forceinline__ int root_of(int i, int nr, const int *__restrict__ rlo)
 {
     int lo = 0, hi = nr - 1;
@@ -118,30 +120,67 @@ __device__ __forceinline__ int root_of(int i, int nr, const int *__restrict__ rl
     return lo;
 }
 
-// Root cells, their empty bounds and the level state.
-__global__ void k_gt_roots(int n, int nr, const int *__restrict__ rlo,
-                           const int *__restrict__ rhi,
-                           GNode *__restrict__ nd, unsigned long long *__restrict__ box,
-                           int *__restrict__ unit, GLevel *__restrict__ L)
+// The systems by size, so that a forest of very many small ones costs what
+// its particles cost: those of more than MID particles are the cells of the
+// first level (with bounds), those of more than LMAX go to k_gt_mid, those
+// of more than nBucket to k_gt_sub (those of at most LSML first), and the
+// rest are buckets (k_gt_tiny).  The host gives every 256 systems their first
+// entries of the lists.  A single system is the whole store and has none of
+// these arrays.
+struct Roots {
+    int n, nr, nBucket;
+    int nbig, nunit, nsub[2], maxTiny;   // systems of each list, the largest bucket
+    const int *lo, *hi;                  // particle ranges
+    const int *bslot, *blo, *bhi;        // those of more than MID particles
+    const int *base[3];                  // per 256 systems: nsub[0], nsub[1], nunit
+    const int *tslot, *toff;             // those of more than LMAX: slot, first tile of the
+    int ntroot;                          // type orders
+};
+
+// Root cells, their lists, the empty bounds and the level state.
+__global__ __launch_bounds__(256) void k_gt_roots(Roots R, GNode *__restrict__ nd,
+                                                  unsigned long long *__restrict__ box,
+                                                  int *__restrict__ unit, int *__restrict__ sub,
+                                                  GLevel *__restrict__ L)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int ws[4][3];
+    const int k = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (k == 0) {
         L->a = 0;
-        L->b = L->next = nr;
-        L->ntile = L->nunit = L->nloc = L->nsub = L->err = 0;
-        L->need[0] = L->need[1] = L->maxb = 0;
+        L->b = L->next = R.nr;
+        L->nunit = R.nunit;
+        L->nsub = R.nsub[0] + R.nsub[1];
+        L->maxb = R.maxTiny;
+        L->ntile = L->nloc = L->err = 0;
+        L->need[0] = L->need[1] = 0;
     }
-    if (k >= nr) return;
-    GNode &g = nd[k];
-    g.lo = nr > 1 ? rlo[k] : 0;
-    g.hi = nr > 1 ? rhi[k] : n - 1;
-    g.par = -1;
-    g.root = k;
-    g.ch0 = g.ch1 = -1;
-    g.dim = -1;
-    g.split = 0.0;
-    box_init(box + BOX_N * (size_t)k);
-    unit[k] = k;
+    if (k < R.nbig) box_init(box + BOX_N * (size_t)k);
+    int cnt = 0;
+    if (k < R.nr) {
+        GNode &g = nd[k];
+        g.lo = R.nr > 1 ? R.lo[k] : 0;
+        g.hi = R.nr > 1 ? R.hi[k] : R.n - 1;
+        g.par = -1;
+        g.root = k;
+        g.ch0 = g.ch1 = -1;
+        g.dim = -1;
+        g.split = 0.0;
+        cnt = g.hi - g.lo + 1;
+    }
+    const int cls = cnt <= R.nBucket ? -1 : cnt <= LSML ? 0 : cnt <= LMAX ? 1 : cnt <= MID ? 2 : -1;
+    unsigned long long m[3];
+    for (int q = 0; q < 3; ++q) {
+        m[q] = __ballot(cls == q);
+        if (lane == 0) ws[w][q] = __popcll(m[q]);
+    }
+    __syncthreads();
+    for (int q = 0; q < 3; ++q) {
+        if (cls != q) continue;
+        int at = (R.nr > 1 ? R.base[q][blockIdx.x] : 0) + __popcll(m[q] & ((1ull << lane) - 1));
+        for (int v = 0; v < w; ++v) at += ws[v][q];
+        if (q == 2) unit[at] = k;
+        else sub[q ? R.nsub[0] + at : at] = k;
+    }
 }
 
 // Min/max of a wavefront's lo/hi.  Lanes 0, 8, 16 return the lower bounds x,
@@ -192,10 +231,10 @@ __device__ __forceinline__ unsigned long long block_box(double *lo, double *hi, 
 
 constexpr int INIT_E = 8;        // particles per thread of k_gt_init
 
-// Positions into storage order, the roots' bounds, and whether a particle
-// lacks the type bits of msrBuildTree's orders (*need, master.c:4262).
-__global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__restrict__ rlo,
-                                                 const double *__restrict__ r,
+// Positions into storage order, the bounds of the systems of more than MID
+// particles, and whether a particle lacks the type bits of msrBuildTree's
+// orders (*need, master.c:4262).
+__global__ __launch_bounds__(256) void k_gt_init(Roots R, const double *__restrict__ r,
                                                  const uint32_t *__restrict__ bits,
                                                  double *__restrict__ x, double *__restrict__ y,
                                                  double *__restrict__ z, int *__restrict__ src,
@@ -203,11 +242,27 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
                                                  GLevel *__restrict__ L)
 {
     __shared__ double sm[4][6];
-    const int first = blockIdx.x * (256 * INIT_E), last = min(n, first + 256 * INIT_E) - 1;
-    const int r0 = root_of(first, nr, rlo), r1 = root_of(last, nr, rlo);
+    const int first = blockIdx.x * (256 * INIT_E), last = min(R.n, first + 256 * INIT_E) - 1;
+    const int lane = threadIdx.x & 63;
+    // the system of a position among the large ones (-1: of none), and its end
+    auto big = [&](int i, int &end) {
+        if (R.nr == 1) {
+            end = R.n - 1;
+            return R.nbig - 1;
+        }
+        if (R.nbig == 0 || i < R.blo[0]) return -1;
+        const int q = root_of(i, R.nbig, R.blo);
+        end = R.bhi[q];
+        return i <= end ? q : -1;
+    };
+    int e0 = 0, e1 = 0;
+    const int r0 = big(first, e0), r1 = big(last, e1);
+    // all of the block in one large system, or none of it in any (a large
+    // system is longer than a block)
+    static_assert(MID >= 256 * INIT_E, "a large system within a block holds one of its ends");
+    const bool one = r0 == r1;
     double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
     bool lack0 = false, lack1 = false;
-    const int lane = threadIdx.x & 63;
     for (int e = 0; e < INIT_E; ++e) {
         const int i = first + e * 256 + threadIdx.x, i0 = i - lane;   // i0: the wavefront's first
         if (i0 > last) break;
@@ -223,12 +278,13 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
             lack0 |= !(t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
             lack1 |= !(t & GG_TYPE_TREEACTIVE);
         }
-        if (r0 != r1) {
+        if (!one) {
             // a block over several systems: 64 particles of one share their
             // atomics (one per particle made a forest of 48 systems of 1024 to
             // 16384 particles take 150 us here, 27 this way)
-            const int q0 = root_of(i0, nr, rlo), q1 = root_of(min(i0 + 63, last), nr, rlo);
-            if (q0 == q1) {
+            int end = 0;
+            const int q0 = big(i0, end);
+            if (q0 >= 0 && min(i0 + 63, last) <= end) {
                 double l[3], h[3];
                 for (int d = 0; d < 3; ++d) {
                     const bool ok = in && v[d] == v[d];
@@ -246,13 +302,17 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
             }
         }
         if (!in) continue;
-        if (r0 == r1) {
+        if (one) {
+            if (r0 < 0) continue;
             for (int d = 0; d < 3; ++d) {
                 lo[d] = v[d] < lo[d] ? v[d] : lo[d];
                 hi[d] = v[d] > hi[d] ? v[d] : hi[d];
             }
         } else {
-            unsigned long long *b = box + BOX_N * (size_t)root_of(i, nr, rlo);
+            int end = 0;
+            const int q = big(i, end);
+            if (q < 0) continue;
+            unsigned long long *b = box + BOX_N * (size_t)q;
             for (int d = 0; d < 3; ++d) {
                 if (v[d] != v[d]) continue;
                 atomicMin(b + BOX_S * d, ord_key(v[d]));
@@ -265,7 +325,7 @@ __global__ __launch_bounds__(256) void k_gt_init(int n, int nr, const int *__res
         if (m0) atomicOr(&L->need[0], 1);
         if (m1) atomicOr(&L->need[1], 1);
     }
-    if (r0 != r1) return;
+    if (!one || r0 < 0) return;
     const unsigned long long k = block_box(lo, hi, sm);
     unsigned long long *b = box + BOX_N * (size_t)r0 + BOX_S * threadIdx.x;
     if (threadIdx.x < 3) atomicMin(b, k);
@@ -283,16 +343,17 @@ __global__ void k_gt_tell(const int *__restrict__ v, int *__restrict__ host)
     tell_host(host, *v);
 }
 
-// One workgroup decides the level's cells (mode 0, pkd.c:2489-2505): cells of
-// more than MID particles with any extent split at the middle of their
-// longest axis and get two child ids; the others join the unit list.  Then
-// the tiles of the splitting cells.  mode 1 (the type orders): every cell
-// is partitioned, none split.  The tile count goes to *host.  One workgroup
-// because a level has at most 2 n / MID cells and every later launch waits
-// for it: 4-6 us a level, against the three scans, the decision and id
-// kernels and the host's wait it replaces.
+// One workgroup decides the level's cells (pkd.c:2489-2505): cells of more
+// than MID particles with any extent split at the middle of their longest axis
+// and get two child ids; the others join the unit list.  Then the tiles of the
+// splitting cells.  The first level's cells are the systems of more than MID
+// particles (list, if they are not the only ones).  The tile count goes to
+// *host.  One workgroup because a level has at most 2 n / MID cells and every
+// later launch waits for it: 4-6 us a level, against the three scans, the
+// decision and id kernels and the host's wait it replaces.
 constexpr int CTL_T = 1024;
-__global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, int cap, GLevel *L,
+__global__ __launch_bounds__(CTL_T) void k_gt_ctl(int ts, int depth, int cap, int nlist,
+                                                  const int *__restrict__ list, GLevel *L,
                                                   GNode *__restrict__ nd,
                                                   const unsigned long long *__restrict__ box,
                                                   unsigned long long *__restrict__ kbox,
@@ -306,20 +367,19 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
     const int a = L->a, b = L->b, nunit0 = L->nunit;
     const bool bad = L->err != 0;
     __syncthreads();                     // (read before any wavefront below sets it)
+    const int nc = list ? nlist : b - a;
     int nsp = 0, ntl = 0, nun = 0;       // splits, tiles and units so far
-    for (int base = a; base < b && !bad; base += CTL_T) {
-        const int c = base + tid;
+    for (int base = 0; base < nc && !bad; base += CTL_T) {
+        const int i = base + tid, c = i >= nc ? 0 : list ? list[i] : a + i;
         int split = 0, nt = 0, un = 0, lo = 0;
-        if (c < b) {
+        if (i < nc) {
             GNode &g = nd[c];
             lo = g.lo;
             const int cnt = g.hi - lo + 1;
-            if (mode == 1) {
-                nt = (cnt + ts - 1) / ts;
-            } else if (cnt <= MID) {
+            if (cnt <= MID) {
                 un = 1;
             } else {
-                const unsigned long long *k = box + BOX_N * (size_t)(c - a);
+                const unsigned long long *k = box + BOX_N * (size_t)i;
                 double bmin[3], bmax[3];
                 for (int d = 0; d < 3; ++d) {
                     bmin[d] = ord_val(k[BOX_S * d]);
@@ -327,7 +387,7 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
                 }
                 bool extent = false;
                 for (int d = 0; d < 3; ++d) extent |= bmax[d] > bmin[d];
-                if (extent && b + 2 * (c - a) + 2 > cap) {   // (a bound on its children's slots)
+                if (extent && b + 2 * i + 2 > cap) {   // (a bound on its children's slots)
                     atomicOr(&L->err, 2);
                 } else if (extent) {
                     int d = 0;
@@ -407,13 +467,11 @@ __global__ __launch_bounds__(CTL_T) void k_gt_ctl(int mode, int ts, int depth, i
     }
     if (tid == 0) {
         L->ntile = ntl;
-        if (mode == 0) {
-            L->lv[depth] = a;
-            L->a = b;
-            L->b = L->next = b + 2 * nsp;
-            L->nunit = nunit0 + nun;
-            tell_host(host + 1, nunit0 + nun);
-        }
+        L->lv[depth] = a;
+        L->a = b;
+        L->b = L->next = b + 2 * nsp;
+        L->nunit = nunit0 + nun;
+        tell_host(host + 1, nunit0 + nun);
         tell_host(host, ntl);
     }
 }
@@ -432,6 +490,101 @@ struct TileArgs {
     int *posR;
     int *err;
 };
+
+// The tiles of the type orders: every system of more than LMAX particles is
+// partitioned, none split.
+__global__ __launch_bounds__(256) void k_gt_type_tiles(Roots R, int ts, int ntile,
+                                                       const GNode *__restrict__ nd,
+                                                       int4 *__restrict__ tiles,
+                                                       GLevel *__restrict__ L)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t == 0) L->ntile = ntile;
+    if (t >= ntile) return;
+    int c = 0, t0 = 0, t1 = ntile;
+    if (R.nr > 1) {
+        const int q = root_of(t, R.ntroot, R.toff);
+        c = R.tslot[q];
+        t0 = R.toff[q];
+        t1 = q + 1 < R.ntroot ? R.toff[q + 1] : ntile;
+    }
+    tiles[t] = make_int4(c, nd[c].lo + (t - t0) * ts, t0, t1);
+}
+
+// Both type orders of the systems of at most LMAX particles, a wavefront each:
+// the Hoare swaps on the particles' indices in LDS, then the particles in
+// that order.  (As tiles, systems of 4 particles would take six launches of a
+// workgroup each.)
+constexpr int TY_W = 4;
+__global__ __launch_bounds__(64 * TY_W) void k_gt_type_small(Roots R, const double *__restrict__ r,
+                                                             const uint32_t *__restrict__ bits,
+                                                             double *__restrict__ x,
+                                                             double *__restrict__ y,
+                                                             double *__restrict__ z,
+                                                             int *__restrict__ src)
+{
+    __shared__ short idx_[TY_W][LMAX], posR_[TY_W][LMAX];
+    __shared__ unsigned char bit_[TY_W][LMAX];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    short *idx = idx_[w], *posR = posR_[w];
+    unsigned char *bit = bit_[w];
+    const unsigned long long below = (1ull << lane) - 1;
+    auto wave_fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    for (int k = blockIdx.x * TY_W + w; k < R.nr; k += gridDim.x * TY_W) {
+        const int lo = R.nr > 1 ? R.lo[k] : 0, cnt = (R.nr > 1 ? R.hi[k] : R.n - 1) - lo + 1;
+        if (cnt < 2 || cnt > LMAX) continue;
+        for (int i = lane; i < cnt; i += 64) {
+            const uint32_t t = bits[lo + i];
+            idx[i] = (short)i;
+            bit[i] = (t & GG_TYPE_TREEACTIVE ? 2 : 0) |
+                     (t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE) ? 1 : 0);
+        }
+        wave_fence();
+        for (int mask = 1; mask <= 2; ++mask) {
+            int nl = 0;
+            for (int c0 = 0; c0 < cnt; c0 += 64)
+                nl += __popcll(__ballot(c0 + lane < cnt && (bit[idx[c0 + lane]] & mask)));
+            int run = 0;
+            for (int c0 = 0; c0 < cnt; c0 += 64) {   // upper positions holding a lower one
+                const int i = c0 + lane;
+                const bool f = i < cnt && (bit[idx[i]] & mask);
+                const unsigned long long m = __ballot(f);
+                const int ex = run + __popcll(m & below);
+                if (f && i >= nl) posR[nl - 1 - ex] = (short)i;
+                run += __popcll(m);
+            }
+            wave_fence();
+            run = 0;
+            for (int c0 = 0; c0 < nl; c0 += 64) {    // lower positions holding an upper one
+                const int i = c0 + lane;
+                const bool in = i < nl, f = in && (bit[idx[i]] & mask);
+                const unsigned long long m = __ballot(f);
+                const int ex = run + __popcll(m & below);
+                if (in && !f) {
+                    const int j = posR[i - ex];
+                    const short u = idx[i];
+                    idx[i] = idx[j];
+                    idx[j] = u;
+                }
+                run += __popcll(m);
+            }
+            wave_fence();
+        }
+        for (int i = lane; i < cnt; i += 64) {
+            const int s = idx[i];
+            if (s == i) continue;
+            src[lo + i] = lo + s;
+            x[lo + i] = r[3 * (size_t)(lo + s)];
+            y[lo + i] = r[3 * (size_t)(lo + s) + 1];
+            z[lo + i] = r[3 * (size_t)(lo + s) + 2];
+        }
+        wave_fence();
+    }
+}
 
 // mode 0: the coordinate below the cell's split; mode 1: a type bit of mask.
 template <int MODE>
@@ -1081,19 +1234,28 @@ struct TreeArgs {
 // second child to arrive computing the parent, so a level needs no barrier
 // there.  Moments come from the children's by shifting (31 values, ~400
 // operations a cell) instead of from every particle of every cell.
-constexpr int SUB_T = 256, SN = 2 * LMAX;
-template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs A)
+// Two forms: LM = LMAX particles by T = 256 threads (57 KB of LDS, two
+// workgroups a CU) for the parts of larger cells, and LM = LSML by one
+// wavefront (14 KB, eleven a CU) for small systems, of which a forest may have
+// very many and each takes its latency whatever its size.  A workgroup takes
+// entries t0 to t1 of the list (t1 < 0: all) in turn, and slots for several
+// small subtrees by one atomic (chunk, where there is room to lose part of
+// one): the atomics on the level's line, 10 ns each, bound a forest of small
+// systems whatever the occupancy.  200000 systems of 20 particles, a build:
+// 14.0 ms with the first form alone, 11.1 with the second, 2.5 with both.
+template <int ORDER, int LM, int T>
+__global__ __launch_bounds__(T) void k_gt_sub(TreeArgs A, int t0, int t1, int chunk)
 {
 #pragma clang fp contract(off)
-    constexpr int GS = gm_stride(ORDER);
-    __shared__ double lx[LMAX], ly[LMAX], lz[LMAX], nsp[SN];
-    __shared__ double lm[LMAX], lh[LMAX];
-    __shared__ int ls[LMAX], arr[SN];
-    __shared__ short posR[LMAX];
+    constexpr int GS = gm_stride(ORDER), SN = 2 * LM;
+    __shared__ double lx[LM], ly[LM], lz[LM], nsp[SN];
+    __shared__ double lm[LM], lh[LM];
+    __shared__ int ls[LM], arr[SN];
+    __shared__ short posR[LM];
     __shared__ short nlo[SN], nhi[SN], npar[SN], nch[SN], nsz[SN], nac[SN], npre[SN], nbp[SN];
     __shared__ signed char ndm[SN];
-    __shared__ unsigned char lact[LMAX];
-    __shared__ short qa[3][2][LMAX / 2];  // open cells of a level: larger, smaller than 33
+    __shared__ unsigned char lact[LM];
+    __shared__ short qa[3][2][LM / 2];  // open cells of a level: larger, smaller than 33
     __shared__ int qn[3][2], nloc_sh, slot_sh, maxb_sh;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, half = lane >> 5, l32 = lane & 31;
     // No early exit when slots have run out: other workgroups of this launch
@@ -1101,11 +1263,13 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
     // differently and part of them leave the rest to LDS they never filled.
     // Every listed subtree is valid whatever the bit; room, one value for the
     // workgroup, guards the writes past the slots.
-    const int nsub = A.L->nsub;
-    for (int t = blockIdx.x; t < nsub; t += gridDim.x) {
+    const int nsub = t1 < 0 ? A.L->nsub : t1, next = A.L->next;
+    int slot = 0, left = 0;              // slots in hand (thread 0)
+    if (tid == 0) maxb_sh = 0;
+    for (int t = t0 + blockIdx.x; t < nsub; t += gridDim.x) {
         const int root = A.sub[t];
         const int glo = A.nd[root].lo, cnt = A.nd[root].hi - glo + 1, troot = A.nd[root].root;
-        for (int i = tid; i < cnt; i += SUB_T) {
+        for (int i = tid; i < cnt; i += T) {
             lx[i] = A.px[glo + i];
             ly[i] = A.py[glo + i];
             lz[i] = A.pz[glo + i];
@@ -1118,7 +1282,6 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
             ndm[0] = -1;
             nsp[0] = 0.0;
             nloc_sh = 1;
-            maxb_sh = 0;
             for (int k = 0; k < 3; ++k) qn[k][0] = qn[k][1] = 0;
             if (cnt > A.nBucket) {
                 const int big = cnt > 32 ? 0 : 1;
@@ -1152,7 +1315,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
             const int nxt = cur == 2 ? 0 : cur + 1, nn2 = nxt == 2 ? 0 : nxt + 1;
             const int nbig = qn[cur][0], nsml = qn[cur][1];
             if (tid == 0) qn[nn2][0] = qn[nn2][1] = 0;   // the queue after the next
-            for (int b = w; b < nbig; b += SUB_T / 64) {
+            for (int b = w; b < nbig; b += T / 64) {
                 const int k = qa[cur][0][b];
                 const int lo = nlo[k], hi = nhi[k];
                 double bmin[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
@@ -1214,7 +1377,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                 }
                 if (lane == 0) children(k, lo, hi, s, dim, split, nxt);
             }
-            for (int b = 2 * w; b < nsml; b += SUB_T / 32) {   // at most 32 particles: half a
+            for (int b = 2 * w; b < nsml; b += T / 32) {   // at most 32 particles: half a
                 const bool have = b + half < nsml;             // wavefront each
                 const int k = have ? qa[cur][1][b + half] : 0;
                 const int lo = have ? nlo[k] : 0, hi = have ? nhi[k] : -1;
@@ -1266,8 +1429,23 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
         }
         // storage-order particles; the cells' slots
         const int nloc = nloc_sh;
-        if (tid == 0) slot_sh = nloc > 1 ? atomicAdd(&A.L->nloc, nloc - 1) : 0;
-        for (int i = tid; i < cnt; i += SUB_T) {
+        if (tid == 0) {
+            const int need = nloc - 1;
+            if (need == 0) {
+                slot_sh = 0;
+            } else if (4 * need > chunk) {
+                slot_sh = atomicAdd(&A.L->nloc, need);
+            } else {
+                if (need > left) {
+                    slot = atomicAdd(&A.L->nloc, chunk);
+                    left = chunk;
+                }
+                slot_sh = slot;
+                slot += need;
+                left -= need;
+            }
+        }
+        for (int i = tid; i < cnt; i += T) {
             const int s = ls[i];
             const double mm = A.m[s], hh = A.h[s];
             const uint32_t bt = A.bits[s];
@@ -1282,13 +1460,13 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
             A.ph[glo + i] = hh;
             A.pact[glo + i] = bt;
         }
-        for (int k = tid; k < nloc; k += SUB_T) arr[k] = 0;
+        for (int k = tid; k < nloc; k += T) arr[k] = 0;
         __syncthreads();
         const int used = slot_sh + nloc - 1;             // from the last slot down
-        const bool room = A.L->next + used <= A.cap;
+        const bool room = next + used <= A.cap;
         if (!room && tid == 0) atomicOr(&A.L->err, 2);
         // sizes and active buckets, climbing from the buckets
-        for (int k = tid; k < nloc; k += SUB_T) {
+        for (int k = tid; k < nloc; k += T) {
             if (nch[k] >= 0) continue;
             int na = 0;
             for (int i = nlo[k]; i <= nhi[k]; ++i) na |= lact[i];
@@ -1305,7 +1483,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
             }
         }
         __syncthreads();
-        for (int k = tid; k < nloc; k += SUB_T) {        // preorder ids and bucket ranks
+        for (int k = tid; k < nloc; k += T) {        // preorder ids and bucket ranks
             int p = 0, bp = 0;
             for (int c = k; npar[c] >= 0; c = npar[c]) {
                 const int c0 = nch[npar[c]];
@@ -1331,7 +1509,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                 hh = lh[i];
                 return lact[i] != 0;
             };
-            for (int k = tid; k < nloc; k += SUB_T) {    // records, climbing likewise
+            for (int k = tid; k < nloc; k += T) {    // records, climbing likewise
                 if (nch[k] >= 0) continue;
                 double g[GS];
                 for (int q = 0; q < GS; ++q) g[q] = 0.0;
@@ -1357,7 +1535,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                 }
             }
             __syncthreads();
-            for (int k = tid >> 4; k < nloc; k += SUB_T / 16) {   // Bmax, 16 lanes per cell
+            for (int k = tid >> 4; k < nloc; k += T / 16) {   // Bmax, 16 lanes per cell
                 if (nch[k] < 0) continue;                // buckets have theirs
                 double *o = A.gm + (size_t)GS * slot(k);
                 const double cm[3] = {o[2], o[3], o[4]};
@@ -1372,7 +1550,7 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                 }
                 if ((tid & 15) == 0) o[GM_B] = b2;
             }
-            for (int k = tid; k < nloc; k += SUB_T) {
+            for (int k = tid; k < nloc; k += T) {
                 GNode &g = A.nd[slot(k)];
                 const int c = nch[k];
                 if (k > 0) {
@@ -1389,13 +1567,44 @@ template <int ORDER> __global__ __launch_bounds__(SUB_T) void k_gt_sub(TreeArgs 
                 g.ch0 = c < 0 ? -1 : slot(c);
                 g.ch1 = c < 0 ? -1 : slot(c + 1);
             }
-            if (tid == 0) {
-                A.subn[t] = make_int2(s1, nloc - 1);
-                atomicMax(&A.L->maxb, maxb_sh);
-            }
+            if (tid == 0) A.subn[t] = make_int2(s1, nloc - 1);
         }
         __syncthreads();
     }
+    if (tid == 0 && maxb_sh > 0) atomicMax(&A.L->maxb, maxb_sh);
+}
+
+// The systems of at most nBucket particles, a bucket each, by one thread.
+template <int ORDER> __global__ __launch_bounds__(256) void k_gt_tiny(int nr, TreeArgs A)
+{
+    constexpr int GS = gm_stride(ORDER);
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= nr) return;
+    GNode &g = A.nd[c];
+    if (g.hi - g.lo >= A.nBucket) return;
+    for (int i = g.lo; i <= g.hi; ++i) {
+        const int s = A.perm[i];
+        A.pm[i] = A.m[s];
+        A.ph[i] = A.h[s];
+        A.pact[i] = A.bits[s];
+    }
+    double v[GS];
+    for (int k = 0; k < GS; ++k) v[k] = 0.0;
+    const int na = bucket_record<ORDER>(
+        g.lo, g.hi,
+        [&](int i, double *p, double &m, double &h) {
+            p[0] = A.px[i];
+            p[1] = A.py[i];
+            p[2] = A.pz[i];
+            m = A.pm[i];
+            h = A.ph[i];
+            return (A.pact[i] & 1u) != 0;
+        },
+        v, A.bb8 + 8 * (size_t)c);
+    double *o = A.gm + (size_t)GS * c;
+    for (int k = 0; k < GS; ++k) o[k] = v[k];
+    g.size = 1;
+    g.nab = na > 0;
 }
 
 // A closed cell above LMAX, by a pair of lanes (q 0, 1): its record and its
@@ -1470,9 +1679,11 @@ template <int ORDER> __global__ __launch_bounds__(64) void k_gt_up_unit(TreeArgs
 // few, so what it costs is one record's chain of loads: about 2 us between
 // barriers against 4.7 us for a launch of its own (18 of them on a galaxy of
 // 50k particles, 26 on 2^21).
-constexpr int TOP_T = 512;
+constexpr int TOP_T = 512, TOP_R = 8;                    // TOP_R: roots per thread
 template <int ORDER>
-__global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs A, int *host)
+__global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlist,
+                                                     const int *__restrict__ list, int nlev,
+                                                     TreeArgs A, int *host)
 {
     __shared__ int2 ws[TOP_T / 64];
     int2 run = make_int2(0, 0);
@@ -1485,16 +1696,29 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
         const GNode &g = A.nd[c];
         return g.hi - g.lo >= MID && g.dim >= 0;
     };
+    // a level's cells (the first one's may be a list)
+    auto count = [&](int d) { return d == 0 && list ? nlist : A.L->lv[d + 1] - A.L->lv[d]; };
+    auto cell = [&](int d, int i) { return d == 0 && list ? list[i] : A.L->lv[d] + i; };
     for (int d = lev - 1; d >= 0; --d) {
-        const int c1 = A.L->lv[d + 1];
-        for (int c = A.L->lv[d] + (tid >> 1); c < c1; c += TOP_T / 2)
+        const int nc = count(d);
+        for (int i = tid >> 1; i < nc; i += TOP_T / 2) {
+            const int c = cell(d, i);
             if (splits(c)) upper_record<ORDER>(A, c, tid & 1);
+        }
         __syncthreads();
     }
-    for (int b = 0; b < nr; b += TOP_T) {
-        const int k = b + tid;
-        const int sz = k < nr ? A.nd[k].size : 0, na = k < nr ? A.nd[k].nab : 0;
-        int is = sz, ia = na;
+    for (int b = 0; b < nr; b += TOP_T * TOP_R) {
+        const int k0 = b + tid * TOP_R;
+        int sz[TOP_R], na[TOP_R], ts = 0, ta = 0;
+        for (int q = 0; q < TOP_R; ++q) {
+            sz[q] = k0 + q < nr ? A.nd[k0 + q].size : 0;
+            na[q] = k0 + q < nr ? A.nd[k0 + q].nab : 0;
+        }
+        for (int q = 0; q < TOP_R; ++q) {
+            ts += sz[q];
+            ta += na[q];
+        }
+        int is = ts, ia = ta;
         for (int o = 1; o < 64; o <<= 1) {
             const int us = __shfl_up(is, o), ua = __shfl_up(ia, o);
             if (lane >= o) {
@@ -1504,7 +1728,7 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
         }
         if (lane == 63) ws[w] = make_int2(is, ia);
         __syncthreads();
-        int ps = run.x + is - sz, pa = run.y + ia - na;
+        int ps = run.x + is - ts, pa = run.y + ia - ta;
         for (int q = 0; q < TOP_T / 64; ++q) {
             if (q < w) {
                 ps += ws[q].x;
@@ -1513,9 +1737,12 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
             run.x += ws[q].x;
             run.y += ws[q].y;
         }
-        if (k < nr) {
-            A.nd[k].pre = ps;
-            A.nd[k].bpre = pa;
+        for (int q = 0; q < TOP_R; ++q) {
+            if (k0 + q >= nr) break;
+            A.nd[k0 + q].pre = ps;
+            A.nd[k0 + q].bpre = pa;
+            ps += sz[q];
+            pa += na[q];
         }
         __syncthreads();
     }
@@ -1528,8 +1755,9 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlev, TreeArgs 
         tell_host(host, err);
     }
     for (int d = 0; d < lev; ++d) {
-        const int c1 = A.L->lv[d + 1];
-        for (int c = A.L->lv[d] + tid; c < c1; c += TOP_T) {
+        const int nc = count(d);
+        for (int i = tid; i < nc; i += TOP_T) {
+            const int c = cell(d, i);
             if (!splits(c)) continue;
             const GNode &g = A.nd[c];
             GNode &l = A.nd[g.ch0], &u = A.nd[g.ch1];
@@ -1766,16 +1994,18 @@ __device__ __forceinline__ void emit_cell(const TreeArgs &A, const EmitArgs &E, 
     }
 }
 
-// Blocks below nub: a thread per slot above LMAX.  The others: a wavefront
-// per subtree of k_gt_sub, its cells in preorder (consecutive slots and ids).
+// Blocks below nub: a thread per slot above LMAX and per system that is a
+// bucket.  The others: a wavefront per subtree of k_gt_sub, its cells in
+// preorder (consecutive slots and ids).
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_gt_emit(int nub, int nup, int nsub, TreeArgs A, EmitArgs E)
+__global__ __launch_bounds__(256) void k_gt_emit(int nub, int nup, int nsub, int nr, TreeArgs A,
+                                                 EmitArgs E)
 {
     if ((int)blockIdx.x < nub) {
         const int c = blockIdx.x * 256 + threadIdx.x;
         if (c >= nup) return;
         const GNode &g = A.nd[c];
-        if (g.hi - g.lo < LMAX) return;                  // with its subtree
+        if (g.hi - g.lo < LMAX && !(c < nr && g.hi - g.lo < A.nBucket)) return;   // with its subtree
         const int2 p = climb(A.nd, A.L->b, c);
         emit_cell<ORDER>(A, E, c, p.x, p.y);
         return;
@@ -1831,20 +2061,65 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     GravDev &G = pkd->grav;
     hipStream_t st = pkd->stream;
     const int n = pkd->nLocal;
-    // roots: the non-empty systems
-    std::vector<int> rlo;
-    int maxRoot = 0;
-    for (int s = 0; s < nSys; ++s)
-        if (sysOff[s + 1] > sysOff[s]) {
-            rlo.push_back(sysOff[s]);
-            maxRoot = std::max(maxRoot, sysOff[s + 1] - sysOff[s]);
-        }
-    const int nr = (int)rlo.size();
-    for (int k = 0; k < nr; ++k) rlo.push_back(k + 1 < nr ? rlo[k + 1] - 1 : n - 1);
-    const size_t n1 = (size_t)n;
+    // roots: the non-empty systems, their ranges and what each size's stage
+    // reads (Roots), in one array for the device
     const int ts = tile_size(n);
-    const size_t mtile = n1 / ts + n1 / MID + nr + 1;                // tiles of a level, at most
-    const size_t mbox = std::max<size_t>(2 * (n1 / MID) + 2, nr);    // its cells
+    std::vector<int> up;
+    int nr = 0;
+    for (int s = 0; s < nSys; ++s) nr += sysOff[s + 1] > sysOff[s];
+    Roots R{};
+    R.n = n;
+    R.nr = nr;
+    R.nBucket = nBucket;
+    size_t oBig = 0, oBase[3] = {0, 0, 0}, oT = 0;
+    int nttile = 0;                  // tiles of the type orders
+    if (nr == 1) {                   // the whole store
+        R.nbig = n > MID;
+        R.nunit = n > LMAX && n <= MID;
+        R.nsub[n > LSML] = n > nBucket && n <= LMAX;
+        R.maxTiny = n <= nBucket ? n : 0;
+        if (n > LMAX) nttile = nblk(n, ts);
+    } else {
+        std::vector<int> big, mid, base[3];              // (roots above MID and LMAX)
+        up.resize(2 * (size_t)nr);
+        for (int s = 0, k = 0; s < nSys; ++s) {
+            const int cnt = sysOff[s + 1] - sysOff[s];
+            if (cnt <= 0) continue;
+            if ((k & 255) == 0) {
+                base[0].push_back(R.nsub[0]);
+                base[1].push_back(R.nsub[1]);
+                base[2].push_back(R.nunit);
+            }
+            up[k] = sysOff[s];
+            up[nr + k] = sysOff[s + 1] - 1;
+            if (cnt > MID) big.push_back(k);
+            else if (cnt > LMAX) ++R.nunit;
+            else if (cnt > nBucket) ++R.nsub[cnt > LSML];
+            else R.maxTiny = std::max(R.maxTiny, cnt);
+            if (cnt > LMAX) mid.push_back(k);
+            ++k;
+        }
+        R.nbig = (int)big.size();
+        R.ntroot = (int)mid.size();
+        auto add = [&](const std::vector<int> &v) {
+            const size_t at = up.size();
+            up.insert(up.end(), v.begin(), v.end());
+            return at;
+        };
+        oBig = add(big);
+        for (int k : big) up.push_back(up[k]);
+        for (int k : big) up.push_back(up[nr + k]);
+        for (int q = 0; q < 3; ++q) oBase[q] = add(base[q]);
+        oT = add(mid);
+        for (int k : mid) {
+            up.push_back(nttile);
+            nttile += nblk(up[nr + k] - up[k] + 1, ts);
+        }
+    }
+    const size_t n1 = (size_t)n;
+    // tiles of a level, or of the type orders, and a level's cells, at most
+    const size_t mtile = std::max<size_t>(n1 / ts + n1 / MID + 1, nttile);
+    const size_t mbox = 2 * (n1 / MID) + 2;
     const int order = iOrder >= 4 ? 4 : (iOrder == 3 ? 3 : 2);
     GG_TRY(G.px.reserve(sizeof(double) * n1));
     GG_TRY(G.py.reserve(sizeof(double) * n1));
@@ -1866,7 +2141,7 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     GG_TRY(G.gsub.reserve((sizeof(int) + sizeof(int2)) * (size_t)n));
     GG_TRY(G.gseg.reserve(sizeof(int) * 2 * n1));
     GG_TRY(G.glev.reserve(sizeof(GLevel)));
-    GG_TRY(G.groot.reserve(sizeof(int) * 2 * nr));
+    GG_TRY(G.groot.reserve(sizeof(int) * std::max<size_t>(up.size(), 1)));
     if (!G.hst)
         GG_HIP(hipHostMalloc((void **)&G.hst, sizeof(int) * GravDev::NHST, hipHostMallocDefault));
     GLevel *L = G.glev.as<GLevel>();
@@ -1897,18 +2172,27 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     T.useg = useg;
     T.seg = seg;
     T.segl = segl;
-    const int *rl = G.groot.as<int>(), *rh = rl + nr;
+    const int *rl = G.groot.as<int>();
+    R.lo = rl;
+    R.hi = rl + nr;
+    R.bslot = rl + oBig;
+    R.blo = R.bslot + R.nbig;
+    R.bhi = R.blo + R.nbig;
+    for (int q = 0; q < 3; ++q) R.base[q] = rl + oBase[q];
+    R.tslot = rl + oT;
+    R.toff = R.tslot + R.ntroot;
+    const int *list = nr > 1 ? R.bslot : nullptr;        // the first level's cells
     unsigned long long *box[2];
     box[0] = G.gbox.as<unsigned long long>();
     box[1] = box[0] + BOX_N * mbox;
     volatile int *hv = G.hst;
     for (int k = 0; k < 16; ++k) hv[k] = -1;
-    if (nr > 1)   // (a single root is the whole store)
-        GG_HIP(hipMemcpyAsync(G.groot.p, rlo.data(), sizeof(int) * 2 * nr, hipMemcpyHostToDevice,
+    if (nr > 1)
+        GG_HIP(hipMemcpyAsync(G.groot.p, up.data(), sizeof(int) * up.size(), hipMemcpyHostToDevice,
                               st));
-    hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, n, nr, rl, rh, T.nd,
-                       box[0], unit, L);
-    hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, n, nr, rl,
+    hipLaunchKernelGGL(k_gt_roots, dim3(nblk(nr, 256)), dim3(256), 0, st, R, T.nd, box[0], unit,
+                       sub, L);
+    hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, R,
                        pkd->f[GG_R].as<double>(), T.bits, T.px, T.py, T.pz, T.perm, box[0], L);
     hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need[1], G.hst);
     GG_HIP(hipGetLastError());
@@ -1928,32 +2212,35 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     A.tpre = A.tcnt + mtile;
     A.posR = G.gposR.as<int>();
     A.err = &L->err;
-    const int grid = (int)mtile;
-    auto ctl = [&](int mode, int depth, int *host) {
-        hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, mode, ts, depth, cap, L, T.nd,
-                           box[depth & 1], box[(depth & 1) ^ 1], G.gtile.as<int4>(), unit, host);
-    };
     // msrBuildTree's active-type orders (master.c:4262).  A particle with
     // the second order's bit has one of the first's, so where all have it
     // both orders leave everything in place.
     int lack = 0;
     GG_TRY(host_word(st, G.hst, &lack));
-    if (lack) {
-        ctl(1, 0, G.hst + 1);
+    if (lack && nttile > 0) {
+        hipLaunchKernelGGL(k_gt_type_tiles, dim3(nblk(nttile, 256)), dim3(256), 0, st, R, ts,
+                           nttile, T.nd, G.gtile.as<int4>(), L);
         A.mask = GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE;
-        GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
+        GG_TRY(gt_partition<1>(G, st, A, nttile, nullptr));
         A.mask = GG_TYPE_TREEACTIVE;
-        GG_TRY(gt_partition<1>(G, st, A, grid, nullptr));
+        GG_TRY(gt_partition<1>(G, st, A, nttile, nullptr));
     }
-    int nunit = nr, nlev = 0;
-    if (maxRoot > MID) {
+    const int ntroot = nr > 1 ? R.ntroot : n > LMAX;
+    if (lack && ntroot < nr)
+        hipLaunchKernelGGL(k_gt_type_small, dim3(std::min(nblk(nr, TY_W), 8192)), dim3(64 * TY_W),
+                           0, st, R, pkd->f[GG_R].as<double>(), T.bits, T.px, T.py, T.pz, T.perm);
+    int nunit = R.nunit, nlev = 0;
+    if (R.nbig > 0) {
+        const int grid = (int)(n1 / ts + n1 / MID + 1);  // tiles of a level
         // The levels.  The host learns a level's tile count while its
         // partition runs, in time to queue the next level behind it.
         for (int depth = 0;; ++depth) {
             GG_CHECK(depth < DMAX, GG_EUNSUP, "tree deeper than %d levels", DMAX);
             int *h = G.hst + 16 + 4 * (depth & 3);
             for (int k = 0; k < 2; ++k) ((volatile int *)h)[k] = -1;
-            ctl(0, depth, h);
+            hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, ts, depth, cap, R.nbig,
+                               depth ? nullptr : list, L, T.nd, box[depth & 1],
+                               box[(depth & 1) ^ 1], G.gtile.as<int4>(), unit, h);
             GG_TRY(gt_partition<0>(G, st, A, grid, box[(depth & 1) ^ 1]));
             int nt = 0;
             GG_TRY(host_word(st, h, &nt));
@@ -1969,17 +2256,28 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     if (nunit > 0)
         hipLaunchKernelGGL(k_gt_mid, dim3(nunit), dim3(MID_T), 0, st, unit, cap, L, T.nd, T.px,
                            T.py, T.pz, T.perm, sub, seg, segl, useg);
-    const int gsub = std::min(std::max(n / 64, 1), 2048);
-#define GG_BY_ORDER(K, GRID, BLOCK, ...)                                                          \
-    do {                                                                                          \
-        if (order == 4) hipLaunchKernelGGL(K<4>, GRID, BLOCK, 0, st, __VA_ARGS__);                \
-        else if (order == 3) hipLaunchKernelGGL(K<3>, GRID, BLOCK, 0, st, __VA_ARGS__);           \
-        else hipLaunchKernelGGL(K<2>, GRID, BLOCK, 0, st, __VA_ARGS__);                           \
-    } while (0)
-    GG_BY_ORDER(k_gt_sub, dim3(gsub), dim3(SUB_T), T);
-    if (nunit > 0) GG_BY_ORDER(k_gt_up_unit, dim3(nunit), dim3(64), T);
-    GG_BY_ORDER(k_gt_up_top, dim3(1), dim3(TOP_T), nr, nlev, T, ht);
-    if (nunit > 0) GG_BY_ORDER(k_gt_up_bmax, dim3(nunit), dim3(BM_T), T);
+    auto by_order = [&](auto f) {
+        if (order == 4) f(std::integral_constant<int, 4>{});
+        else if (order == 3) f(std::integral_constant<int, 3>{});
+        else f(std::integral_constant<int, 2>{});
+    };
+    by_order([&](auto o) {
+        constexpr int O = decltype(o)::value;
+        if (R.nsub[0] > 0) {
+            const int grid = std::min(R.nsub[0], 2560);
+            hipLaunchKernelGGL((k_gt_sub<O, LSML, 64>), dim3(grid), dim3(64), 0, st, T, 0,
+                               R.nsub[0], cap < 2 * n + 2 ? R.nsub[0] / grid : 0);
+        }
+        if (R.nsub[1] + nunit > 0)
+            hipLaunchKernelGGL((k_gt_sub<O, LMAX, 256>), dim3(std::min(std::max(n / 64, 1), 2048)),
+                               dim3(256), 0, st, T, R.nsub[0], -1, 0);
+        if (R.maxTiny > 0)
+            hipLaunchKernelGGL(k_gt_tiny<O>, dim3(nblk(nr, 256)), dim3(256), 0, st, nr, T);
+        if (nunit > 0) hipLaunchKernelGGL(k_gt_up_unit<O>, dim3(nunit), dim3(64), 0, st, T);
+        hipLaunchKernelGGL(k_gt_up_top<O>, dim3(1), dim3(TOP_T), 0, st, nr, R.nbig, list, nlev, T,
+                           ht);
+        if (nunit > 0) hipLaunchKernelGGL(k_gt_up_bmax<O>, dim3(nunit), dim3(BM_T), 0, st, T);
+    });
     GG_HIP(hipGetLastError());
     int tot[6];   // error word, cells, active buckets, largest bucket, slots above LMAX, subtrees
     for (int k = 0; k < 6; ++k) GG_TRY(host_word(st, ht + k, tot + k));
@@ -2009,8 +2307,10 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
     E.broot = G.broot.as<int>();
     E.bbox = G.bbox.as<double>();
     const int nub = nblk(nup, 256);
-    GG_BY_ORDER(k_gt_emit, dim3(nub + nblk(nsub, 4)), dim3(256), nub, nup, nsub, T, E);
-#undef GG_BY_ORDER
+    by_order([&](auto o) {
+        hipLaunchKernelGGL(k_gt_emit<decltype(o)::value>, dim3(nub + nblk(nsub, 4)), dim3(256), 0,
+                           st, nub, nup, nsub, nr, T, E);
+    });
     GG_HIP(hipGetLastError());
     G.nNodes = nn;
     G.nb = nb;

@@ -143,3 +143,28 @@ def test_split_with_an_empty_side_is_refused(gpu, n):
             pk.build_binary(16, 1, 0.7, 2)
             T = O.Tree(r, m, np.full(n, 0.01), nBucket=16, dTheta=0.7, iOrder=2)
             assert np.array_equal(pk.tree_info()[1], T.perm())
+
+
+@pytest.mark.parametrize("lack", [False, True])
+@pytest.mark.parametrize("big", [(), (600,), (9000, 513, 4096, 4097)])
+def test_forest_of_many_small_systems(gpu, big, lack):
+    # more systems than one pass of the roots' scan takes, buckets and
+    # subtrees among them, the larger ones at both ends and between
+    rng = np.random.default_rng(len(big) + 10 * lack)
+    sizes = rng.integers(0, 12, 4300)
+    sizes[rng.integers(0, 4300, 60)] = rng.integers(17, 513, 60)
+    sizes[7:12] = 512, 64, 16, 128, 129
+    sizes[[2150, 0, 4299, 2151][:len(big)]] = big
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    n = int(off[-1])
+    act = rng.choice(np.array([0, 1, 2, 3], np.uint32), n) if lack else None
+    check(gpu, rng.normal(size=(n, 3)), rng.uniform(0.5, 1.5, n), np.full(n, 0.01), 16, 3,
+          act=act, off=off)
+
+
+def test_forest_that_takes_slots_for_several_systems_at_once(gpu):
+    sizes = np.random.default_rng(4).integers(17, 20, 21000)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    n = int(off[-1])
+    r = np.random.default_rng(5).normal(size=(n, 3))
+    check(gpu, r, np.full(n, 1.0), np.full(n, 0.01), 16, 2, off=off)
