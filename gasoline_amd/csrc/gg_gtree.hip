@@ -779,7 +779,8 @@ __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long 
 // parts hold at most LMAX (listed for k_gt_sub).  The cells it closes (split,
 // or coincident and left buckets) are listed in seg from the cell's first
 // particle on, level by level, with the levels' ends in segl and their
-// numbers in useg, for the upward pass.
+// numbers in useg (that of the levels negative if buckets are among the
+// cells), for the upward pass.
 // At most MID / LMAX parts are open at a time, so a level is a handful of
 // wavefront passes over the particles between barriers instead of four
 // launches.  Its barriers and LDS round trips bound it: 88 us for a cell of 4096
@@ -813,7 +814,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     const int troot = nd[rootId].root;
     if (cnt > MID || cnt <= LMAX) {
         if (tid == 0) {
-            useg[blockIdx.x] = make_int2(cnt > MID, cnt > MID);
+            useg[blockIdx.x] = make_int2(cnt > MID, -(cnt > MID));
             if (cnt > MID) {             // coincident particles: a bucket
                 seg[glo] = rootId;
                 segl[glo] = 1;
@@ -841,6 +842,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
     const int w0 = w * (MID / (MID_T / 64));             // this wavefront's particles
     constexpr int WN = MID / MID_T;                      // its words
     int cur = 0, depth = 0, nseg = 0, nsubl = 0;        // (the counts: wavefront 0)
+    bool leaves = false;
     for (; nopen[cur] > 0; ++depth) {
         const int no = nopen[cur];
         for (int q = 0; q < no; ++q) {                   // bounds
@@ -971,6 +973,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
             if (sp && sub1) subl[su0 + sub0] = id0 + 1;
             const int me = in ? onode[cur][lane] : 0;
             if (in) seg[glo + nseg + lane] = me;
+            leaves |= __ballot(in && !sp) != 0;
             nseg += no;
             if (lane == 0) segl[glo + depth] = nseg;
             if (sp) {
@@ -1020,7 +1023,7 @@ __global__ __launch_bounds__(MID_T) void k_gt_mid(const int *__restrict__ unit, 
         if (full) return;
     }
     if (tid == 0) {
-        useg[blockIdx.x] = make_int2(nseg, depth);
+        useg[blockIdx.x] = make_int2(nseg, leaves ? -depth : depth);
         sub0_sh = nsubl ? atomicAdd(&L->nsub, nsubl) : 0;
         nsub_sh = nsubl;
     }
@@ -1607,39 +1610,110 @@ template <int ORDER> __global__ __launch_bounds__(256) void k_gt_tiny(int nr, Tr
     g.nab = na > 0;
 }
 
-// A closed cell above LMAX, by a pair of lanes (q 0, 1): its record and its
-// subtree's counts from its children's, or, of a bucket of coincident
-// particles, from its particles (by lane 0).
+// The record of a bucket of more than LMAX coincident particles, by one
+// wavefront: 64 particles at a time into registers, the sums that follow the
+// storage order (mass, softening, centre) taken from them lane by lane, all
+// else by lane and reduced.  By one lane each particle cost two chains of
+// loads: a build with 10^5 of them took 69 ms, 9.9 this way.
+__device__ __forceinline__ double lane_d(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+template <int ORDER> __device__ void large_bucket(const TreeArgs &A, int c, int lane)
+{
+#pragma clang fp contract(off)
+    constexpr int GS = gm_stride(ORDER);
+    GNode &g = A.nd[c];
+    const int lo = g.lo, hi = g.hi;
+    double M = 0.0, S = 0.0, R[3] = {0.0, 0.0, 0.0};
+    double bl[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, bh[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+    double fsm = 0.0;
+    int na = 0;
+    for (int b = lo; b <= hi; b += 64) {
+        const int i = b + lane;
+        double m = 0.0, mh = 0.0, mp[3] = {0.0, 0.0, 0.0};
+        bool act = false;
+        if (i <= hi) {
+            const int s = A.perm[i];
+            const double p[3] = {A.px[i], A.py[i], A.pz[i]}, h = A.h[s];
+            const uint32_t t = A.bits[s];
+            m = A.m[s];
+            A.pm[i] = m;
+            A.ph[i] = h;
+            A.pact[i] = t;
+            act = t & 1u;
+            mh = m * h;
+            if (h > fsm) fsm = h;
+            for (int d = 0; d < 3; ++d) {
+                mp[d] = m * p[d];
+                if (act && p[d] < bl[d]) bl[d] = p[d];
+                if (act && p[d] > bh[d]) bh[d] = p[d];
+            }
+        }
+        na += __popcll(__ballot(act));
+        const int n = min(64, hi - b + 1);
+        for (int l = 0; l < n; ++l) {
+            M += lane_d(m, l);
+            S += lane_d(mh, l);
+            for (int d = 0; d < 3; ++d) R[d] += lane_d(mp[d], l);
+        }
+    }
+    if (M > 0) {
+        S /= M;
+        for (int d = 0; d < 3; ++d) R[d] /= M;
+    }
+    double v[GS], b2 = 0.0;
+    for (int k = 0; k < GS; ++k) v[k] = 0.0;
+    for (int i = lo + lane; i <= hi; i += 64) {
+        const double d2 = cm_d2(A.px[i], A.py[i], A.pz[i], R);
+        if (d2 > b2) b2 = d2;
+        const double d[3] = {A.px[i] - R[0], A.py[i] - R[1], A.pz[i] - R[2]};
+        mom_particle<ORDER>(A.pm[i], d, v);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        double t = __shfl_xor(b2, o);
+        b2 = t > b2 ? t : b2;
+        t = __shfl_xor(fsm, o);
+        fsm = t > fsm ? t : fsm;
+        for (int d = 0; d < 3; ++d) {
+            t = __shfl_xor(bl[d], o);
+            bl[d] = t < bl[d] ? t : bl[d];
+            t = __shfl_xor(bh[d], o);
+            bh[d] = t > bh[d] ? t : bh[d];
+        }
+        for (int k = GM_Q; k < GS; ++k) v[k] += __shfl_xor(v[k], o);
+    }
+    if (lane) return;
+    v[0] = M;
+    v[1] = S;
+    for (int d = 0; d < 3; ++d) v[2 + d] = R[d];
+    v[GM_B] = b2;
+    double *o = A.gm + (size_t)GS * c, *bb = A.bb8 + 8 * (size_t)c;
+    for (int k = 0; k < GS; ++k) o[k] = v[k];
+    for (int d = 0; d < 3; ++d) {
+        bb[d] = bl[d];
+        bb[3 + d] = bh[d];
+    }
+    bb[6] = fsm;
+    bb[7] = (double)na;
+    g.size = 1;
+    g.nab = na > 0;
+    atomicMax(&A.L->maxb, hi - lo + 1);
+}
+
+// A split cell above LMAX, by a pair of lanes (q 0, 1): its record and its
+// subtree's counts from its children's.
 template <int ORDER> __device__ __forceinline__ void upper_record(const TreeArgs &A, int c, int q)
 {
 #pragma clang fp contract(off)
     constexpr int GS = gm_stride(ORDER);
     GNode &g = A.nd[c];
-    double *o = A.gm + (size_t)GS * c;
     double v[GS];
     for (int k = 0; k < GS; ++k) v[k] = 0.0;
-    const bool leaf = g.dim < 0;
-    if (leaf) {
-        if (q) return;
-        const int na = bucket_record<ORDER>(
-            g.lo, g.hi,
-            [&](int i, double *p, double &m, double &h) {
-                const int s = A.perm[i];
-                p[0] = A.px[i];
-                p[1] = A.py[i];
-                p[2] = A.pz[i];
-                A.pm[i] = m = A.m[s];
-                A.ph[i] = h = A.h[s];
-                A.pact[i] = A.bits[s];
-                return (A.pact[i] & 1u) != 0;
-            },
-            v, A.bb8 + 8 * (size_t)c);
-        for (int k = 0; k < GS; ++k) o[k] = v[k];
-        g.size = 1;
-        g.nab = na > 0;
-        atomicMax(&A.L->maxb, g.hi - g.lo + 1);
-        return;
-    }
     const int i0 = g.ch0, i1 = g.ch1;
     const double *c0 = A.gm + (size_t)GS * i0, *c1 = A.gm + (size_t)GS * i1;
     mass_children(c0, c1, v);
@@ -1649,6 +1723,7 @@ template <int ORDER> __device__ __forceinline__ void upper_record(const TreeArgs
     for (int k = GM_Q; k < GS; ++k) v[k] += __shfl_xor(v[k], 1);
     if (q) return;
     v[GM_B] = 0.0;
+    double *o = A.gm + (size_t)GS * c;
     for (int k = 0; k < GS; ++k) o[k] = v[k];
     const int s0 = A.nd[i0].size, a0 = A.nd[i0].nab;
     g.sizeLo = s0;
@@ -1657,7 +1732,8 @@ template <int ORDER> __device__ __forceinline__ void upper_record(const TreeArgs
     g.nab = a0 + A.nd[i1].nab;
 }
 
-// What k_gt_mid closed in one unit, deepest level first (one wavefront).
+// What k_gt_mid closed in one unit: buckets, then the split cells, deepest
+// level first (one wavefront).
 template <int ORDER> __global__ __launch_bounds__(64) void k_gt_up_unit(TreeArgs A)
 {
     const int lane = threadIdx.x;
@@ -1665,9 +1741,21 @@ template <int ORDER> __global__ __launch_bounds__(64) void k_gt_up_unit(TreeArgs
     const int2 u = A.useg[blockIdx.x];
     if (u.y == 0) return;
     const int base = A.nd[A.unit[blockIdx.x]].lo;
-    for (int l = u.y - 1; l >= 0; --l) {
+    const bool leaves = u.y < 0;
+    if (leaves) {
+        for (int e = 0; e < u.x; e += 64) {
+            const int c = e + lane < u.x ? A.seg[base + e + lane] : -1;
+            for (unsigned long long m = __ballot(c >= 0 && A.nd[c].dim < 0); m; m &= m - 1)
+                large_bucket<ORDER>(A, __shfl(c, __ffsll((long long)m) - 1), lane);
+        }
+        __syncthreads();
+    }
+    for (int l = abs(u.y) - 1; l >= 0; --l) {
         const int e0 = l ? A.segl[base + l - 1] : 0, e1 = A.segl[base + l];
-        for (int e = e0 + (lane >> 1); e < e1; e += 32) upper_record<ORDER>(A, A.seg[base + e], lane & 1);
+        for (int e = e0 + (lane >> 1); e < e1; e += 32) {
+            const int c = A.seg[base + e];
+            if (!(leaves && A.nd[c].dim < 0)) upper_record<ORDER>(A, c, lane & 1);
+        }
         __syncthreads();
     }
 }
@@ -1697,16 +1785,17 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlist,
         return g.hi - g.lo >= MID && g.dim >= 0;
     };
     // a level's cells (the first one's may be a list)
-    auto count = [&](int d) { return d == 0 && list ? nlist : A.L->lv[d + 1] - A.L->lv[d]; };
-    auto cell = [&](int d, int i) { return d == 0 && list ? list[i] : A.L->lv[d] + i; };
-    for (int d = lev - 1; d >= 0; --d) {
-        const int nc = count(d);
-        for (int i = tid >> 1; i < nc; i += TOP_T / 2) {
-            const int c = cell(d, i);
-            if (splits(c)) upper_record<ORDER>(A, c, tid & 1);
+    auto cells = [&](int d, int first, int step, auto f) {
+        const int *ls = d ? nullptr : list;
+        const int a = A.L->lv[d], nc = ls ? nlist : A.L->lv[d + 1] - a;
+        for (int i = first; i < nc; i += step) {
+            const int c = ls ? ls[i] : a + i;
+            if (splits(c)) f(c);
         }
         __syncthreads();
-    }
+    };
+    for (int d = lev - 1; d >= 0; --d)
+        cells(d, tid >> 1, TOP_T / 2, [&](int c) { upper_record<ORDER>(A, c, tid & 1); });
     for (int b = 0; b < nr; b += TOP_T * TOP_R) {
         const int k0 = b + tid * TOP_R;
         int sz[TOP_R], na[TOP_R], ts = 0, ta = 0;
@@ -1754,20 +1843,15 @@ __global__ __launch_bounds__(TOP_T) void k_gt_up_top(int nr, int nlist,
         tell_host(host + 5, A.L->nsub);
         tell_host(host, err);
     }
-    for (int d = 0; d < lev; ++d) {
-        const int nc = count(d);
-        for (int i = tid; i < nc; i += TOP_T) {
-            const int c = cell(d, i);
-            if (!splits(c)) continue;
+    for (int d = 0; d < lev; ++d)
+        cells(d, tid, TOP_T, [&](int c) {
             const GNode &g = A.nd[c];
             GNode &l = A.nd[g.ch0], &u = A.nd[g.ch1];
             l.pre = g.pre + 1;
             l.bpre = g.bpre;
             u.pre = g.pre + 1 + g.sizeLo;
             u.bpre = g.bpre + g.nabLo;
-        }
-        __syncthreads();
-    }
+        });
 }
 
 // Largest squared distances of the cells above LMAX: per unit, those of the

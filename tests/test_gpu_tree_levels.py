@@ -168,3 +168,15 @@ def test_forest_that_takes_slots_for_several_systems_at_once(gpu):
     n = int(off[-1])
     r = np.random.default_rng(5).normal(size=(n, 3))
     check(gpu, r, np.full(n, 1.0), np.full(n, 0.01), 16, 2, off=off)
+
+
+@pytest.mark.parametrize("clump", [513, 577, 4097])
+def test_large_coincident_bucket_of_unequal_particles(gpu, clump):
+    # the sums follow the storage order: with unequal masses another order
+    # shows; the type orders move the clump's particles first
+    n = clump + 1500
+    rng = np.random.default_rng(clump)
+    r = rng.normal(size=(n, 3))
+    r[rng.permutation(n)[:clump]] = r[0]
+    check(gpu, r, rng.uniform(0.5, 1.5, n), rng.uniform(0.01, 0.02, n), 16, 3,
+          act=rng.choice(np.array([0, 2, 3], np.uint32), n))
