@@ -125,6 +125,7 @@ struct SphDev {
     uint32_t gasMask = 0;
     int64_t nExtra = 0;
     int nExtraDev = 0;                         // > 0: nExtra still in that many partials in nxd
+    int reused = 0;                            // the last re-smooth took the kNN's lists
     DevBuf key, order, k2, v2, sortTmp, sel, pos, gidx, part;
     DevBuf sx, sy, sz;                         // slot order positions
     DevBuf child, rng, sparse;                 // radix tree, bucket-box sparse table

@@ -2961,6 +2961,7 @@ extern "C" int gg_resmooth(GGPKD pkd, const gg_smf *smf, int nSmooth, int bPerio
         reuse = S.rb[0] == 0;
         exact = reuse && S.rb[1] == 0;
     }
+    S.reused = reuse;
     const int64_t *off;
     const int *idx;
     if (reuse) {
@@ -3236,9 +3237,9 @@ extern "C" int gg_smooth_stats(GGPKD pkd, int64_t *s, int n)
         for (int64_t v : part) S.nExtra += v;
         S.nExtraDev = 0;
     }
-    const int64_t v[10] = {(int64_t)S.retried, (int64_t)S.ties, S.nExtra, (int64_t)S.listQueries,
+    const int64_t v[11] = {(int64_t)S.retried, (int64_t)S.ties, S.nExtra, (int64_t)S.listQueries,
                            (int64_t)S.diag[0], (int64_t)S.diag[1], (int64_t)S.diag[2],
-                           (int64_t)S.diag[3], (int64_t)S.passes, S.cand};
-    for (int k = 0; k < n && k < 10; ++k) s[k] = v[k];
+                           (int64_t)S.diag[3], (int64_t)S.passes, S.cand, S.reused};
+    for (int k = 0; k < n && k < 11; ++k) s[k] = v[k];
     return GG_OK;
 }

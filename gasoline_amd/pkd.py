@@ -468,11 +468,12 @@ class Pkd:
         return out
 
     def smooth_stats(self):
-        s = np.zeros(10, np.int64)
-        _check(lib().gg_smooth_stats(self.h, _p(s, _i64p), 10))
+        s = np.zeros(11, np.int64)
+        _check(lib().gg_smooth_stats(self.h, _p(s, _i64p), 11))
         return dict(retried=int(s[0]), ties=int(s[1]), extras=int(s[2]), queries=int(s[3]),
                     groups_overflowed=int(s[4]), short_at_RL=int(s[5]), unsettled=int(s[6]),
-                    max_buckets=int(s[7]), extra_passes=int(s[8]), candidates=int(s[9]))
+                    max_buckets=int(s[7]), extra_passes=int(s[8]), candidates=int(s[9]),
+                    lists_reused=bool(s[10]))
 
     def reorder(self, want_perm=True):
         """Permute the store into the SPH structure's order (gg_reorder);

@@ -419,7 +419,8 @@ int gg_smooth_lists(GGPKD pkd, int nSmooth, int *nbr);
  * the group radius, s[6] queries whose radius search did not settle, s[7]
  * largest number of buckets in a group; search work of the last gg_smooth:
  * s[8] trial balls beyond the first (widened or narrowed), s[9] candidate
- * particles whose distance was computed.  n <= 10. */
+ * particles whose distance was computed; s[10] whether the last gg_resmooth
+ * took the kNN's lists (1) or gathered the balls (0).  n <= 11. */
 int gg_smooth_stats(GGPKD pkd, int64_t *s, int n);
 
 /* --------------------------------------------- ensembles, graphs, tuning */

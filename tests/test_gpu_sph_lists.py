@@ -118,6 +118,46 @@ def test_resmooth_of_fewer_particles(gpu, n, part):
             for k, w in (("a", 3), ("uDotPdV", 1), ("mumax", 1)):
                 pk.put(k, np.zeros((n, w)) if w > 1 else np.zeros(n))
             pk.resmooth(smf, K, False)
+            # (with no query there is no list to differ)
+            assert pk.smooth_stats()["lists_reused"] == (f is fb2 or not on.any())
             out.append([pk.get(k) for k in ("a", "uDotPdV", "mumax")])
     for x, y in zip(*out):
         assert (not y.any() and not x.any()) if not on.any() else scaled(x, y) < 1e-12
+
+
+def test_dendvdx_of_fewer_particles_then_forces_of_all(gpu):
+    # DenDVDX again for some of the particles takes the kNN's lists (the same
+    # sums, bit for bit) and finds extras of those only: the forces of all that
+    # follow find their own
+    K = 32
+    d = ics.evrard(9000, seed=7)
+    n = len(d["m"])
+    on = np.random.default_rng(2).uniform(size=n) < 0.3
+    smf = gpu.Smf.default()
+    forces = (("a", 3), ("uDotPdV", 1), ("mumax", 1))
+    dens = ("fDensity", "divv", "curlv", "BalsaraSwitch")
+    out = []
+    with gpu.Pkd(n, prec=gpu.PREC_FP64) as pk:
+        put_gas(pk, d)
+        pk.put("iActive", np.where(on, 7 + 16, 7).astype(np.uint32) | gpu.TYPE_GAS)
+        pk.build_local()
+        pk.smooth(smf, K, False)
+        pk.gas_pressure(smf)
+        assert pk.smooth_stats()["ties"] == 0
+        first = {k: pk.get(k) for k in dens}
+        for again in (False, True):
+            if again:
+                assert pk.active_type(16, gpu.TYPE_SMOOTHACTIVE) == on.sum()
+                pk.put("fDensity", np.where(on, 0.0, first["fDensity"]))
+                pk.resmooth(smf, K, False, gpu.SMX_DENDVDX)
+                assert pk.smooth_stats()["lists_reused"]
+                for k in dens:
+                    assert np.array_equal(pk.get(k), first[k])
+                assert pk.active_type(gpu.TYPE_GAS, gpu.TYPE_SMOOTHACTIVE) == n
+            for k, w in forces:
+                pk.put(k, np.zeros((n, w)) if w > 1 else np.zeros(n))
+            pk.resmooth(smf, K, False)
+            assert pk.smooth_stats()["lists_reused"]
+            out.append([pk.get(k) for k, w in forces])
+    for x, y in zip(*out):
+        assert scaled(x, y) < 1e-12
