@@ -21,14 +21,18 @@
  * success and a negative GG_E* code on error, with a message available from
  * gg_last_error() (gasoline itself asserts; errors here are returned).
  * All calls on one GGPKD are issued on that handle's HIP stream, in order.
- * gg_build_local, gg_smooth, gg_gas_pressure and gg_resmooth may return
- * before their last kernels have finished (each still waits for what its
- * host side must read: counts, error words); every call that hands results
- * to the host (gg_get, gg_grav_all's counters, gg_timings, ...) waits for
- * the stream first.  A caller that reads the store's device memory on a
- * stream of its own synchronises the handle's stream (or the device)
- * before it does.  The other calls are synchronous with respect to the
- * host unless stated otherwise.
+ * These may return before their last kernels have finished:
+ * gg_build_binary, gg_build_forest; gg_build_local, gg_smooth,
+ * gg_gas_pressure, gg_resmooth; gg_drift, gg_kick_vpred, gg_grav_step; and
+ * the calls on type bits and rungs, gg_active_mask_rung, gg_active_type,
+ * gg_active_type_rung, gg_active_exact_type, gg_set_type, gg_reset_type and
+ * gg_sph_curr_rung.  Each still waits for what its host side must read
+ * (counts, error words); every call that hands fields or times to the host
+ * (gg_get, gg_tree_info, gg_timings, ...) waits for the stream first.  A
+ * caller that reads the store's device memory on a stream of its own
+ * synchronises the handle's stream (or the device) before it does.  The
+ * other calls are synchronous with respect to the host unless stated
+ * otherwise.
  */
 #ifndef GASOLINE_AMD_H
 #define GASOLINE_AMD_H
