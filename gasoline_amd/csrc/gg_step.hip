@@ -66,22 +66,26 @@ __global__ void k_kick(KickArgs K)
 // threads, each over every gridDim-th chunk, and add up a block's lanes in LDS
 // first: one atomic a wavefront on one address is served at about 10 ns each,
 // which was most of gg_active_type's 201 us at 1M particles (20 us so).
-constexpr int TB = 512, MAXB = 512;
-int red_grid(size_t n)
+// k_grav_step, three dependent loads and little written, takes blocks of
+// TB_WIDE: on 4 10^7 particles 258 us with blocks of TB, 168 so (179 without a
+// limit on the blocks); the kicks and drifts, which stream, are slower so
+// (k_drift on 10^7 149 -> 159).
+constexpr int TB = 512, TB_WIDE = 1024, MAXB = 512;
+int red_grid(size_t n, int tb = TB)
 {
-    const size_t b = (n + TB - 1) / TB;
+    const size_t b = (n + tb - 1) / tb;
     return (int)(b < (size_t)MAXB ? b : (size_t)MAXB);
 }
 
-template <class T, class F>
+template <int B = TB, class T, class F>
 __device__ __forceinline__ T block_red(T v, F f)
 {
-    __shared__ T part[TB / 64];
+    __shared__ T part[B / 64];
     for (int o = 32; o > 0; o >>= 1) v = f(v, __shfl_xor(v, o));
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
     v = part[0];
-    for (int k = 1; k < TB / 64; ++k) v = f(v, part[k]);
+    for (int k = 1; k < B / 64; ++k) v = f(v, part[k]);
     __syncthreads();
     return v;
 }
@@ -168,8 +172,8 @@ __global__ void k_grav_step(int n, double dEta, const uint32_t *__restrict__ bit
                             unsigned *__restrict__ red, unsigned *__restrict__ h)
 {
     unsigned long long bad = 0;
-    for (size_t i = (size_t)blockIdx.x * TB + threadIdx.x; i < (size_t)n;
-         i += (size_t)gridDim.x * TB) {
+    for (size_t i = (size_t)blockIdx.x * TB_WIDE + threadIdx.x; i < (size_t)n;
+         i += (size_t)gridDim.x * TB_WIDE) {
         if (!(bits[i] & GG_TYPE_ACTIVE)) continue;
         if (!(dtg[i] > 0.0)) {
             ++bad;
@@ -178,7 +182,7 @@ __global__ void k_grav_step(int n, double dEta, const uint32_t *__restrict__ bit
         const double d = dEta / sqrt(dtg[i]);
         if (d < dt[i]) dt[i] = d;
     }
-    bad = block_red(bad, [](auto p, auto q) { return p + q; });
+    bad = block_red<TB_WIDE>(bad, [](auto p, auto q) { return p + q; });
     if (threadIdx.x == 0) hand_over(bad, red, h);
 }
 
@@ -614,8 +618,8 @@ extern "C" int gg_grav_step(GGPKD pkd, double dEta)
     unsigned *red;
     unsigned long long bad = 0;
     GG_TRY(red_begin(pkd, &red));
-    hipLaunchKernelGGL(k_grav_step, dim3(red_grid(n)), dim3(TB), 0, pkd->stream, n, dEta,
-                       pkd->f[GG_IACTIVE].as<uint32_t>(), pkd->f[GG_DTGRAV].as<double>(),
+    hipLaunchKernelGGL(k_grav_step, dim3(red_grid(n, TB_WIDE)), dim3(TB_WIDE), 0, pkd->stream, n,
+                       dEta, pkd->f[GG_IACTIVE].as<uint32_t>(), pkd->f[GG_DTGRAV].as<double>(),
                        pkd->f[GG_DT].as<double>(), red, pkd->redHost);
     GG_HIP(hipGetLastError());
     GG_TRY(red_count(pkd, &bad, nullptr, nullptr));

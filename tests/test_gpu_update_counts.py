@@ -49,3 +49,26 @@ def test_counts_and_reductions(gpu, n):
     w = r + 0.25
     assert np.array_equal(pk.get("r"), np.where(w >= 0.5, w - 1.0, w))
     pk.close()
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 524287, 524289, 1100001])
+def test_grav_step_over_its_blocks(gpu, n):
+    rng = np.random.default_rng(n)
+    on = rng.uniform(size=n) < 0.7
+    on[-1] = True
+    dtg, dt = rng.uniform(0.5, 2.0, n), rng.uniform(0.05, 0.2, n)
+    with gpu.Pkd(n, prec=gpu.PREC_FP64) as pk:
+        pk.put("r", np.zeros((n, 3)))
+        pk.put("iActive", on.astype(np.uint32))
+        pk.put("dtGrav", dtg)
+        for _ in range(2):
+            pk.put("dt", dt)
+            pk.grav_step(0.1)
+            assert np.array_equal(pk.get("dt"), np.where(on, np.minimum(dt, 0.1 / np.sqrt(dtg)), dt))
+        bad = on & (rng.uniform(size=n) < 0.1)
+        bad[-1] = True
+        pk.put("dtGrav", np.where(bad, 0.0, dtg))
+        with pytest.raises(gpu.GGError, match=f" {bad.sum()} active particles"):
+            pk.grav_step(0.1)
+        pk.put("dtGrav", dtg)
+        pk.grav_step(0.1)
