@@ -518,6 +518,12 @@ __device__ __forceinline__ void stage_soft(Stage<T, ORDER> &L, int lane, int ic,
     for (int k = 0; k < 6; ++k) L.f[5 + k][lane] = (T)c[CR_QR + k];
 }
 
+// FP32's cell terms take (8 / r^2)^l with moments divided by 8^l: the constants
+// staged with the moments (newt_terms) would bring the contractions to FP32's
+// limit at shorter lengths than term by term (10^12 in mass at a few 10^3 in
+// length).  One operation a cell; the values are the same.
+template <typename T> constexpr double dir2_unit() { return sizeof(T) == 4 ? 8.0 : 1.0; }
+
 template <typename T, int ORDER>
 __device__ __forceinline__ void stage_newt(Stage<T, ORDER> &L, int lane, int ic, const IArgs &A,
                                            double cx, double cy, double cz)
@@ -527,12 +533,13 @@ __device__ __forceinline__ void stage_newt(Stage<T, ORDER> &L, int lane, int ic,
     L.f[1][lane] = (T)(c[CR_X + 1] - cy);
     L.f[2][lane] = (T)(c[CR_X + 2] - cz);
     L.f[3][lane] = (T)c[CR_M];
-    for (int k = 0; k < 6; ++k) L.f[4 + k][lane] = (T)(3.0 * c[CR_QT + k]);
+    constexpr double e = dir2_unit<T>();
+    for (int k = 0; k < 6; ++k) L.f[4 + k][lane] = (T)(3.0 / e * c[CR_QT + k]);
     if constexpr (ORDER >= 3) {
         const double *oh = A.momOH + (size_t)OH_N * ic;
-        for (int k = 0; k < 7; ++k) L.f[10 + k][lane] = (T)(7.5 * oh[k]);
+        for (int k = 0; k < 7; ++k) L.f[10 + k][lane] = (T)(7.5 / (e * e) * oh[k]);
         if constexpr (ORDER >= 4)
-            for (int k = 0; k < 9; ++k) L.f[17 + k][lane] = (T)(17.5 * oh[10 + k]);
+            for (int k = 0; k < 9; ++k) L.f[17 + k][lane] = (T)(17.5 / (e * e * e) * oh[10 + k]);
     }
 }
 
@@ -641,9 +648,9 @@ __device__ __forceinline__ void eval_soft(const Stage<T, ORDER> &L, int m, const
 // traces folded into the monomials, the sums QEVAL forms over all components
 // regroup into seven cubic (octupole: five quadratic) combinations shared by
 // the three components of the field.  The constants of the powers of dir are
-// in the staged moments (3, 15/2, 105/6), those of the potential and the
-// radial term follow from u_l, the order's contraction times dir^(2l+1):
-// about 110 operations for a hexadecapole cell, 25 fewer than term by term
+// in the staged moments (3, 15/2, 105/6; and dir2_unit), those of the
+// potential and the radial term follow from u_l, the order's contraction times
+// dir^(2l+1): about 110 operations for a hexadecapole cell, 25 fewer than term by term
 // (FP32 on 3 10^5 particles 1.78 -> 1.69 ms; the vector units are busy all
 // the time in FP32 and 82% of it in FP64, so operations are what counts).
 template <typename T, int ORDER>
@@ -660,7 +667,7 @@ __device__ __forceinline__ void newt_terms(const Stage<T, ORDER> &L, int e, T mi
         const T qx = xz * dz + xy * dy + xx * dx;
         const T qy = yz * dz + xy * dx + yy * dy;
         const T qz = yz * dy + xz * dx + zz * dz;
-        const T d5 = d3 * dir2;
+        const T s2 = T(dir2_unit<T>()) * dir2, d5 = d3 * s2;
         const T u2 = d5 * (qx * dx + qy * dy + qz * dz);
         P.ax += d5 * qx;
         P.ay += d5 * qy;
@@ -677,7 +684,7 @@ __device__ __forceinline__ void newt_terms(const Stage<T, ORDER> &L, int e, T mi
             const T ox = xxx * cP + xyy * cR + xxy * cxy + xxz * cxz + xyz * cyz;
             const T oy = xxy * cP + yyy * cR + xyy * cxy + xyz * cxz + yyz * cyz;
             const T oz = xxz * cP + yyz * cR + xyz * cxy - (xxx + xyy) * cxz - (xxy + yyy) * cyz;
-            const T d7 = d5 * dir2;
+            const T d7 = d5 * s2;
             const T u3 = d7 * (ox * dx + oy * dy + oz * dz);
             P.ax += d7 * ox;
             P.ay += d7 * oy;
@@ -701,7 +708,7 @@ __device__ __forceinline__ void newt_terms(const Stage<T, ORDER> &L, int e, T mi
                              + yyyy * cF + yyyz * cG;
                 const T hz = xxxz * cA + xxyz * cB - xxxx * cC - xxyy * (cC + cG)
                              + xyyz * cD - (xxxy + xyyy) * cE + yyyz * cF - yyyy * cG;
-                const T d9 = d7 * dir2;
+                const T d9 = d7 * s2;
                 const T u4 = d9 * (hx * dx + hy * dy + hz * dz);
                 P.ax += d9 * hx;
                 P.ay += d9 * hy;

@@ -426,3 +426,23 @@ def test_periodic_tree_error_vs_direct_ewald(gpu, periodic_box):
     e2, e1 = rel_err(a2, ad), rel_err(a1, ad)
     assert np.sqrt(np.mean(e2 * e2)) < 1e-4
     assert 2e-4 < np.sqrt(np.mean(e1 * e1)) < 2e-3
+
+
+@pytest.mark.parametrize("order,mass,length", [(2, 1e6, 10 ** 7.5), (2, 1e12, 1e6), (3, 1.0, 1e5),
+                                               (3, 1e12, 5e3), (4, 1.0, 1e4), (4, 1e12, 10 ** 2.5),
+                                               (4, 1e12, 1e-2)])
+def test_fp32_in_units_of_large_masses_and_lengths(gpu, order, mass, length):
+    # FP32 against FP64 of the same tree where the multipole terms near FP32's
+    # limits (10^12 in mass and some 100 in length is a galaxy in solar masses
+    # and kpc)
+    r, v, m = ics.plummer(20000, seed=3)
+    out = []
+    for prec in (gpu.PREC_FP32, gpu.PREC_FP64):
+        with setup_pkd(gpu, r * length, m * mass, np.full(len(m), 0.01 * length), prec) as pk:
+            pk.build_binary(16, 1, 0.7, order)
+            pk.grav_all(order)
+            out.append((pk.get("a"), pk.get("fPot")))
+    (a, p), (A, P) = out
+    assert np.isfinite(a).all() and np.isfinite(p).all()
+    assert np.linalg.norm(a - A) < 1e-5 * np.linalg.norm(A)
+    assert np.linalg.norm(p - P) < 1e-5 * np.linalg.norm(P)
