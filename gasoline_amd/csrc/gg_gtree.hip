@@ -77,7 +77,7 @@ struct GLevel {
     int nloc;            // slots taken from the last one down
     int nsub;            // cells left to k_gt_sub
     int err;             // 1: a split left one side empty, 2: out of slots
-    int need[2];         // particles lacking a type bit of each order
+    int need;            // a particle lacks the type bit of the orders
     int maxb;            // largest bucket
     int lv[DMAX + 1];    // first cell of each level
 };
@@ -151,8 +151,7 @@ __global__ __launch_bounds__(256) void k_gt_roots(Roots R, GNode *__restrict__ n
         L->nunit = R.nunit;
         L->nsub = R.nsub[0] + R.nsub[1];
         L->maxb = R.maxTiny;
-        L->ntile = L->nloc = L->err = 0;
-        L->need[0] = L->need[1] = 0;
+        L->ntile = L->nloc = L->err = L->need = 0;
     }
     if (k < R.nbig) box_init(box + BOX_N * (size_t)k);
     int cnt = 0;
@@ -232,8 +231,8 @@ __device__ __forceinline__ unsigned long long block_box(double *lo, double *hi, 
 constexpr int INIT_E = 8;        // particles per thread of k_gt_init
 
 // Positions into storage order, the bounds of the systems of more than MID
-// particles, and whether a particle lacks the type bits of msrBuildTree's
-// orders (*need, master.c:4262).
+// particles, and whether a particle lacks the type bit of msrBuildTree's
+// second order (L->need, master.c:4262).
 __global__ __launch_bounds__(256) void k_gt_init(Roots R, const double *__restrict__ r,
                                                  const uint32_t *__restrict__ bits,
                                                  double *__restrict__ x, double *__restrict__ y,
@@ -262,7 +261,7 @@ __global__ __launch_bounds__(256) void k_gt_init(Roots R, const double *__restri
     static_assert(MID >= 256 * INIT_E, "a large system within a block holds one of its ends");
     const bool one = r0 == r1;
     double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    bool lack0 = false, lack1 = false;
+    bool lack = false;
     for (int e = 0; e < INIT_E; ++e) {
         const int i = first + e * 256 + threadIdx.x, i0 = i - lane;   // i0: the wavefront's first
         if (i0 > last) break;
@@ -274,9 +273,7 @@ __global__ __launch_bounds__(256) void k_gt_init(Roots R, const double *__restri
             y[i] = v[1];
             z[i] = v[2];
             src[i] = i;
-            const uint32_t t = bits[i];
-            lack0 |= !(t & (GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE));
-            lack1 |= !(t & GG_TYPE_TREEACTIVE);
+            lack |= !(bits[i] & GG_TYPE_TREEACTIVE);
         }
         if (!one) {
             // a block over several systems: 64 particles of one share their
@@ -320,11 +317,7 @@ __global__ __launch_bounds__(256) void k_gt_init(Roots R, const double *__restri
             }
         }
     }
-    const unsigned long long m0 = __ballot(lack0), m1 = __ballot(lack1);
-    if ((threadIdx.x & 63) == 0) {
-        if (m0) atomicOr(&L->need[0], 1);
-        if (m1) atomicOr(&L->need[1], 1);
-    }
+    if (__ballot(lack) && lane == 0) atomicOr(&L->need, 1);
     if (!one || r0 < 0) return;
     const unsigned long long k = block_box(lo, hi, sm);
     unsigned long long *b = box + BOX_N * (size_t)r0 + BOX_S * threadIdx.x;
@@ -2128,8 +2121,7 @@ static int tile_size(int n) { return n < (1 << 19) ? 1024 : (n < (1 << 22) ? 204
 
 // One partition pass over the tiles k_gt_ctl listed.
 template <int MODE>
-static int gt_partition(GravDev &G, hipStream_t st, const TileArgs &A, int grid,
-                        unsigned long long *kbox)
+static int gt_partition(hipStream_t st, const TileArgs &A, int grid, unsigned long long *kbox)
 {
     hipLaunchKernelGGL(k_gt_count<MODE>, dim3(grid), dim3(256), 0, st, A);
     hipLaunchKernelGGL(k_gt_rank<MODE>, dim3(grid), dim3(256), 0, st, A);
@@ -2278,7 +2270,7 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
                        sub, L);
     hipLaunchKernelGGL(k_gt_init, dim3(nblk(n, 256 * INIT_E)), dim3(256), 0, st, R,
                        pkd->f[GG_R].as<double>(), T.bits, T.px, T.py, T.pz, T.perm, box[0], L);
-    hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need[1], G.hst);
+    hipLaunchKernelGGL(k_gt_tell, dim3(1), dim3(1), 0, st, &L->need, G.hst);
     GG_HIP(hipGetLastError());
     TileArgs A;
     A.ts = ts;
@@ -2305,9 +2297,9 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
         hipLaunchKernelGGL(k_gt_type_tiles, dim3(nblk(nttile, 256)), dim3(256), 0, st, R, ts,
                            nttile, T.nd, G.gtile.as<int4>(), L);
         A.mask = GG_TYPE_ACTIVE | GG_TYPE_TREEACTIVE;
-        GG_TRY(gt_partition<1>(G, st, A, nttile, nullptr));
+        GG_TRY(gt_partition<1>(st, A, nttile, nullptr));
         A.mask = GG_TYPE_TREEACTIVE;
-        GG_TRY(gt_partition<1>(G, st, A, nttile, nullptr));
+        GG_TRY(gt_partition<1>(st, A, nttile, nullptr));
     }
     const int ntroot = nr > 1 ? R.ntroot : n > LMAX;
     if (lack && ntroot < nr)
@@ -2325,7 +2317,7 @@ static int gtree_try(GGPKD pkd, int nSys, const int *sysOff, int nBucket, int iO
             hipLaunchKernelGGL(k_gt_ctl, dim3(1), dim3(CTL_T), 0, st, ts, depth, cap, R.nbig,
                                depth ? nullptr : list, L, T.nd, box[depth & 1],
                                box[(depth & 1) ^ 1], G.gtile.as<int4>(), unit, h);
-            GG_TRY(gt_partition<0>(G, st, A, grid, box[(depth & 1) ^ 1]));
+            GG_TRY(gt_partition<0>(st, A, grid, box[(depth & 1) ^ 1]));
             int nt = 0;
             GG_TRY(host_word(st, h, &nt));
             if (nt == 0) {
