@@ -615,7 +615,7 @@ template <int MODE> __global__ __launch_bounds__(256) void k_gt_count(TileArgs A
     if (threadIdx.x == 0) A.tcnt[t] = wc[0] + wc[1] + wc[2] + wc[3];
 }
 
-constexpr int TW = 64;                   // flag words of the largest tile
+constexpr int TW = 64;                   // flag words of a tile, at most (one wavefront scans them)
 
 // The tile's flag words and, before each, the number of flags of its cell
 // (pre: those of the cell's earlier tiles).
@@ -2116,8 +2116,12 @@ int host_word(hipStream_t st, const int *p, int *v)
 }
 
 // Particles per tile: enough tiles to fill the chip on a small store, fewer
-// of them (each block adds up its cell's tile counts) on a large one.
-static int tile_size(int n) { return n < (1 << 19) ? 1024 : (n < (1 << 22) ? 2048 : 4096); }
+// of them (each block adds up its cell's tile counts) on a large one.  Builds
+// of Plummer spheres with 1024 / 2048 / 4096, us: 5000 particles 392 / 400 / 416,
+// 30011 718 / 773 / 890, 3 10^5 1026 / 1125 / 1339, 2^20 1789 / 1857 / 2088,
+// 2^21 2930 / 2933 / 3114, 2^22 5133 / 5020 / 5140, 2^24 19822 / 18933 / 19131;
+// uniform boxes the same way.
+static int tile_size(int n) { return n < (1 << 21) ? 1024 : 2048; }
 
 // One partition pass over the tiles k_gt_ctl listed.
 template <int MODE>
