@@ -697,9 +697,9 @@ template <int MODE> __global__ __launch_bounds__(256) void k_gt_rank(TileArgs A)
 // upper particle (counted up from lo) <-> posR[lo + k], each pair swapped
 // by its lower member.  Every particle passes through registers once, so
 // the children's bounds are taken on the way (mode 0).  It moves 24-28 bytes
-// a particle and 56 a swapped one.  Measured per level: 25 us on a 2^21
-// Plummer sphere (count 6.3, rank 4.6, control 5.9) and 14 us on 3 10^5
-// particles (4.3, 3.9, 5.4), where the chain of loads and the bounds'
+// a particle and 56 a swapped one.  Measured per level: 23 us on a 2^21
+// Plummer sphere (count 6.0, rank 4.6, control 6.0) and 10.3 us on 3 10^5
+// particles (4.1, 3.8, 5.1), where the chain of loads and the bounds'
 // reduction bound it rather than the bytes.
 template <int MODE>
 __global__ __launch_bounds__(256) void k_gt_swap(TileArgs A, unsigned long long *__restrict__ kbox)
