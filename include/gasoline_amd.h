@@ -418,9 +418,10 @@ int gg_smooth_lists(GGPKD pkd, int nSmooth, int *nbr);
  * nSmooth-th and (nSmooth+1)-th distances tie (their neighbour set is not
  * unique; gasoline's priority queue keeps the one met first), s[2] entries
  * of the force pass's extras lists, s[3] smooth-active particles; search
- * diagnostics of the bucket-group kNN: s[4] groups too large to search
- * (more than 192 buckets or 4096 particles), s[5] queries with fewer than nSmooth candidates in
- * the group radius, s[6] queries whose radius search did not settle, s[7]
+ * diagnostics of the bucket-group kNN, over the buckets that hold a
+ * smooth-active particle: s[4] groups too large to search (more than 192
+ * buckets or 4096 particles), s[5] queries with fewer than nSmooth candidates
+ * in the group radius, s[6] queries whose radius search did not settle, s[7]
  * largest number of buckets in a group; search work of the last gg_smooth:
  * s[8] trial balls beyond the first (widened or narrowed), s[9] candidate
  * particles whose distance was computed; s[10] whether the last gg_resmooth
