@@ -520,8 +520,11 @@ __device__ __forceinline__ void stage_soft(Stage<T, ORDER> &L, int lane, int ic,
 
 // FP32's cell terms take (8 / r^2)^l with moments divided by 8^l: the constants
 // staged with the moments (newt_terms) would bring the contractions to FP32's
-// limit at shorter lengths than term by term (10^12 in mass at a few 10^3 in
-// length).  One operation a cell; the values are the same.
+// limit at lengths up to twice shorter than term by term (10^12 in mass at a
+// few 10^2 in length, hexadecapole).  The values are the same.  One operation
+// a cell: 256 King models (4 10^6 particles) 14.0 -> 14.1 ms hexadecapole, 6.38
+// -> 6.51 quadrupole; a unit of length for the cells instead, with no operation
+// a cell, took 14.4 and 6.46.
 template <typename T> constexpr double dir2_unit() { return sizeof(T) == 4 ? 8.0 : 1.0; }
 
 template <typename T, int ORDER>
@@ -650,9 +653,9 @@ __device__ __forceinline__ void eval_soft(const Stage<T, ORDER> &L, int m, const
 // the three components of the field.  The constants of the powers of dir are
 // in the staged moments (3, 15/2, 105/6; and dir2_unit), those of the
 // potential and the radial term follow from u_l, the order's contraction times
-// dir^(2l+1): about 110 operations for a hexadecapole cell, 25 fewer than term by term
-// (FP32 on 3 10^5 particles 1.78 -> 1.69 ms; the vector units are busy all
-// the time in FP32 and 82% of it in FP64, so operations are what counts).
+// dir^(2l+1): about 110 operations for a hexadecapole cell, 25 fewer than term
+// by term (FP32 on 3 10^5 particles 1.78 -> 1.69 ms; the vector units are busy
+// all the time in FP32 and 82% of it in FP64, so operations are what counts).
 template <typename T, int ORDER>
 __device__ __forceinline__ void newt_terms(const Stage<T, ORDER> &L, int e, T mi, T dx, T dy, T dz,
                                            T dir, Part<T> &P, T &dtg)
