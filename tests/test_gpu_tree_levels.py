@@ -180,3 +180,27 @@ def test_large_coincident_bucket_of_unequal_particles(gpu, clump):
     r[rng.permutation(n)[:clump]] = r[0]
     check(gpu, r, rng.uniform(0.5, 1.5, n), rng.uniform(0.01, 0.02, n), 16, 3,
           act=rng.choice(np.array([0, 2, 3], np.uint32), n))
+
+
+def test_level_of_more_cells_than_one_pass_takes(gpu):
+    # 1100 copies of one system of more than 4096 particles: the first levels
+    # have more cells than the workgroup that decides them has threads
+    n, k = 4200, 1100
+    r, v, m = ics.plummer(n, seed=11)
+    T = O.Tree(r, m, np.full(n, 0.01), nBucket=32, dTheta=0.7, iOrder=2)
+    oi, od = T.nodes()
+    nn = len(oi)
+    with gpu.Pkd(n * k, prec=gpu.PREC_FP64) as pk:
+        pk.put("r", np.tile(r, (k, 1)))
+        pk.put("fMass", np.tile(m, k))
+        pk.put("fSoft", np.full(n * k, 0.01))
+        pk.build_forest((n * np.arange(k + 1)).astype(np.int32), 32, 1, 0.7, 2)
+        root, perm, ints, dbls = pk.tree_info()
+    at = np.arange(k)[:, None]
+    assert np.array_equal(perm.reshape(k, n), T.perm()[None] + n * at)
+    ints = ints.reshape(k, nn, 6)
+    for c, step in ((0, 0), (1, n), (2, n), (3, nn), (4, nn)):
+        assert np.array_equal(ints[:, :, c], np.where(oi[:, c] >= 0, oi[:, c] + step * at, oi[:, c]))
+    dbls = dbls.reshape(k, nn, 8)
+    assert np.array_equal(dbls[:, :, :6], np.tile(od[:, [7, 8, 9, 10, 11, 12]], (k, 1, 1)))
+    assert np.array_equal(dbls[:, :, 6], np.tile(od[:, 44], (k, 1)))
